@@ -2,6 +2,7 @@
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -18,24 +19,35 @@ def _stale(obj, deps):
     return not os.path.exists(obj) or any(os.path.getmtime(d) > os.path.getmtime(obj) for d in deps)
 
 
+# translation units: (source, object, extra flags, further dependencies); the kernels compile as shards
+UNITS = [("mgo_kernels.hip", f"mgo_kernels_{k}.o", [f"-DMGO_SHARD={k}"], []) for k in range(14)]
+UNITS.append(("mgo_host.cpp", "mgo_host.o", ["-x", "hip", "-ffp-contract=off"], ["mgo_serve.inc"]))
+
+
 def build(verbose=False, only_changed=False):
-    """Compile both translation units and link libmgo.so; with only_changed, an object newer than its
-    sources and headers is reused."""
-    objs = []
-    os.makedirs(os.path.join(HERE, "_obj"), exist_ok=True)
-    headers = [os.path.join(CSRC, "mgo_internal.h"), os.path.join(HERE, "..", "include", "mgo.h")]
-    for src, extra, deps in (("mgo_kernels.hip", [], []),
-                             ("mgo_host.cpp", ["-x", "hip", "-ffp-contract=off"], ["mgo_serve.inc"])):
-        obj = os.path.join(HERE, "_obj", src + ".o")
-        objs_deps = [os.path.join(CSRC, src)] + [os.path.join(CSRC, d) for d in deps] + headers
-        if only_changed and not _stale(obj, objs_deps):
-            objs.append(obj)
+    """Compile the translation units (in parallel) and link libmgo.so; with only_changed, an object newer than
+    its sources and headers is reused."""
+    objdir = os.path.join(HERE, "_obj")
+    os.makedirs(objdir, exist_ok=True)
+    headers = [os.path.join(CSRC, h) for h in ("mgo_internal.h", "mgo_npi.h")]
+    headers.append(os.path.join(HERE, "..", "include", "mgo.h"))
+    objs, cmds = [], []
+    for src, name, extra, deps in UNITS:
+        obj = os.path.join(objdir, name)
+        objs.append(obj)
+        if only_changed and not _stale(obj, [os.path.join(CSRC, d) for d in [src, *deps]] + headers):
             continue
-        cmd = [HIPCC, *COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
+        cmds.append([HIPCC, *COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj])
+    # the largest shards first
+    cmds.sort(key=lambda c: not any(f"MGO_SHARD={k}" in " ".join(c) for k in (9, 10, 11, 12)))
+
+    def compile_one(cmd):
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.run(cmd, check=True)
-        objs.append(obj)
+
+    with ThreadPoolExecutor(max(1, min(8, os.cpu_count() or 1, int(os.environ.get("MAX_JOBS", 8))))) as pool:
+        list(pool.map(compile_one, cmds))
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", OUT + ".tmp", *objs, "-lpthread"]
     if verbose:
         print(" ".join(cmd), flush=True)

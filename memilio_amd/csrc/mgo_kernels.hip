@@ -16,6 +16,10 @@
 //   return_phase<G>    per node lane: the returns with the negative-value fix-up, in parallel passes over
 //                      the nodes whose inputs changed (fixup_check between passes)
 //   replay_phase<G>    per flagged instance: sequential return pass with the negative-value fix-up
+//
+// The file is compiled once per shard (MGO_SHARD, see memilio_amd/build.py), in parallel: shard 0 holds the
+// launch dispatch and the kernels without a G, shards 1..8 the kernels of that G, shards 9..12 the node kernel
+// over mixed G of integrator kind MGO_SHARD - 9, shard 13 the edge kernels over mixed G.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -526,7 +530,7 @@ __device__ __forceinline__ void clock_one(InstDev& I)
 
 // One block: the first threads clear the cycle flags, then every instance advances its clock and flags the
 // phases it needs (every writer stores 1).
-__global__ void __launch_bounds__(1024) clock_kernel(InstDev* inst, int n, int32_t* cyc)
+static __global__ void __launch_bounds__(1024) clock_kernel(InstDev* inst, int n, int32_t* cyc)
 {
     if (cyc) {
         if (threadIdx.x < CYC_FLAGS) {
@@ -1435,7 +1439,7 @@ __device__ __forceinline__ void return_body(const LaunchDev& ld, InstDev* __rest
 }
 
 // After a return pass: settle the instance, schedule another pass, or hand it to the sequential replay.
-__global__ void fixup_check(LaunchDev ld, InstDev* inst)
+static __global__ void fixup_check(LaunchDev ld, InstDev* inst)
 {
     const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= ld.num_inst) {
@@ -1580,11 +1584,13 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
     depart_body<G>(ld, inst);
 }
 
+#if MGO_SHARD == 13
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) depart_phase_mixed(LaunchDev ld,
                                                                                              InstDev* __restrict__ inst)
 {
     MGO_DISPATCH_G(block_groups(ld), (depart_body<GG>(ld, inst)))
 }
+#endif
 
 template <int G, bool FIRST>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) return_phase(LaunchDev ld,
@@ -1606,6 +1612,7 @@ __global__ void __launch_bounds__(WAVE) replay_phase(LaunchDev ld, InstDev* __re
     replay_body<G>(ld, inst);
 }
 
+#if MGO_SHARD == 13
 __global__ void __launch_bounds__(WAVE) replay_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
 {
     const InstDev& I = inst[ld.inst_ids[blockIdx.x]];
@@ -1614,11 +1621,12 @@ __global__ void __launch_bounds__(WAVE) replay_phase_mixed(LaunchDev ld, InstDev
     }
     MGO_DISPATCH_G(ld.segs[I.seg].G, (replay_body<GG>(ld, inst)))
 }
+#endif
 
 // ------------------------------------------------------------------------------- launchers
 
 template <int G>
-static hipError_t launch_node_g(const LaunchDev& c, InstDev* inst, hipStream_t s)
+hipError_t launch_node_g(const LaunchDev& c, InstDev* inst, hipStream_t s)
 {
     const int nb = c.num_blocks;
 #define MGO_NODE_LAUNCH(KIND)                                                                                  \
@@ -1647,7 +1655,7 @@ static hipError_t launch_node_g(const LaunchDev& c, InstDev* inst, hipStream_t s
 }
 
 template <int G>
-static hipError_t launch_edge_g(const LaunchDev& c, InstDev* inst, hipStream_t s)
+hipError_t launch_edge_g(const LaunchDev& c, InstDev* inst, hipStream_t s)
 {
     const int nb = c.num_blocks;
     hipLaunchKernelGGL((depart_phase<G>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
@@ -1669,6 +1677,61 @@ static hipError_t launch_edge_g(const LaunchDev& c, InstDev* inst, hipStream_t s
     return hipGetLastError();
 }
 
+template <int K>
+hipError_t launch_node_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s)
+{
+    hipLaunchKernelGGL((node_phase_mixed<K>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+    return hipGetLastError();
+}
+
+
+hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s);
+
+#if MGO_SHARD >= 1 && MGO_SHARD <= 8
+template hipError_t launch_node_g<MGO_SHARD>(const LaunchDev&, InstDev*, hipStream_t);
+template hipError_t launch_edge_g<MGO_SHARD>(const LaunchDev&, InstDev*, hipStream_t);
+#elif MGO_SHARD >= 9 && MGO_SHARD <= 12
+template hipError_t launch_node_mixed<MGO_SHARD - 9>(const LaunchDev&, InstDev*, hipStream_t);
+#elif MGO_SHARD == 13
+hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s)
+{
+    const int nb = c.num_blocks;
+    hipLaunchKernelGGL(depart_phase_mixed, dim3(nb), dim3(BLOCK), 0, s, c, inst);
+    hipLaunchKernelGGL((return_phase_mixed<true>), dim3(nb), dim3(BLOCK), 0, s, c, inst, 0);
+    hipError_t err = hipGetLastError();
+    const int ni   = (c.num_inst + 255) / 256;
+    for (int p = 1; p < FX_MAX_PASSES && err == hipSuccess; ++p) {
+        hipLaunchKernelGGL(fixup_check, dim3(ni), dim3(256), 0, s, c, inst);
+        hipLaunchKernelGGL((return_phase_mixed<false>), dim3(nb), dim3(BLOCK), 0, s, c, inst, p);
+        err = hipGetLastError();
+    }
+    if (err != hipSuccess) {
+        return err;
+    }
+    hipLaunchKernelGGL(fixup_check, dim3(ni), dim3(256), 0, s, c, inst);
+    if (c.num_inst > 0) {
+        hipLaunchKernelGGL(replay_phase_mixed, dim3(c.num_inst), dim3(WAVE), 0, s, c, inst);
+    }
+    return hipGetLastError();
+}
+#else // MGO_SHARD == 0
+#define MGO_EXTERN_G(GG)                                                                                       \
+    extern template hipError_t launch_node_g<GG>(const LaunchDev&, InstDev*, hipStream_t);                     \
+    extern template hipError_t launch_edge_g<GG>(const LaunchDev&, InstDev*, hipStream_t);
+MGO_EXTERN_G(1)
+MGO_EXTERN_G(2)
+MGO_EXTERN_G(3)
+MGO_EXTERN_G(4)
+MGO_EXTERN_G(5)
+MGO_EXTERN_G(6)
+MGO_EXTERN_G(7)
+MGO_EXTERN_G(8)
+#undef MGO_EXTERN_G
+extern template hipError_t launch_node_mixed<MGO_INTEGRATOR_CASH_KARP54>(const LaunchDev&, InstDev*, hipStream_t);
+extern template hipError_t launch_node_mixed<MGO_INTEGRATOR_RKF45>(const LaunchDev&, InstDev*, hipStream_t);
+extern template hipError_t launch_node_mixed<MGO_INTEGRATOR_CASH_KARP54_FIXED>(const LaunchDev&, InstDev*, hipStream_t);
+extern template hipError_t launch_node_mixed<MGO_INTEGRATOR_EULER>(const LaunchDev&, InstDev*, hipStream_t);
+
 hipError_t launch_clock(InstDev* inst, int n, int32_t* cyc, hipStream_t s)
 {
     hipLaunchKernelGGL(clock_kernel, dim3(1), dim3(1024), 0, s, inst, n, cyc);
@@ -1681,7 +1744,7 @@ hipError_t launch_clock(InstDev* inst, int n, int32_t* cyc, hipStream_t s)
 // one launch each per loop iteration instead of one copy per request.
 static_assert(sizeof(InstDev) % 8 == 0, "instance records are copied as 8-byte words");
 
-__global__ void scatter_slots_kernel(InstDev* __restrict__ table, const InstDev* __restrict__ src,
+static __global__ void scatter_slots_kernel(InstDev* __restrict__ table, const InstDev* __restrict__ src,
                                      const int32_t* __restrict__ ids, int n)
 {
     constexpr int W = int(sizeof(InstDev) / 8);
@@ -1693,7 +1756,7 @@ __global__ void scatter_slots_kernel(InstDev* __restrict__ table, const InstDev*
     reinterpret_cast<uint64_t*>(table + ids[k])[w] = reinterpret_cast<const uint64_t*>(src + k)[w];
 }
 
-__global__ void set_segments_kernel(InstDev* __restrict__ table, const int32_t* __restrict__ ids, int n)
+static __global__ void set_segments_kernel(InstDev* __restrict__ table, const int32_t* __restrict__ ids, int n)
 {
     const int k = int(blockIdx.x * blockDim.x + threadIdx.x);
     if (k < n) {
@@ -1720,53 +1783,20 @@ hipError_t launch_set_segments(InstDev* table, const int32_t* ids, int n, hipStr
     return hipGetLastError();
 }
 
-static hipError_t launch_node_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s)
-{
-    const int nb = c.num_blocks;
-    switch (c.kind) {
-    case MGO_INTEGRATOR_CASH_KARP54:
-        hipLaunchKernelGGL((node_phase_mixed<MGO_INTEGRATOR_CASH_KARP54>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
-        break;
-    case MGO_INTEGRATOR_RKF45:
-        hipLaunchKernelGGL((node_phase_mixed<MGO_INTEGRATOR_RKF45>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
-        break;
-    case MGO_INTEGRATOR_CASH_KARP54_FIXED:
-        hipLaunchKernelGGL((node_phase_mixed<MGO_INTEGRATOR_CASH_KARP54_FIXED>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
-        break;
-    default:
-        hipLaunchKernelGGL((node_phase_mixed<MGO_INTEGRATOR_EULER>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
-        break;
-    }
-    return hipGetLastError();
-}
-
-static hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s)
-{
-    const int nb = c.num_blocks;
-    hipLaunchKernelGGL(depart_phase_mixed, dim3(nb), dim3(BLOCK), 0, s, c, inst);
-    hipLaunchKernelGGL((return_phase_mixed<true>), dim3(nb), dim3(BLOCK), 0, s, c, inst, 0);
-    hipError_t err = hipGetLastError();
-    const int ni   = (c.num_inst + 255) / 256;
-    for (int p = 1; p < FX_MAX_PASSES && err == hipSuccess; ++p) {
-        hipLaunchKernelGGL(fixup_check, dim3(ni), dim3(256), 0, s, c, inst);
-        hipLaunchKernelGGL((return_phase_mixed<false>), dim3(nb), dim3(BLOCK), 0, s, c, inst, p);
-        err = hipGetLastError();
-    }
-    if (err != hipSuccess) {
-        return err;
-    }
-    hipLaunchKernelGGL(fixup_check, dim3(ni), dim3(256), 0, s, c, inst);
-    if (c.num_inst > 0) {
-        hipLaunchKernelGGL(replay_phase_mixed, dim3(c.num_inst), dim3(WAVE), 0, s, c, inst);
-    }
-    return hipGetLastError();
-}
-
 hipError_t launch_node(const LaunchDev& c, InstDev* inst, hipStream_t s)
 {
     switch (c.G) {
     case 0:
-        return launch_node_mixed(c, inst, s);
+        switch (c.kind) {
+        case MGO_INTEGRATOR_CASH_KARP54:
+            return launch_node_mixed<MGO_INTEGRATOR_CASH_KARP54>(c, inst, s);
+        case MGO_INTEGRATOR_RKF45:
+            return launch_node_mixed<MGO_INTEGRATOR_RKF45>(c, inst, s);
+        case MGO_INTEGRATOR_CASH_KARP54_FIXED:
+            return launch_node_mixed<MGO_INTEGRATOR_CASH_KARP54_FIXED>(c, inst, s);
+        default:
+            return launch_node_mixed<MGO_INTEGRATOR_EULER>(c, inst, s);
+        }
     case 1:
         return launch_node_g<1>(c, inst, s);
     case 2:
@@ -1814,10 +1844,6 @@ hipError_t launch_edge(const LaunchDev& c, InstDev* inst, hipStream_t s)
     }
 }
 
-} // namespace mgo
-
-namespace mgo
-{
 // ------------------------------------------------------------------------------- ensemble analysis
 // Post-processing of the daily outputs of several runs of the same shape (cpp/memilio/data/
 // analyze_result.h:267-343). A "position" is one (day, node, compartment) value of a run's output; run r's
@@ -1943,5 +1969,7 @@ hipError_t launch_ensemble_select(const double* out, const int64_t* base, int ru
                        positions, ranks, num_ranks, sel);
     return hipGetLastError();
 }
+
+#endif // MGO_SHARD
 
 } // namespace mgo

@@ -36,6 +36,7 @@ hipError_t launch_scatter_slots(InstDev* table, const InstDev* src, const int32_
 hipError_t launch_set_segments(InstDev* table, const int32_t* ids, int n, hipStream_t s);
 hipError_t launch_node(const LaunchDev& c, InstDev* inst, hipStream_t s);
 hipError_t launch_edge(const LaunchDev& c, InstDev* inst, hipStream_t s);
+hipError_t launch_weights(const LaunchDev& c, InstDev* inst, int inst_offset, hipStream_t s);
 hipError_t launch_ensemble_mean(const double* out, const int64_t* base, int runs, int64_t positions, double* mean,
                                 hipStream_t s);
 hipError_t launch_sum_nodes(const double* out, const int64_t* base, int runs, int days, int nodes, int width,
@@ -306,6 +307,10 @@ struct EdgeStructHost {
     std::vector<int32_t> in_ptr, out_ptr, split, seq;
     std::vector<EdgeEnt> in_ent, out_ent;
     std::vector<double> in_min, out_min; // uniform minimum per entry (empty: the graph has no minimum)
+    // per node, over its out-edges: sums of the coefficients and minima (uniform: one value, else 10 G)
+    std::vector<double> out_sum, out_min_sum;
+    bool uniform  = true;  // one coefficient per edge
+    bool negative = false; // some coefficient or minimum is negative
     int n = 0, num_edges = 0;
 };
 
@@ -335,7 +340,7 @@ struct ClassHost {
     std::vector<int> insts; // global instance indices
     int num_nodes = 0;
     // device buffers
-    DevBuf y, snap, ypre, rc, yint, lcoef, cbase, cdelta, nodep, dtime, dmat, tnode, dtnode, steps, attempts, out,
+    DevBuf y, dep, arr, ypre, kap, kicu, wst, wmin, yint, lcoef, cbase, cdelta, nodep, dtime, dmat, tnode, dtnode, steps, attempts, out,
         ipool, epool, cvec, cvec_min, mpool, estructs, inst_ids;
     DevBuf fx_rec, fx_pool, fx_dirty;  // fix-up records of the return passes
     DevBuf node_order;                 // node-kernel lane slot -> node (empty: identity)
@@ -602,7 +607,11 @@ void build_edges(const mgo_graph_desc* g, EdgeStructHost& es, std::vector<double
             continue;
         }
         E ed{src, dst, c[0], mn ? mn[0] : 0.0, -1};
+        for (int q = 0; q < len; ++q) {
+            es.negative = es.negative || !(c[q] >= 0.0) || (mn && !(mn[q] >= 0.0));
+        }
         if (!uniform) {
+            es.uniform = false;
             ed.cidx = int(cvec.size() / size_t(nv));
             cvec.insert(cvec.end(), c, c + nv);
             if (mn) {
@@ -651,6 +660,20 @@ void build_edges(const mgo_graph_desc* g, EdgeStructHost& es, std::vector<double
         es.seq.push_back(e.s);
         es.seq.push_back(e.d);
         es.seq.push_back(ko);
+    }
+    // sums over every node's out-edges, in their order
+    const size_t w = es.uniform ? 1 : size_t(nv);
+    es.out_sum.assign(size_t(n) * w, 0.0);
+    if (g->edge_coeff_minimum) {
+        es.out_min_sum.assign(size_t(n) * w, 0.0);
+    }
+    for (auto& e : edges) {
+        for (size_t q = 0; q < w; ++q) {
+            es.out_sum[size_t(e.s) * w + q] += e.cidx < 0 ? e.cval : cvec[size_t(e.cidx) * size_t(nv) + q];
+            if (!es.out_min_sum.empty()) {
+                es.out_min_sum[size_t(e.s) * w + q] += e.cidx < 0 ? e.cmin : cvec_min[size_t(e.cidx) * size_t(nv) + q];
+            }
+        }
     }
 }
 
@@ -861,6 +884,11 @@ struct Batch {
                 build_class(ci, runs, idev);
             }
             inst_dev.upload(idev, stream);
+            for (ClassHost& C : classes) {
+                if (C.wst.p) {
+                    hip_check(launch_weights(C.launch, inst_dev.as<InstDev>(), inst_offset, stream), "return weights");
+                }
+            }
         }
         catch (...) {
             // an allocation failed part-way (a full serving arena): the uploads already queued must land
@@ -996,6 +1024,10 @@ struct Batch {
         struct StructOff {
             size_t in_ptr, out_ptr, split, seq, in_ent, out_ent;
             int64_t in_min = -1, out_min = -1; // offsets into mpool, -1 = no minimum
+            size_t in_src = 0, out_dst = 0;    // into ipool (uniform structures)
+            int64_t in_c = -1, out_c = -1;     // into mpool (uniform structures)
+            int64_t sum = -1, min_sum = -1;    // into mpool
+            bool uniform, negative;
             int n, num_edges;
         };
         std::vector<StructOff> soffs;
@@ -1005,11 +1037,14 @@ struct Batch {
         int64_t out_total = 0;
         int64_t fx_total  = 0;
         int64_t pool_slots = 0;
+        int wplanes        = 5;
+        bool any_icu = false, any_general = false;
         for (int ii : C.insts) {
             RunSpec& r    = runs[size_t(ii)];
             InstHost& I   = inst[size_t(ii)];
             const auto* g = r.g;
             inst_ids.push_back(ii);
+            bool icu = false, general = false;
             for (int v = 0; v < g->num_nodes; ++v) {
                 const size_t node = size_t(I.node_base) + size_t(v) * size_t(I.node_stride);
                 const double* sc  = g->node_scalars + size_t(v) * MGO_NUM_SCALARS;
@@ -1030,12 +1065,23 @@ struct Batch {
                 }
                 if (np.icu < DBL_MAX) {
                     np.flags |= NF_ICU_ACTIVE;
+                    icu = true;
                 }
                 if (np.det_start < np.det_end) {
                     np.flags |= NF_DETECTION;
                 }
                 for (int a = 0; a < G; ++a) {
-                    lane_coefficients(g, v, a, &lcoef[(node * G + size_t(a)) * NUM_LC]);
+                    double* lc = &lcoef[(node * G + size_t(a)) * NUM_LC];
+                    lane_coefficients(g, v, a, lc);
+                    // closed-form returns need nonnegative travelers (see return_body)
+                    for (int k = LC_E; k <= LC_ICR_R; ++k) {
+                        general = general || !(lc[k] >= 0.0);
+                    }
+                    const double out[] = {lc[LC_E], lc[LC_INS_ISY] + lc[LC_INS_R], lc[LC_ISY_ISEV] + lc[LC_ISY_R],
+                                          (lc[LC_ISEV_ICR] + lc[LC_ISEV_R]) + lc[LC_ISEV_D], lc[LC_ICR_D] + lc[LC_ICR_R]};
+                    for (double o : out) {
+                        general = general || !(r.cfg.dt_graph * o <= 1.0);
+                    }
                     for (int j = 0; j < G; ++j) {
                         const size_t k = (size_t(v) * G + size_t(a)) * G + size_t(j);
                         const double b = g->contact_baseline[k];
@@ -1137,6 +1183,32 @@ struct Batch {
                         so.out_min = int64_t(mpool.size());
                         mpool.insert(mpool.end(), es.out_min.begin(), es.out_min.end());
                     }
+                    auto pool = [&](const std::vector<double>& v) {
+                        const auto off = int64_t(mpool.size());
+                        mpool.insert(mpool.end(), v.begin(), v.end());
+                        return off;
+                    };
+                    so.uniform  = es.uniform;
+                    so.negative = es.negative;
+                    so.sum      = pool(es.out_sum);
+                    if (!es.out_min_sum.empty()) {
+                        so.min_sum = pool(es.out_min_sum);
+                    }
+                    if (es.uniform) {
+                        so.in_src  = ipool.size();
+                        so.out_dst = so.in_src + es.in_ent.size();
+                        for (auto* ent : {&es.in_ent, &es.out_ent}) {
+                            std::vector<double> cv;
+                            for (const EdgeEnt& e : *ent) {
+                                ipool.push_back(e.nbr);
+                                cv.push_back(e.cval);
+                            }
+                            (ent == &es.in_ent ? so.in_c : so.out_c) = pool(cv);
+                        }
+                    }
+                    else {
+                        wplanes = 7;
+                    }
                     sidx = int(soffs.size());
                     soffs.push_back(so);
                     struct_cache[key] = sidx;
@@ -1144,8 +1216,13 @@ struct Batch {
                 if (soffs[size_t(sidx)].num_edges > 0) {
                     D.estruct   = sidx;
                     I.has_edges = true;
+                    general     = general || soffs[size_t(sidx)].negative;
+                    any_icu     = any_icu || icu;
+                    any_general = any_general || general;
                 }
             }
+            D.icu     = icu ? 1 : 0;
+            D.general = (D.estruct >= 0 && general) ? 1 : 0;
             D.fx_base      = fx_total;
             D.fx_pool_base = int64_t(pool_slots) * FX_SLOTS * G * NC;
             if (D.estruct >= 0) {
@@ -1181,12 +1258,25 @@ struct Batch {
         up(C.y0, y);
         C.tnode0  = tnode;
         C.dtnode0 = dtnode;
-        C.snap.alloc(N * G * SNAP_STRIDE * sizeof(double));
-        C.ypre.alloc(y.size() * sizeof(double));
-        C.rc.alloc(N * G * RC_STRIDE * sizeof(double));
+        if (!soffs.empty()) {
+            const size_t np = N * size_t(G);
+            for (DevBuf* b : {&C.dep, &C.arr, &C.ypre}) {
+                b->alloc(np * NC * sizeof(double));
+            }
+            C.kap.alloc(np * sizeof(double));
+            if (any_icu) {
+                C.kicu.alloc(np * sizeof(double2));
+            }
+            C.wst.alloc(np * size_t(wplanes) * sizeof(double2));
+            if (!outd.nodes.empty()) {
+                C.wmin.alloc(np * size_t(wplanes) * sizeof(double2));
+            }
+            device_bytes += C.dep.bytes + C.arr.bytes + C.ypre.bytes + C.kap.bytes + C.kicu.bytes + C.wst.bytes +
+                            C.wmin.bytes;
+        }
         C.yint.alloc(N * G * YINT_STRIDE * sizeof(double));
         hip_check(hipMemsetAsync(C.yint.p, 0xff, C.yint.bytes, stream), "clear yint"); // NaN weights: no step yet
-        device_bytes += C.snap.bytes + C.ypre.bytes + C.rc.bytes + C.yint.bytes;
+        device_bytes += C.yint.bytes;
         up(C.lcoef, lcoef);
         up(C.cbase, cbase);
         up(C.cdelta, cdelta);
@@ -1236,6 +1326,18 @@ struct Batch {
             sd.cvec_min             = C.cvec_min.as<double>();
             sd.in_min               = so.in_min >= 0 ? C.mpool.as<double>() + so.in_min : nullptr;
             sd.out_min              = so.out_min >= 0 ? C.mpool.as<double>() + so.out_min : nullptr;
+            const double* mb        = C.mpool.as<double>();
+            auto at                 = [&](int64_t off) {
+                return off >= 0 ? mb + off : nullptr;
+            };
+            sd.in_src               = so.uniform ? ib + so.in_src : nullptr;
+            sd.out_dst              = so.uniform ? ib + so.out_dst : nullptr;
+            sd.in_c                 = at(so.in_c);
+            sd.out_c                = at(so.out_c);
+            sd.out_sum              = so.uniform ? at(so.sum) : nullptr;
+            sd.out_min_sum          = so.uniform ? at(so.min_sum) : nullptr;
+            sd.out_vsum             = so.uniform ? nullptr : at(so.sum);
+            sd.out_vmin_sum         = so.uniform ? nullptr : at(so.min_sum);
             sd.n                    = so.n;
             sd.num_edges            = so.num_edges;
         }
@@ -1279,9 +1381,14 @@ struct Batch {
         d.G         = G;
         d.num_nodes = C.num_nodes;
         d.y         = C.y.as<double>();
-        d.snap      = C.snap.as<double>();
-        d.ypre      = C.ypre.as<double>();
-        d.rc        = C.rc.as<double>();
+        d.wplanes   = wplanes;
+        d.dep       = C.dep.as<double2>();
+        d.arr       = C.arr.as<double2>();
+        d.ypre      = C.ypre.as<double2>();
+        d.kap       = C.kap.as<double>();
+        d.kicu      = C.kicu.as<double2>();
+        d.wst       = C.wst.as<double2>();
+        d.wmin      = C.wmin.as<double2>();
         d.yint      = C.yint.as<double>();
         d.lcoef     = C.lcoef.as<double>();
         d.cbase     = C.cbase.as<double>();
@@ -1326,6 +1433,7 @@ struct Batch {
         ld.G           = G;
         ld.kind        = C.kind;
         ld.npi         = (C.npi.nodes0.empty() && C.oute.nodes0.empty()) ? 0 : 1;
+        ld.general     = any_general ? 1 : 0;
         ld.cyc         = cyc.as<int32_t>();
     }
 

@@ -6,14 +6,16 @@
 // launch covers the segments of one class through a block -> segment table; kernels are specialised
 // per (G, integrator). Within a segment:
 //   lane slot   = node * G + g   (one GPU lane per (node, age group); 64/G nodes per wavefront)
-//   y, ypre             [node][g][10]          state, pre-return state
+//   y                   [node][g][10]          state
 //   yint                [node][g][YINT_STRIDE] state before the last step of a phase ending on an output day
-//   snap                [node][g][SNAP_STRIDE] departure row: snapshot (10), ISy mobility factor, commuter
-//                                              nondetection factor at the departure time
+//   dep, arr, ypre      [5][node][g] double2   planes of compartment pairs: departure row (travelers per unit
+//                                              of coefficient), arrivals of the last departure, pre-return state
 //   lcoef               [node][g][NUM_LC]      per-lane rate coefficients (see LaneCoef)
 //   cbase, cdelta       [node][g][G]           contact row B_g., B_g. - M_g.
-//   rc                  [node][g][RC_STRIDE]   return coefficients of the node as a destination, frozen at
-//                                              the departure time (see RetCoef)
+//   kap                 [node][g]              force of infection on returning travelers, frozen at the
+//                                              departure time
+//   kicu                [node][g] double2      their ICU-adjusted ISev rates (classes with an ICU limit)
+//   wst, wmin           [wplanes][node][g]     sums over the out-edges of coefficient (minimum) x rate
 //   nodep               [node]                 scalar parameters + instance index
 //   tnode, dtnode       [node]                 integrator time and carried step size
 // Instances (one graph simulation each) live in a device table; a clock kernel turns the instance
@@ -31,6 +33,8 @@
 #pragma once
 
 #include <cstdint>
+
+#include <hip/hip_vector_types.h>
 
 namespace mgo
 {
@@ -64,30 +68,6 @@ enum LaneCoef : int {
     LC_TISEV,      // TimeInfectedSevere
     NUM_LC
 };
-
-// Return coefficients of a destination lane, computed from its post-departure state (the `pop` of
-// calculate_mobility_returns, metapopulation_mobility_instant.h:460-471) at the departure time.
-enum RetCoef : int {
-    RC_KAPPA = 0, // season(t_dep) * tp * sum_j C_gj(t_dep) w_j(pop): S->E rate per traveler in S
-    RC_E,
-    RC_INS_ISY,
-    RC_INS_R,
-    RC_ISY_ISEV,
-    RC_ISY_R,
-    RC_ISEV_ICR,  // ICU-adjusted at the departure state
-    RC_ISEV_R,
-    RC_ISEV_D,    // ICU-adjusted at the departure state
-    RC_ICR_D,
-    RC_ICR_R,
-    RC_STRIDE = 12
-};
-
-// departure row of a lane: the snapshot of SimulationNode::m_last_state, the ISy mobility factor
-// (get_mobility_factors) and the commuter nondetection factor (test_commuters) at the departure time;
-// 96 bytes, read with 16-byte loads
-constexpr int SNAP_FAC    = 10;
-constexpr int SNAP_ND     = 11;
-constexpr int SNAP_STRIDE = 12;
 
 // last step of a lane's phase that ends on an output day d: the state before that step and the weight
 // (d - t_prev) / (t_end - t_prev) of interpolate_simulation_result (analyze_result.h:235-252), or -1 when the
@@ -166,17 +146,21 @@ struct InstDev {
     // negative-value fix-up iteration of the current return phase (see return_walk)
     int64_t fx_base;      // first in-edge record pair of this instance in SegDev::fx_rec (in pairs)
     int64_t fx_pool_base; // first double of this instance's slots in SegDev::fx_pool
-    int32_t fx_pass;      // pass being run (0 = the first return walk)
-    int32_t fx_state;     // 0 first pass, 1 iterating, 2 sequential replay needed, 3 settled
-    int32_t fx_changed;   // set by a pass in which a fix-up record changed
+    int32_t fx_neg;       // negative travelers left at the last departure: their returns walk the edges
+    int32_t fx_state;     // 2: the record pool is full, sequential replay needed
+    int32_t fx_changed;   // set when nodes are marked to walk their edges in the next pass
     int32_t fx_count;     // pool slots used in this return phase
     int32_t fx_passes;    // extra passes run so far (statistics)
     int32_t fx_sequential; // resolve fix-ups with the sequential replay only
     int32_t seg;          // segment (index into LaunchDev::segs of its class) holding the nodes
     int32_t fx_epoch;     // record tag of pass 0 of the current return phase (grows by FX_EPOCH_STEP)
     int32_t node_stride;  // segment index of local node v = node_base + v * node_stride (see Tiling)
+    int32_t icu;          // some node has an ICU limit: the ISev rates of the returns depend on the state
+    int32_t general;      // every return walks the edges: some edge coefficient or rate is negative, or a rate
+                          // exceeds 1 / dt_graph (see return_body)
     int32_t pad3;
 };
+static_assert(sizeof(InstDev) % 8 == 0, "instance records are copied as 8-byte words");
 
 // Fix-up records. Each in-edge keeps two tagged versions {tag, slot}; tag = fx_epoch + pass of the pass
 // that wrote it, slot = pool slot of the fixed traveler vector or -1 (unfixed). A pass p reads the newest
@@ -191,13 +175,15 @@ constexpr int FX_SLOTS      = 1024; // pool slots per instance and return phase
 constexpr int FX_MAX_PASSES = 8;    // passes before falling back to the sequential replay
 constexpr int FX_EPOCH_STEP = 16;   // > FX_MAX_PASSES
 
-// Cycle flags, written by the clock kernel (cleared, then set by the instances) and by fixup_check: which
-// phases of this half-day cycle have work anywhere in the batch, so that the launches of idle phases (the
-// departure kernel in a return cycle, fix-up passes nobody needs) exit at once.
-constexpr int CYC_DEPART = 0;                    // some instance departs
-constexpr int CYC_RETURN = 1;                    // some instance returns
-constexpr int CYC_PASS0  = 2;                    // CYC_PASS0 + p: some instance runs fix-up pass p
-constexpr int CYC_FLAGS  = CYC_PASS0 + FX_MAX_PASSES;
+constexpr int SETTLE_BLOCK  = 512;  // threads of an instance's block (eight walks at a time)
+constexpr int SETTLE_LIST   = 1024; // marked nodes an instance's block holds in LDS at a time
+
+// Cycle flags, written by the clock kernel (cleared, then set by the instances): which phases of this half-day
+// cycle have work anywhere in the batch, so that the launches of idle phases (the departure kernel in a return
+// cycle) exit at once.
+constexpr int CYC_DEPART = 0; // some instance departs
+constexpr int CYC_RETURN = 1; // some instance returns
+constexpr int CYC_FLAGS  = 2;
 
 // CSR edge structure of one graph (node indices local to the instance). In-edges of node v are sorted
 // by source; in_split[v] = number of in-edges whose source < v, so walking
@@ -223,6 +209,17 @@ struct EdgeStructDev {
     const double* in_min;    // minimum coefficient of each uniform in-entry, or NULL (zero)
     const double* out_min;   // minimum coefficient of each uniform out-entry, or NULL (zero)
     const double* cvec_min;  // minimum coefficient vectors [k][10*G] (parallel to cvec), or NULL (zero)
+    // graphs with one coefficient per edge: neighbours and coefficients of the in- and out-entries, and per node
+    // the sums of its out-edges' coefficients and minima (NULL: zero)
+    const int32_t* in_src;
+    const int32_t* out_dst;
+    const double* in_c;
+    const double* out_c;
+    const double* out_sum;
+    const double* out_min_sum;
+    // graphs with coefficient vectors (out_sum NULL): the sums per compartment [n][10*G]
+    const double* out_vsum;
+    const double* out_vmin_sum;
     int32_t n;
     int32_t num_edges;
 };
@@ -230,10 +227,16 @@ struct EdgeStructDev {
 struct SegDev {
     int32_t G;
     int32_t num_nodes;
+    int32_t wplanes;               // planes of wst and wmin: 5 (one coefficient per edge) or 7
+    int32_t pad;
     double* y;
-    double* snap;
-    double* ypre;
-    double* rc;
+    double2* dep;
+    double2* arr;
+    double2* ypre;
+    double* kap;
+    double2* kicu;                 // NULL: no node of the class has an ICU limit
+    double2* wst;
+    double2* wmin;                 // NULL: no out-dampings in the class
     double* yint;                  // [node][g][YINT_STRIDE] last step before a phase-end output day
     const double* lcoef;
     const double* cbase;
@@ -275,7 +278,7 @@ struct LaunchDev {
     int32_t G;                  // age groups of every segment, or 0: segments differ (mixed kernels)
     int32_t kind;
     int32_t npi;                // some node has dynamic NPIs (per-G kernels only)
-    int32_t pad;
+    int32_t general;            // some instance's returns walk the edges (InstDev::general)
     int32_t* cyc;               // [CYC_FLAGS] cycle flags of the batch (or NULL: every phase runs its checks)
 };
 

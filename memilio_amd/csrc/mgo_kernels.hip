@@ -9,13 +9,15 @@
 // Kernels per half-day cycle (GraphSimulation::advance, cpp/memilio/mobility/graph_simulation.h:101-120):
 //   clock_kernel       per instance: step size, edge action and output day of this cycle
 //   node_phase<G,K>    per node lane: SystemIntegrator::advance to t+dt with integrator K; writes the
-//                      departure row (departure cycles) or the pre-return state and the return
-//                      coefficients (return cycles)
-//   depart_phase<G>    per node lane: the node's departures over all incident edges, walked in the
-//                      reference's edge order (deterministic segmented sum, no atomics)
-//   return_phase<G>    per node lane: the returns with the negative-value fix-up, in parallel passes over
-//                      the nodes whose inputs changed (fixup_check between passes)
-//   replay_phase<G>    per flagged instance: sequential return pass with the negative-value fix-up
+//                      departure row and takes the departing travelers off (departure cycles) or writes the
+//                      pre-return state and the return coefficients (return cycles)
+//   depart_phase<G>    per node lane: the arriving travelers, one sum over the node's in-edges in the
+//                      reference's edge order (deterministic, no atomics)
+//   return_phase<G>    per node lane: the returns in closed form; marks the nodes on which the negative-value
+//                      fix-up can act
+//   walk_phase<G>      per node lane of the instances whose returns need the edge walk (see InstDev::general)
+//   settle_phase<G>    per instance: marked nodes walk their edges with the fix-up, in passes over the nodes
+//                      whose inputs changed; sequential replay where these do not settle
 //
 // The file is compiled once per shard (MGO_SHARD, see memilio_amd/build.py), in parallel: shard 0 holds the
 // launch dispatch and the kernels without a G, shards 1..8 the kernels of that G, shards 9..12 the node kernel
@@ -25,6 +27,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/mgo.h"
 #include "mgo_internal.h"
@@ -34,6 +37,31 @@ namespace mgo
 {
 
 #define MGO_PI 3.14159265358979323846
+
+// Segment and edge-structure descriptors do not change during a launch and are read from the constant address
+// space: the pointers they hold are then known to be global. Read as ordinary memory they are generic, and every
+// access through them is a FLAT instruction, which occupies the LDS path too and is waited for with it.
+using Seg = const __attribute__((address_space(4))) SegDev;
+using Est = const __attribute__((address_space(4))) EdgeStructDev;
+
+__device__ __forceinline__ Seg* segment(const LaunchDev& ld, int seg)
+{
+    return (Seg*)(ld.segs + seg);
+}
+__device__ __forceinline__ Est& edge_struct(Seg& c, int k)
+{
+    return *(Est*)(c.estructs + k);
+}
+// pointers held by other records (instances, node parameters) are cast to global where they are used
+using gdouble = __attribute__((address_space(1))) double;
+
+// orders a wavefront's LDS accesses across its lanes (LDS instructions of a wavefront complete in order)
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // cpp/memilio/math/smoother.h:46-60
 __device__ __forceinline__ double smoother_cosine(double x, double xl, double xr, double yl, double yr)
@@ -131,7 +159,7 @@ struct Lane {
 
 // Effective contact row C(t)_age,. = B - D(t) o (B - M) (contact_matrix.h:190-194, damping.h:381-396)
 template <int G>
-__device__ __forceinline__ void contact_row(const SegDev& c, Lane<G>& L, double t)
+__device__ __forceinline__ void contact_row(Seg& c, Lane<G>& L, double t)
 {
     const double* B = c.cbase + (size_t(L.node) * G + L.age) * G;
     if (!(L.np.flags & NF_DAMPED)) {
@@ -141,15 +169,15 @@ __device__ __forceinline__ void contact_row(const SegDev& c, Lane<G>& L, double 
         }
         return;
     }
-    const double* tk = L.np.damp_time;
-    int k            = 1;
+    const gdouble* tk = (const gdouble*)L.np.damp_time;
+    int k             = 1;
     while (k < L.np.damp_cnt - 1 && !(tk[k] > t)) {
         ++k;
     }
     const double xr    = tk[k];
     const double xl    = xr - 1.0;
-    const double* Dl   = L.np.damp_mat + (size_t(k - 1) * G + L.age) * G;
-    const double* Dr   = L.np.damp_mat + (size_t(k) * G + L.age) * G;
+    const gdouble* Dl  = (const gdouble*)L.np.damp_mat + (size_t(k - 1) * G + L.age) * G;
+    const gdouble* Dr  = (const gdouble*)L.np.damp_mat + (size_t(k) * G + L.age) * G;
     const double* Dd   = c.cdelta + (size_t(L.node) * G + L.age) * G;
     const bool left    = t <= xl;
     const bool right   = t >= xr;
@@ -204,7 +232,7 @@ __device__ __forceinline__ double stage_season(const Lane<G>& L, const StageSeas
 // w_j = divN_j * (rel_j pop[INS_j] + risk_j pop[ISy_j]) (model.h:99-145, factored over j). Also returns
 // the ICU-adjusted ISev->ICr / ISev->D coefficients (model.h:147-152, 196-204).
 template <int G>
-__device__ __forceinline__ double force_of_infection(const SegDev& c, Lane<G>& L, const double (&pop)[NC], double t,
+__device__ __forceinline__ double force_of_infection(Seg& c, Lane<G>& L, const double (&pop)[NC], double t,
                                                      double season, double& c_icr, double& c_d)
 {
     double risk = L.c[LC_RISK];
@@ -274,7 +302,7 @@ __device__ __forceinline__ void flows_to_dydt(const double (&y)[NC], double kapp
 
 // Right-hand side of the node ODE, pop == y (osecir::Model::get_flows + FlowModel::get_derivatives)
 template <int G>
-__device__ __forceinline__ void rhs(const SegDev& c, Lane<G>& L, const double (&y)[NC], double t, double season,
+__device__ __forceinline__ void rhs(Seg& c, Lane<G>& L, const double (&y)[NC], double t, double season,
                                     double (&dy)[NC])
 {
     double c_icr, c_d;
@@ -301,7 +329,7 @@ constexpr double E1 = 37.0 / 378.0 - 2825.0 / 27648.0, E3 = 250.0 / 621.0 - 1857
 
 // One Cash-Karp step from (y, k1 = f(y, t)) with step h: 5th-order solution in yo, embedded error in er.
 template <int G>
-__device__ __forceinline__ void cash_karp_stages(const SegDev& c, Lane<G>& L, const double (&y)[NC],
+__device__ __forceinline__ void cash_karp_stages(Seg& c, Lane<G>& L, const double (&y)[NC],
                                                  const double (&k1)[NC], double t, double h, double (&yo)[NC],
                                                  double (&er)[NC], bool want_err, double& season_end)
 {
@@ -364,7 +392,7 @@ constexpr double D1 = BH1 - BL1, D3 = BH3 - BL3, D4 = BH4 - BL4, D5 = BH5 - BL5,
 } // namespace rkf
 
 template <int G>
-__device__ __forceinline__ void rkf45_stages(const SegDev& c, Lane<G>& L, const double (&y)[NC],
+__device__ __forceinline__ void rkf45_stages(Seg& c, Lane<G>& L, const double (&y)[NC],
                                              const double (&k1)[NC], double t, double h, double (&yo)[NC],
                                              double (&er)[NC], double& season_end)
 {
@@ -408,7 +436,7 @@ __device__ __forceinline__ void rkf45_stages(const SegDev& c, Lane<G>& L, const 
 }
 
 template <int G>
-__device__ __forceinline__ const SegDev* load_lane(const LaunchDev& ld, Lane<G>& L, double* wx)
+__device__ __forceinline__ Seg* load_lane(const LaunchDev& ld, Lane<G>& L, double* wx)
 {
     L.wx = wx + (threadIdx.x / WAVE) * WAVE;
     L.ws = wx + BLOCK + (threadIdx.x / WAVE) * WAVE;
@@ -421,7 +449,7 @@ __device__ __forceinline__ const SegDev* load_lane(const LaunchDev& ld, Lane<G>&
     if (seg < 0) {
         return nullptr;
     }
-    const SegDev* c = ld.segs + seg;
+    Seg* c = segment(ld, seg);
     const int wave  = (lb - ld.block_first[seg]) * (BLOCK / WAVE) + int(threadIdx.x) / WAVE;
     const int lane  = int(threadIdx.x) % WAVE;
     const int grp   = lane / G;
@@ -473,7 +501,6 @@ __device__ __forceinline__ void clock_one(InstDev& I)
     I.c_active  = 0;
     I.c_action  = 0;
     I.c_out_day = -1;
-    I.fx_pass   = 0;
     I.fx_state  = 0;
     I.fx_changed = 0;
     I.fx_count   = 0;
@@ -508,6 +535,7 @@ __device__ __forceinline__ void clock_one(InstDev& I)
             }
             else {
                 I.c_action = 1;
+                I.fx_neg   = 0;
                 I.pending  = 1;
                 I.t_dep    = tn;
                 I.ret_time = tn + step;
@@ -551,9 +579,9 @@ static __global__ void __launch_bounds__(1024) clock_kernel(InstDev* inst, int n
 }
 
 // daily output of local node v: [day][v][g][10]
-__device__ __forceinline__ double* out_ptr(const InstDev& I, int v, int age, int G, int day)
+__device__ __forceinline__ gdouble* out_ptr(const InstDev& I, int v, int age, int G, int day)
 {
-    return I.out + (size_t(day) * I.num_nodes + v) * size_t(G * NC) + size_t(age) * NC;
+    return (gdouble*)I.out + (size_t(day) * I.num_nodes + v) * size_t(G * NC) + size_t(age) * NC;
 }
 
 // linear_interpolation (math/interpolation.h:44-48): y_a + w (y_b - y_a), rounded as the reference (no FMA)
@@ -569,12 +597,12 @@ __device__ __forceinline__ double lerp_ref(double ya, double yb, double w)
 // state before the node's last step and y when that step ends at or after d (weight 1 when it ends on d);
 // else y, the last value so far: then the next phase's first step encloses d and overwrites the day.
 template <int G>
-__device__ __forceinline__ void write_phase_end_day(const SegDev& c, const InstDev& I, size_t lane, int v, int age,
+__device__ __forceinline__ void write_phase_end_day(Seg& c, const InstDev& I, size_t lane, int v, int age,
                                                     const double (&y)[NC])
 {
     const double* pr = c.yint + lane * YINT_STRIDE;
     const double w   = pr[YINT_W];
-    double* op       = out_ptr(I, v, age, G, I.c_out_day);
+    gdouble* op       = out_ptr(I, v, age, G, I.c_out_day);
     if (w >= 0.0) {
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
@@ -595,27 +623,113 @@ __device__ __forceinline__ size_t seg_node(const InstDev& I, int v)
     return size_t(I.node_base) + size_t(v) * size_t(I.node_stride);
 }
 
+// Plane arrays (SegDev::dep, arr, ypre, wst): every compartment pair is one 16-byte plane over the segment's
+// lanes, so a wavefront's access to it is one contiguous run.
+// ten compartments of a lane from / to planes
+__device__ __forceinline__ void load_planes(const double2* p, size_t stride, size_t lane, double (&v)[NC])
+{
+#pragma unroll
+    for (int q = 0; q < NC / 2; ++q) {
+        const double2 t = p[size_t(q) * stride + lane];
+        v[2 * q]        = t.x;
+        v[2 * q + 1]    = t.y;
+    }
+}
+__device__ __forceinline__ void store_planes(double2* p, size_t stride, size_t lane, const double (&v)[NC])
+{
+#pragma unroll
+    for (int q = 0; q < NC / 2; ++q) {
+        p[size_t(q) * stride + lane] = double2{v[2 * q], v[2 * q + 1]};
+    }
+}
+
 // Return coefficients of the lane's node as a destination (calculate_mobility_returns,
-// metapopulation_mobility_instant.h:460-471): rates and force of infection of the state pop at the departure
-// time, frozen for the Euler step of the returning travelers.
+// metapopulation_mobility_instant.h:460-471): the force of infection and the ICU-adjusted rates of the state
+// pop at the departure time, frozen for the Euler step of the returning travelers (the other rates are lane
+// constants).
 template <int G>
-__device__ __forceinline__ void return_coefficients(const SegDev& c, Lane<G>& L, const InstDev& I,
+__device__ __forceinline__ void return_coefficients(Seg& c, Lane<G>& L, const InstDev& I,
                                                     const double (&pop)[NC])
 {
     double c_icr, c_d;
     const double kappa = force_of_infection<G>(c, L, pop, I.c_tdep, season_at<G>(L, I.c_tdep), c_icr, c_d);
-    double* rc         = c.rc + (size_t(L.node) * G + L.age) * RC_STRIDE;
-    rc[RC_KAPPA]       = kappa;
-    rc[RC_E]           = L.c[LC_E];
-    rc[RC_INS_ISY]     = L.c[LC_INS_ISY];
-    rc[RC_INS_R]       = L.c[LC_INS_R];
-    rc[RC_ISY_ISEV]    = L.c[LC_ISY_ISEV];
-    rc[RC_ISY_R]       = L.c[LC_ISY_R];
-    rc[RC_ISEV_ICR]    = c_icr;
-    rc[RC_ISEV_R]      = L.c[LC_ISEV_R];
-    rc[RC_ISEV_D]      = c_d;
-    rc[RC_ICR_D]       = L.c[LC_ICR_D];
-    rc[RC_ICR_R]       = L.c[LC_ICR_R];
+    const size_t lane  = size_t(L.node) * G + L.age;
+    c.kap[lane]        = kappa;
+    if (c.kicu) {
+        c.kicu[lane] = double2{c_icr, c_d};
+    }
+}
+
+// Coefficient at the departure time, B - D (B - M) (DampingMatrixExpression::get_matrix_at,
+// contact_matrix.h:190-194), of an edge or of a sum over edges of one source. D: the source's damping factor.
+__device__ __forceinline__ double damped(double b, double m, double D)
+{
+#pragma clang fp contract(off)
+    return b - D * (b - m);
+}
+
+// Departures of the lane's node at c_t1 (metapopulation_mobility_instant.h:605-621): the departure row (the
+// traveler vector per unit of coefficient: SimulationNode::m_last_state with the ISy mobility factor and the
+// commuter nondetection factor), and the node's state without all its travelers. Every out-edge takes the same
+// row times its coefficient, so the sum over the out-edges is the row times the sum of the coefficients (a
+// constant of the graph): no walk over the out-edges.
+template <int G>
+__device__ __forceinline__ void leave(Seg& c, const Lane<G>& L, InstDev& I, double fac, double nd, double D,
+                                      double (&y)[NC])
+{
+#pragma clang fp contract(off)
+    Est& es = edge_struct(c, I.estruct);
+    const size_t lane       = size_t(L.node) * G + L.age;
+    double row[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        row[i] = y[i];
+    }
+    row[ISY] = row[ISY] * fac;
+    double gone[NC];
+    const int v = L.np.local;
+    if (es.out_sum) {
+        double sum = es.out_sum[v];
+        if (D != 0.0) {
+            sum = damped(sum, es.out_min_sum ? es.out_min_sum[v] : 0.0, D);
+        }
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            gone[i] = row[i] * sum;
+        }
+    }
+    else {
+        const size_t off = (size_t(v) * G + L.age) * NC;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            double sum = es.out_vsum[off + i];
+            if (D != 0.0) {
+                sum = damped(sum, es.out_vmin_sum ? es.out_vmin_sum[off + i] : 0.0, D);
+            }
+            gone[i] = row[i] * sum;
+        }
+    }
+    if (nd != 1.0) {
+        // test_commuters on the source: detected commuters stay home as confirmed cases
+        y[INS] -= gone[INS] * (1 - nd);
+        y[INSC] += gone[INS] * (1 - nd);
+        y[ISY] -= gone[ISY] * (1 - nd);
+        y[ISYC] += gone[ISY] * (1 - nd);
+        gone[ISY] *= nd;
+        gone[INS] *= nd;
+        row[ISY] *= nd;
+        row[INS] *= nd;
+    }
+    bool odd = !(D >= 0.0 && D <= 1.0);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        y[i] -= gone[i];
+        odd = odd || !(row[i] >= 0.0);
+    }
+    store_planes(c.dep, size_t(c.num_nodes) * G, lane, row);
+    if (odd) {
+        I.fx_neg = 1; // negative travelers: the returns of this departure walk their edges (every writer stores 1)
+    }
 }
 
 // ------------------------------------------------------------------------------- dynamic NPIs
@@ -625,7 +739,7 @@ __device__ __forceinline__ void return_coefficients(const SegDev& c, Lane<G>& L,
 // group implements the NPI on the node's damping list and cache (mgo_npi.h). Returns true in `changed`
 // when the contact matrix changed.
 template <int G>
-__device__ double npi_piece(const SegDev& c, Lane<G>& L, InstDev& I, const double (&y)[NC], double t, double tmax,
+__device__ double npi_piece(Seg& c, Lane<G>& L, InstDev& I, const double (&y)[NC], double t, double tmax,
                             bool& changed)
 {
     NpiNode* nn         = c.npi + L.node;
@@ -696,7 +810,7 @@ __device__ double npi_piece(const SegDev& c, Lane<G>& L, InstDev& I, const doubl
 // directive; begin t, end t + duration, per-group mobility dampings), then on a departure the damping factor
 // D of the lane's age group at t (Dampings::get_matrix_at, damping.h:381-396) for the edge kernels.
 template <int G>
-__device__ void out_damping(const SegDev& c, Lane<G>& L, InstDev& I, const double (&y)[NC])
+__device__ double out_damping(Seg& c, Lane<G>& L, InstDev& I, const double (&y)[NC])
 {
     NpiNode* od    = c.out_npi + L.node;
     const double t = I.c_t1;
@@ -760,7 +874,9 @@ __device__ void out_damping(const SegDev& c, Lane<G>& L, InstDev& I, const doubl
             d = 0.5 * (Dl - Dr) * cos(MGO_PI / (xr - xl) * (t - xl)) + 0.5 * (Dl + Dr);
         }
         c.out_d[size_t(L.node) * G + L.age] = d;
+        return d;
     }
+    return 0.0;
 }
 
 // ------------------------------------------------------------------------------- node phase
@@ -775,11 +891,11 @@ template <int G, int K, bool NPI = false>
 __device__ __forceinline__ void node_body(const LaunchDev& ld, InstDev* __restrict__ inst, double* wx)
 {
     Lane<G> L;
-    const SegDev* cp = load_lane<G>(ld, L, wx);
+    Seg* cp = load_lane<G>(ld, L, wx);
     if (!cp) {
         return;
     }
-    const SegDev& c = *cp;
+    Seg& c = *cp;
     InstDev& I = inst[L.np.inst];
     if (!I.c_active) {
         return;
@@ -980,7 +1096,7 @@ __device__ __forceinline__ void node_body(const LaunchDev& ld, InstDev* __restri
                     const double dd = double(next_day + I.day0);
                     if (dd > ta) {
                         const double w = (dd - ta) / (t - ta);
-                        double* op     = out_ptr(I, L.np.local, L.age, G, next_day);
+                        gdouble* op     = out_ptr(I, L.np.local, L.age, G, next_day);
 #pragma unroll
                         for (int i = 0; i < NC; ++i) {
                             op[i] = lerp_ref(y[i], yo[i], w);
@@ -1021,46 +1137,38 @@ __device__ __forceinline__ void node_body(const LaunchDev& ld, InstDev* __restri
         need_k1 = true;
     }
     dt = fmax(dt, dt_restore);
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yp[i] = y[i];
-    }
     if (L.age == 0) {
         c.tnode[L.node]  = t;
         c.dtnode[L.node] = dt;
         c.steps[L.node] += nsteps;
         c.attempts[L.node] += natt;
     }
-    const size_t off = (size_t(L.node) * G + L.age) * NC;
+    double D = 0.0;
     if (NPI && (L.np.flags & NF_OUT_DAMP) && I.c_action != 0) {
-        out_damping<G>(c, L, I, y);
+        D = out_damping<G>(c, L, I, y);
+    }
+    if (I.c_action == 2) {
+        store_planes(c.ypre, size_t(c.num_nodes) * G, size_t(L.node) * G + L.age, y);
+        return; // the return phase writes the state and the day
     }
     if (I.c_action == 1) {
-        // departure row: SimulationNode::m_last_state, the ISy mobility factor and the commuter
-        // nondetection factor at the departure time
-        double* row = c.snap + (size_t(L.node) * G + L.age) * SNAP_STRIDE;
-#pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            row[i] = y[i];
-        }
-        row[SNAP_FAC] = mobility_factor<G>(L, y);
-        row[SNAP_ND]  = (L.np.flags & NF_DETECTION) ? detect_nondetection(L.np, I.c_t1) : 1.0;
-    }
-    else if (I.c_action == 2) {
-#pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            c.ypre[off + i] = y[i];
-        }
+        // the departure phase adds the arrivals and writes the day
+        leave<G>(c, L, I, mobility_factor<G>(L, y),
+                 (L.np.flags & NF_DETECTION) ? detect_nondetection(L.np, I.c_t1) : 1.0, D, y);
     }
     else if (I.c_out_day >= 0) {
         write_phase_end_day<G>(c, I, size_t(L.node) * G + L.age, L.np.local, L.age, y);
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        yp[i] = y[i];
     }
 }
 
 // ------------------------------------------------------------------------------- edge phase
 // Lane -> (segment, node, age group) without loading the lane's coefficients (edge kernels need none).
 template <int G>
-__device__ __forceinline__ const SegDev* lane_map(const LaunchDev& ld, int& node, int& age, int& base)
+__device__ __forceinline__ Seg* lane_map(const LaunchDev& ld, int& node, int& age, int& base)
 {
     constexpr int NPW = WAVE / G;
     const int lb      = xcd_block();
@@ -1071,7 +1179,7 @@ __device__ __forceinline__ const SegDev* lane_map(const LaunchDev& ld, int& node
     if (seg < 0) {
         return nullptr;
     }
-    const SegDev* c = ld.segs + seg;
+    Seg* c = segment(ld, seg);
     const int wave  = (lb - ld.block_first[seg]) * (BLOCK / WAVE) + int(threadIdx.x) / WAVE;
     const int lane  = int(threadIdx.x) % WAVE;
     const int grp   = lane / G;
@@ -1084,72 +1192,100 @@ __device__ __forceinline__ const SegDev* lane_map(const LaunchDev& ld, int& node
     return c;
 }
 
-// departure row of lane slot `lane` (16-byte loads)
-__device__ __forceinline__ void load_row(const double* snap, size_t lane, double (&r)[SNAP_STRIDE])
-{
-    const double2* p = reinterpret_cast<const double2*>(snap + lane * SNAP_STRIDE);
-#pragma unroll
-    for (int i = 0; i < SNAP_STRIDE / 2; ++i) {
-        const double2 v = p[i];
-        r[2 * i]        = v.x;
-        r[2 * i + 1]    = v.y;
-    }
-}
+// coefficient of entry k of the in- or out-entries for compartments i of age group `age`, at the departure time
+struct EdgeCoef {
+    double c;          // uniform coefficient
+    const double* vec; // else the coefficients of the lane's age group, and their minima (or NULL)
+    const double* vmin;
+    double D;
+};
 
-// traveler vector of one edge from its source's departure row (metapopulation_mobility_instant.h:608-615:
-// snapshot * coefficients * mobility factors, then test_commuters' nondetection on INS and ISy if with_nd).
-// The coefficients at the departure time are B - D (B - M) (DampingMatrixExpression::get_matrix_at,
-// contact_matrix.h:190-194) with the source's out-edge damping factor D; mn: the entry's uniform minimum
-// (entry index k of the in- or out-entries), or NULL.
-__device__ __forceinline__ void traveler_vector(const EdgeStructDev& es, const EdgeEnt& e, const double* mn, int k,
-                                                double D, const double (&row)[SNAP_STRIDE], int G, int age,
-                                                bool with_nd, double (&m)[NC])
+__device__ __forceinline__ EdgeCoef edge_coef(Est& es, const EdgeEnt& e, const double* mn, int k,
+                                              double D, int G, int age)
 {
+    EdgeCoef r{e.cval, nullptr, nullptr, D};
     if (e.cidx < 0) {
-        double cv = e.cval;
         if (D != 0.0) {
-            cv = e.cval - D * (e.cval - (mn ? mn[k] : 0.0));
-        }
-#pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            m[i] = row[i] * cv;
+            r.c = damped(e.cval, mn ? mn[k] : 0.0, D);
         }
     }
     else {
         const size_t off = size_t(e.cidx) * G * NC + size_t(age) * NC;
-        const double* cv = es.cvec + off;
-        if (D != 0.0) {
-            const double* mv = es.cvec_min ? es.cvec_min + off : nullptr;
-#pragma unroll
-            for (int i = 0; i < NC; ++i) {
-                m[i] = row[i] * (cv[i] - D * (cv[i] - (mv ? mv[i] : 0.0)));
-            }
-        }
-        else {
-#pragma unroll
-            for (int i = 0; i < NC; ++i) {
-                m[i] = row[i] * cv[i];
-            }
-        }
+        r.vec            = es.cvec + off;
+        r.vmin           = es.cvec_min ? es.cvec_min + off : nullptr;
     }
-    m[ISY] = m[ISY] * row[SNAP_FAC];
-    if (with_nd && row[SNAP_ND] != 1.0) {
-        m[ISY] *= row[SNAP_ND];
-        m[INS] *= row[SNAP_ND];
+    return r;
+}
+
+__device__ __forceinline__ double coef_of(const EdgeCoef& e, int i)
+{
+    if (!e.vec) {
+        return e.c;
+    }
+    return e.D != 0.0 ? damped(e.vec[i], e.vmin ? e.vmin[i] : 0.0, e.D) : e.vec[i];
+}
+
+// rates of one lane's Euler step of returning travelers (calculate_mobility_returns,
+// metapopulation_mobility_instant.h:460-471; euler.h:54-62), one per flow with the flow's source compartment;
+// f[0] = the force of infection
+constexpr int NFLOW = 15;
+__device__ __forceinline__ constexpr int flow_src(int f)
+{
+    constexpr int src[NFLOW] = {S, E, INS, INS, INSC, INSC, ISY, ISY, ISYC, ISYC, ISEV, ISEV, ISEV, ICR, ICR};
+    return src[f];
+}
+// the flow's rate in the lane coefficients (f >= 1)
+__device__ __forceinline__ constexpr int flow_rate(int f)
+{
+    constexpr int rate[NFLOW] = {-1,          LC_E,      LC_INS_ISY, LC_INS_R,    LC_INS_ISY,
+                                 LC_INS_R,    LC_ISY_ISEV, LC_ISY_R, LC_ISY_ISEV, LC_ISY_R,
+                                 LC_ISEV_ICR, LC_ISEV_R, LC_ISEV_D,  LC_ICR_D,    LC_ICR_R};
+    return rate[f];
+}
+
+__device__ __forceinline__ void lane_rates(Seg& c, bool icu, size_t lane, double (&w)[NFLOW])
+{
+    static_assert(LC_ICR_R == 9 && NUM_LC % 2 == 0, "the flow rates are the first ten lane coefficients");
+    double lc[10];
+    const double2* p = reinterpret_cast<const double2*>(c.lcoef + lane * NUM_LC);
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+        const double2 v = p[q];
+        lc[2 * q]       = v.x;
+        lc[2 * q + 1]   = v.y;
+    }
+    w[0] = c.kap[lane];
+#pragma unroll
+    for (int f = 1; f < NFLOW; ++f) {
+        w[f] = lc[flow_rate(f)];
+    }
+    if (icu) {
+        const double2 k = c.kicu[lane];
+        w[10]           = k.x;
+        w[12]           = k.y;
     }
 }
 
-// one explicit Euler step of the travelers with the destination's return coefficients
-// (calculate_mobility_returns, metapopulation_mobility_instant.h:460-471; euler.h:54-62)
-__device__ __forceinline__ void return_euler(const double* rc, double h, double (&m)[NC])
+// change of the travelers m over one Euler step h with rates w; `dm` in the Flows order of get_derivatives
+__device__ __forceinline__ void euler_change(const double (&m)[NC], const double (&w)[NFLOW], double h,
+                                             double (&dm)[NC])
 {
-    double dy[NC];
-    flows_to_dydt(m, rc[RC_KAPPA], rc[RC_E], rc[RC_INS_ISY], rc[RC_INS_R], rc[RC_ISY_ISEV], rc[RC_ISY_R],
-                  rc[RC_ISEV_ICR], rc[RC_ISEV_R], rc[RC_ISEV_D], rc[RC_ICR_D], rc[RC_ICR_R], dy);
+#pragma clang fp contract(off)
+    double f[NFLOW];
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        m[i] = m[i] + h * dy[i];
+    for (int k = 0; k < NFLOW; ++k) {
+        f[k] = w[k] * m[flow_src(k)];
     }
+    dm[S]    = h * (-f[0]);
+    dm[E]    = h * (f[0] - f[1]);
+    dm[INS]  = h * ((f[1] - f[2]) - f[3]);
+    dm[INSC] = h * (-f[4] - f[5]);
+    dm[ISY]  = h * ((f[2] - f[6]) - f[7]);
+    dm[ISYC] = h * ((f[4] - f[8]) - f[9]);
+    dm[ISEV] = h * ((((f[6] + f[8]) - f[10]) - f[11]) - f[12]);
+    dm[ICR]  = h * ((f[10] - f[13]) - f[14]);
+    dm[R]    = h * (((((f[3] + f[5]) + f[7]) + f[9]) + f[11]) + f[14]);
+    dm[D]    = h * (f[12] + f[13]);
 }
 
 template <int G>
@@ -1188,10 +1324,14 @@ __device__ __forceinline__ bool fixup_negative(const double (&y)[NC], double (&m
     return neg;
 }
 
-// Departures at t_dep = c_t1 (metapopulation_mobility_instant.h:605-621): every edge (s, d) adds its
-// traveler vector to d and subtracts it from s, edges in the global (start, end) order. Node v sees its
-// edges as in[s < v], out[all], in[s > v]; the lane keeps its age group's compartments in registers and
-// walks that sequence (a deterministic segmented sum in the reference's order, no atomics).
+// Arrivals at c_t1 (metapopulation_mobility_instant.h:605-621): every edge (s, d) adds its source's departure
+// row times its coefficient to d. The lane sums its age group over the node's in-edges, in the reference's
+// order; the sum is kept for the returns (return_body).
+//
+// Bound by the gathered rows: 80 B per lane and edge, 4.9 GB per launch for 512 runs of a 400-node, 20k-edge
+// graph with 6 groups. The rows lie in planes of compartment pairs: a wavefront that holds one graph node of
+// several runs reads one contiguous kilobyte per pair, where rows of 96 B touched every line of the rows five
+// times. Measured there: 300 us (16 TB/s from the L2 caches) against 470 us for the walk over rows and out-edges.
 template <int G>
 __device__ __forceinline__ void depart_body(const LaunchDev& ld, InstDev* __restrict__ inst)
 {
@@ -1199,76 +1339,355 @@ __device__ __forceinline__ void depart_body(const LaunchDev& ld, InstDev* __rest
         return; // nobody departs in this cycle
     }
     int node, age, base;
-    const SegDev* cp = lane_map<G>(ld, node, age, base);
+    Seg* cp = lane_map<G>(ld, node, age, base);
     if (!cp) {
         return;
     }
-    const SegDev& c = *cp;
+    Seg& c = *cp;
     InstDev& I      = inst[c.nodep[node].inst];
     if (!I.c_active || I.c_action != 1) {
         return;
     }
-    const EdgeStructDev& es = c.estructs[I.estruct];
+    Est& es = edge_struct(c, I.estruct);
     const int v             = c.nodep[node].local;
     const int in_b = es.in_ptr[v], in_e = es.in_ptr[v + 1];
-    const int in_s          = in_b + es.split[v];
-    const int out_b = es.out_ptr[v], out_e = es.out_ptr[v + 1];
-    const EdgeEnt* ine      = es.in_ent;
-    const EdgeEnt* oute     = es.out_ent;
-    const size_t lane_off   = size_t(node) * G + age;
-    const size_t src_base   = size_t(I.node_base) * G + age;   // lane of local node 0
-    const size_t src_step   = size_t(I.node_stride) * G;       // lanes between local nodes
-    double* yp              = c.y + lane_off * NC;
+    const size_t lane     = size_t(node) * G + age;
+    const size_t src_base = size_t(I.node_base) * G + age;   // lane of local node 0
+    const size_t src_step = size_t(I.node_stride) * G;       // lanes between local nodes
+    const size_t np       = size_t(c.num_nodes) * G;         // lanes of a plane
+    const double2* dep    = c.dep;
+    double M[NC] = {};
+    if (es.out_sum) {
+        const int32_t* src = es.in_src;
+        const double* cf   = es.in_c;
+        const double* mn   = es.in_min;
+        constexpr int U    = 4; // rows in flight per lane
+        int k              = in_b;
+        auto rows          = [&](auto n) {
+            double2 r[decltype(n)::value][NC / 2];
+            double w[decltype(n)::value];
+#pragma unroll
+            for (int u = 0; u < decltype(n)::value; ++u) {
+                const size_t sl = src_base + size_t(src[k + u]) * src_step;
+                w[u]            = cf[k + u];
+                if (c.out_d) {
+                    const double D = c.out_d[sl];
+                    if (D != 0.0) {
+                        w[u] = damped(w[u], mn ? mn[k + u] : 0.0, D);
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < NC / 2; ++q) {
+                    r[u][q] = dep[size_t(q) * np + sl];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < decltype(n)::value; ++u) {
+#pragma unroll
+                for (int q = 0; q < NC / 2; ++q) {
+                    M[2 * q]     = fma(w[u], r[u][q].x, M[2 * q]);
+                    M[2 * q + 1] = fma(w[u], r[u][q].y, M[2 * q + 1]);
+                }
+            }
+        };
+        for (; k + U <= in_e; k += U) {
+            rows(std::integral_constant<int, U>{});
+        }
+        for (; k < in_e; ++k) {
+            rows(std::integral_constant<int, 1>{});
+        }
+    }
+    else {
+        for (int k = in_b; k < in_e; ++k) {
+            const EdgeEnt e   = es.in_ent[k];
+            const size_t sl   = src_base + size_t(e.nbr) * src_step;
+            const EdgeCoef ec = edge_coef(es, e, es.in_min, k, c.out_d ? c.out_d[sl] : 0.0, G, age);
+            double r[NC];
+            load_planes(dep, np, sl, r);
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                M[i] = fma(coef_of(ec, i), r[i], M[i]);
+            }
+        }
+    }
+    store_planes(c.arr, np, lane, M);
+    double* yp = c.y + lane * NC;
     double y[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
-        y[i] = yp[i];
+        y[i]  = yp[i] + M[i];
+        yp[i] = y[i];
     }
-    auto in_range = [&](int k, int end) {
-        for (; k < end; ++k) {
-            const EdgeEnt e = ine[k];
-            double r[SNAP_STRIDE];
-            const size_t sl = src_base + size_t(e.nbr) * src_step;
-            load_row(c.snap, sl, r);
-            double m[NC];
-            traveler_vector(es, e, es.in_min, k, c.out_d ? c.out_d[sl] : 0.0, r, G, age, true, m);
+    if (I.c_out_day >= 0) {
+        write_phase_end_day<G>(c, I, lane, v, age, y);
+    }
+}
+
+// Constant part of the returns of a node as a source (once per batch): per flow, the sum over its out-edges of
+// the coefficient times the destination's rate, in planes; wmin: the same with the minimum coefficients.
+template <int G>
+__device__ __forceinline__ void weights_body(const LaunchDev& ld, InstDev* __restrict__ inst, int inst_offset)
+{
+    int node, age, base;
+    Seg* cp = lane_map<G>(ld, node, age, base);
+    if (!cp) {
+        return;
+    }
+    Seg& c  = *cp;
+    const InstDev& I = inst[c.nodep[node].inst - inst_offset];
+    if (I.estruct < 0) {
+        return;
+    }
+    Est& es = edge_struct(c, I.estruct);
+    const int v             = c.nodep[node].local;
+    const size_t lane       = size_t(node) * G + age;
+    const size_t src_base   = size_t(I.node_base) * G + age;
+    const size_t src_step   = size_t(I.node_stride) * G;
+    const size_t np         = size_t(c.num_nodes) * G;
+    double w[NFLOW] = {}, wm[NFLOW] = {};
+    for (int k = es.out_ptr[v]; k < es.out_ptr[v + 1]; ++k) {
+        const EdgeEnt e  = es.out_ent[k];
+        const double* lc = c.lcoef + (src_base + size_t(e.nbr) * src_step) * NUM_LC;
+        const size_t off = size_t(e.cidx < 0 ? 0 : e.cidx) * G * NC + size_t(age) * NC;
 #pragma unroll
-            for (int i = 0; i < NC; ++i) {
-                y[i] += m[i];
+        for (int f = 1; f < NFLOW; ++f) {
+            const int i       = flow_src(f);
+            const double rate = lc[flow_rate(f)];
+            w[f]              = fma(e.cidx < 0 ? e.cval : es.cvec[off + i], rate, w[f]);
+            if (c.wmin) {
+                const double mn = e.cidx < 0 ? (es.out_min ? es.out_min[k] : 0.0)
+                                             : (es.cvec_min ? es.cvec_min[off + i] : 0.0);
+                wm[f]           = fma(mn, rate, wm[f]);
             }
+        }
+    }
+    auto put = [&](double2* p, const double (&x)[NFLOW]) {
+        if (c.wplanes == 7) {
+#pragma unroll
+            for (int q = 0; q < 7; ++q) {
+                p[size_t(q) * np + lane] = double2{x[1 + 2 * q], x[2 + 2 * q]};
+            }
+        }
+        else { // one coefficient per edge: the confirmed flows have the weights of the unconfirmed ones
+            p[0 * np + lane] = double2{x[1], x[2]};
+            p[1 * np + lane] = double2{x[3], x[6]};
+            p[2 * np + lane] = double2{x[7], x[10]};
+            p[3 * np + lane] = double2{x[11], x[12]};
+            p[4 * np + lane] = double2{x[13], x[14]};
         }
     };
-    in_range(in_b, in_s);
-    if (out_b < out_e) {
-        double sv[SNAP_STRIDE];
-        load_row(c.snap, lane_off, sv);
-        const double nd_v = sv[SNAP_ND];
-        const double D_v  = c.out_d ? c.out_d[lane_off] : 0.0;
-        for (int k = out_b; k < out_e; ++k) {
-            double m[NC];
-            traveler_vector(es, oute[k], es.out_min, k, D_v, sv, G, age, false, m);
-            if (nd_v != 1.0) {
-                // test_commuters on the source: detected commuters stay home as confirmed cases
-                y[INS] -= m[INS] * (1 - nd_v);
-                y[INSC] += m[INS] * (1 - nd_v);
-                y[ISY] -= m[ISY] * (1 - nd_v);
-                y[ISYC] += m[ISY] * (1 - nd_v);
-                m[ISY] *= nd_v;
-                m[INS] *= nd_v;
-            }
+    put(c.wst, w);
+    if (c.wmin) {
+        put(c.wmin, wm);
+    }
+}
+
+__device__ __forceinline__ void load_weights(Seg& c, const double2* p, size_t np, size_t lane,
+                                             double (&x)[NFLOW])
+{
+    if (c.wplanes == 7) {
 #pragma unroll
-            for (int i = 0; i < NC; ++i) {
-                y[i] -= m[i];
+        for (int q = 0; q < 7; ++q) {
+            const double2 t = p[size_t(q) * np + lane];
+            x[1 + 2 * q]    = t.x;
+            x[2 + 2 * q]    = t.y;
+        }
+        return;
+    }
+    const double2 a = p[0 * np + lane], b = p[1 * np + lane], d = p[2 * np + lane], e = p[3 * np + lane],
+                  g = p[4 * np + lane];
+    x[1]  = a.x;
+    x[2]  = x[4] = a.y;
+    x[3]  = x[5] = b.x;
+    x[6]  = x[8] = b.y;
+    x[7]  = x[9] = d.x;
+    x[10] = d.y;
+    x[11] = e.x;
+    x[12] = e.y;
+    x[13] = g.x;
+    x[14] = g.y;
+}
+
+// All travelers that come home to a lane's node, each after its destination's Euler step: the lane's departure
+// row stepped with the sums over the out-edges of coefficient times rate. k0: the sum of the forces of infection;
+// k10, k12: those of the ICU-adjusted rates (used with ICU limits, else the kept constants).
+template <int G>
+__device__ __forceinline__ void homecoming(Seg& c, const InstDev& I, Est& es, int v,
+                                           size_t lane, int age, double D_v, double k0, double k10, double k12,
+                                           double (&home)[NC])
+{
+#pragma clang fp contract(off)
+    const size_t np = size_t(c.num_nodes) * G;
+    double m[NC], dm[NC], w[NFLOW];
+    load_planes(c.dep, np, lane, m);
+    load_weights(c, c.wst, np, lane, w);
+    if (D_v != 0.0) {
+        double wm[NFLOW];
+        load_weights(c, c.wmin, np, lane, wm);
+#pragma unroll
+        for (int f = 1; f < NFLOW; ++f) {
+            w[f] = damped(w[f], wm[f], D_v);
+        }
+    }
+    w[0] = k0;
+    if (I.icu) {
+        w[10] = k10;
+        w[12] = k12;
+    }
+    euler_change(m, w, I.c_step, dm);
+    if (es.out_sum) {
+        double sum = es.out_sum[v];
+        if (D_v != 0.0) {
+            sum = damped(sum, es.out_min_sum ? es.out_min_sum[v] : 0.0, D_v);
+        }
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            home[i] = sum * m[i] + dm[i];
+        }
+    }
+    else {
+        const size_t off = (size_t(v) * G + age) * NC;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            double sum = es.out_vsum[off + i];
+            if (D_v != 0.0) {
+                sum = damped(sum, es.out_vmin_sum ? es.out_vmin_sum[off + i] : 0.0, D_v);
+            }
+            home[i] = sum * m[i] + dm[i];
+        }
+    }
+}
+
+// travelers of one edge after the Euler step at their destination: the source's departure row m in, the
+// returning travelers out
+__device__ __forceinline__ void edge_return(const EdgeCoef& ec, const double (&rates)[NFLOW], double h, double (&m)[NC])
+{
+#pragma clang fp contract(off)
+    double dm[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        m[i] = m[i] * coef_of(ec, i);
+    }
+    euler_change(m, rates, h, dm);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        m[i] = m[i] + dm[i];
+    }
+}
+
+// Returns at c_t1 of the travelers that left at c_tdep (metapopulation_mobility_instant.h:568-603) in closed
+// form. The Euler step of the travelers is linear in them and, per flow, in the destination's rate. So all
+// travelers that a node sends home are one Euler step of its arrivals (the sum that the departure phase kept)
+// with its own rates, and all that come home to it are its departure row stepped with the sums over its
+// out-edges of coefficient times rate: those of the constant rates are kept per lane (weights_body), the
+// force of infection (and, with ICU limits, two more) is summed here, 8 B per lane and edge instead of the
+// 2 x 96 B per lane and edge that a walk over all edges gathers. Measured (512 runs, 400 nodes, 20k edges, 6
+// groups): 350 us per launch against 1315 us for the walk.
+//
+// The fix-up acts where a compartment of a destination falls below zero while its in-edges are taken off one
+// by one. With nonnegative returning travelers every partial difference is at least the full one, ypre - arrivals
+// (homecomings only add), so a node whose full difference is nonnegative has none. The others are marked and
+// walk their edges one by one (walk_node, settle_body). The step's factor of a compartment, 1 - h * (sum of its
+// outgoing rates), keeps travelers nonnegative if it is: coefficients and constant rates are checked on the host
+// (InstDev::general), the departure rows as they are written (InstDev::fx_neg). Only S, whose rate is the force
+// of infection, may step below zero in earnest (more than 1 / h infections per day at a peak). It has no inflow,
+// so all in-edges of a node change it in one direction and its extremes are at the ends of the sequence and at
+// the homecomings: ypre, ypre - arrivals and both with the homecomings added.
+template <int G>
+__device__ __forceinline__ void return_body(const LaunchDev& ld, InstDev* __restrict__ inst)
+{
+#pragma clang fp contract(off)
+    if (ld.cyc && !ld.cyc[CYC_RETURN]) {
+        return; // nobody returns in this cycle
+    }
+    int node, age, base;
+    Seg* cp = lane_map<G>(ld, node, age, base);
+    if (!cp) {
+        return;
+    }
+    Seg& c = *cp;
+    InstDev& I      = inst[c.nodep[node].inst];
+    if (!I.c_active || I.c_action != 2 || I.general) {
+        return;
+    }
+    Est& es = edge_struct(c, I.estruct);
+    const int v             = c.nodep[node].local;
+    const size_t lane       = size_t(node) * G + age;
+    const size_t src_base   = size_t(I.node_base) * G + age;
+    const size_t src_step   = size_t(I.node_stride) * G;
+    const size_t np         = size_t(c.num_nodes) * G;
+    const double h          = I.c_step;
+    const bool icu          = I.icu != 0;
+    const double D_v        = c.out_d ? c.out_d[lane] : 0.0;
+    // sums over the out-edges: force of infection of the destinations, and their ICU-adjusted rates
+    double w[NFLOW];
+    double k0 = 0.0, k10 = 0.0, k12 = 0.0, k_min = 0.0;
+    const int out_b = es.out_ptr[v], out_e = es.out_ptr[v + 1];
+    if (es.out_sum) {
+#pragma unroll 4
+        for (int k = out_b; k < out_e; ++k) {
+            const size_t dl = src_base + size_t(es.out_dst[k]) * src_step;
+            double cf       = es.out_c[k];
+            if (D_v != 0.0) {
+                cf = damped(cf, es.out_min ? es.out_min[k] : 0.0, D_v);
+            }
+            const double kd = c.kap[dl];
+            k0              = fma(cf, kd, k0);
+            k_min           = fmin(k_min, kd);
+            if (icu) {
+                const double2 r = c.kicu[dl];
+                k10             = fma(cf, r.x, k10);
+                k12             = fma(cf, r.y, k12);
             }
         }
     }
-    in_range(in_s, in_e);
+    else {
+        for (int k = out_b; k < out_e; ++k) {
+            const EdgeEnt e   = es.out_ent[k];
+            const size_t dl   = src_base + size_t(e.nbr) * src_step;
+            const EdgeCoef ec = edge_coef(es, e, es.out_min, k, D_v, G, age);
+            const double kd   = c.kap[dl];
+            k0                = fma(coef_of(ec, S), kd, k0);
+            k_min             = fmin(k_min, kd);
+            if (icu) {
+                const double2 r = c.kicu[dl];
+                k10             = fma(coef_of(ec, ISEV), r.x, k10);
+                k12             = fma(coef_of(ec, ISEV), r.y, k12);
+            }
+        }
+    }
+    // travelers sent home
+    double y[NC], m[NC], dm[NC];
+    load_planes(c.ypre, np, lane, y);
+    load_planes(c.arr, np, lane, m);
+    lane_rates(c, icu, lane, w);
+    euler_change(m, w, h, dm);
+    bool mark        = I.fx_neg != 0 || !(w[0] >= 0.0) || !(k_min >= 0.0);
+    const double y_s = y[S];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        y[i] = y[i] - (m[i] + dm[i]);
+        mark = mark || !(y[i] >= 0.0);
+    }
+    // travelers coming home
+    double home[NC];
+    homecoming<G>(c, I, es, v, lane, age, D_v, k0, k10, k12, home);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        y[i] = y[i] + home[i];
+    }
+    mark = mark || !(y_s >= 0.0) || !(y_s + home[S] >= 0.0) || !(y[S] >= 0.0);
+    if (group_any<G>(mark, base) && age == 0 && out_e - out_b + (es.in_ptr[v + 1] - es.in_ptr[v]) > 0) {
+        c.fx_dirty[node] = I.fx_epoch; // walks its edges in pass 1
+        I.fx_changed     = 1;          // every writer stores 1
+    }
+    double* yp = c.y + lane * NC;
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
         yp[i] = y[i];
     }
     if (I.c_out_day >= 0) {
-        write_phase_end_day<G>(c, I, lane_off, v, age, y);
+        write_phase_end_day<G>(c, I, lane, v, age, y);
     }
 }
 
@@ -1285,9 +1704,9 @@ __device__ __forceinline__ int32_t record_slot(const FxRec* r, int32_t lo, int32
     return vb ? b.slot : -1;
 }
 
-// Return walk of one node (returns at c_t1 of the travelers that left at c_tdep,
-// metapopulation_mobility_instant.h:568-603) from the pre-return state, visiting the node's edges in the
-// reference's global (start, end) order.
+// Return walk of one node by one wavefront (returns at c_t1 of the travelers that left at c_tdep,
+// metapopulation_mobility_instant.h:568-603) from the pre-return state, the node's edges in the reference's
+// global (start, end) order: in-edges of lower sources, homecomings, the other in-edges.
 //
 // The fix-up of edge (s, d) depends on d's state at that point of the sequence, which includes d's
 // earlier out-edges (d, x) with their own fix-ups decided at x. Pass p applies the fix-ups of the node's
@@ -1296,218 +1715,263 @@ __device__ __forceinline__ int32_t record_slot(const FxRec* r, int32_t lo, int32
 // values after at most (longest dependency chain + 1) passes; a pass in which no record changes
 // reproduces the sequential result exactly. A node whose out-edge records did not change in pass p-1
 // would repeat its walk of pass p-1 unchanged, so pass p only re-walks the nodes marked dirty then.
-template <int G, bool FIRST>
-__device__ __forceinline__ void return_body(const LaunchDev& ld, InstDev* __restrict__ inst, int launch_pass)
+//
+// A walk is a chain over the in-edges, and only the subtractions and the sign checks depend on the previous
+// edge: the lanes load and step the travelers of 64 / G in-edges at a time (all lanes busy, one gather latency
+// per 64 / G edges), then every group of lanes runs the chain over them from LDS (buf, 64 x 10 doubles per
+// wavefront). With one group of lanes per node and an edge at a time, a pass over nodes of 50 in- and 50
+// out-edges took 120 us and more.
+//
+// Returns (in every lane) WALK_CHANGED if some record changed and WALK_FULL if the record pool is full.
+constexpr int WALK_CHANGED = 1;
+constexpr int WALK_FULL    = 2;
+
+template <int G>
+__device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass, double* buf)
 {
-    if (ld.cyc && !ld.cyc[FIRST ? CYC_RETURN : CYC_PASS0 + launch_pass]) {
-        return; // nobody returns in this cycle, or no instance needs this fix-up pass
-    }
-    int node, age, base;
-    const SegDev* cp = lane_map<G>(ld, node, age, base);
-    if (!cp) {
-        return;
-    }
-    const SegDev& c = *cp;
-    InstDev& I      = inst[c.nodep[node].inst];
-    if (!I.c_active || I.c_action != 2) {
-        return;
-    }
-    const int pass = FIRST ? 0 : I.fx_pass;
-    if (FIRST ? (I.fx_state != 0) : (I.fx_state != 1 || pass == 0)) {
-        return;
-    }
+    constexpr int NPW = WAVE / G;
+    const int lane    = int(threadIdx.x) % WAVE;
+    const int grp     = lane / G;
+    const int age     = lane - grp * G;
+    const bool act    = grp < NPW;
     const int32_t tag = I.fx_epoch + pass;
     // marks of pass p-1 are in plane (p-1)&1; this pass writes plane p&1
-    int32_t* dirty_out = c.fx_dirty + size_t(pass & 1) * c.num_nodes;
-    if (!FIRST && c.fx_dirty[size_t((pass - 1) & 1) * c.num_nodes + node] != tag - 1) {
-        return;
-    }
-    const EdgeStructDev& es = c.estructs[I.estruct];
+    int32_t* dirty_out      = c.fx_dirty + size_t(pass & 1) * c.num_nodes;
+    Est& es = edge_struct(c, I.estruct);
     const int v             = c.nodep[node].local;
     const int in_b = es.in_ptr[v], in_e = es.in_ptr[v + 1];
-    const int in_s          = in_b + es.split[v];
+    const int in_s  = in_b + es.split[v];
     const int out_b = es.out_ptr[v], out_e = es.out_ptr[v + 1];
-    const EdgeEnt* ine      = es.in_ent;
-    const EdgeEnt* oute     = es.out_ent;
-    const size_t lane_off   = size_t(node) * G + age;
-    const size_t src_base   = size_t(I.node_base) * G + age;   // lane of local node 0
-    const size_t src_step   = size_t(I.node_stride) * G;       // lanes between local nodes
-    FxRec* recs             = c.fx_rec + 2 * I.fx_base;
-    double* pool            = c.fx_pool + I.fx_pool_base;
-    const int32_t lo        = I.fx_epoch;
-    const double h          = I.c_step;
-    const double* rc_v      = c.rc + lane_off * RC_STRIDE;
-
-    double y[NC];
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        y[i] = c.ypre[lane_off * NC + i];
+    const size_t own      = size_t(node) * G + age;
+    const size_t src_base = size_t(I.node_base) * G + age;   // lane of local node 0
+    const size_t src_step = size_t(I.node_stride) * G;       // lanes between local nodes
+    const size_t np       = size_t(c.num_nodes) * G;
+    FxRec* recs           = c.fx_rec + 2 * I.fx_base;
+    double* pool          = c.fx_pool + I.fx_pool_base;
+    const int32_t lo      = I.fx_epoch;
+    const double h        = I.c_step;
+    const bool icu        = I.icu != 0;
+    const double D_v      = c.out_d ? c.out_d[own] : 0.0;
+    double rates[NFLOW], y[NC], home[NC];
+    // homecomings: sums over the out-edges, in 64 / G parts
+    double k0 = 0.0, k10 = 0.0, k12 = 0.0;
+    if (act) {
+        for (int k = out_b + grp; k < out_e; k += NPW) {
+            const EdgeEnt e   = es.out_ent[k];
+            const size_t dl   = src_base + size_t(e.nbr) * src_step;
+            const EdgeCoef ec = edge_coef(es, e, es.out_min, k, D_v, G, age);
+            k0                = fma(coef_of(ec, S), c.kap[dl], k0);
+            if (icu) {
+                const double2 r = c.kicu[dl];
+                k10             = fma(coef_of(ec, ISEV), r.x, k10);
+                k12             = fma(coef_of(ec, ISEV), r.y, k12);
+            }
+        }
     }
-    bool changed = false;
-    auto in_edge = [&](int k) {
-        const EdgeEnt e = ine[k];
-        double row[SNAP_STRIDE];
-        const size_t sl = src_base + size_t(e.nbr) * src_step;
-        load_row(c.snap, sl, row);
-        double m[NC];
-        traveler_vector(es, e, es.in_min, k, c.out_d ? c.out_d[sl] : 0.0, row, G, age, true, m);
-        return_euler(rc_v, h, m);
-        const bool any = group_any<G>(fixup_negative(y, m), base);
-        const int32_t ps = FIRST ? -1 : record_slot(recs + 2 * k, lo, tag - 1);
-        bool diff        = (ps >= 0) != any;
-        if (any && !diff) {
-#pragma unroll
-            for (int i = 0; i < NC; ++i) {
-                diff = diff || (pool[(size_t(ps) * G + age) * NC + i] != m[i]);
-            }
+    auto total = [&](double x) {
+        buf[lane] = x;
+        wave_sync();
+        double t = 0.0;
+        for (int j = 0; j < NPW; ++j) {
+            t += buf[j * G + age];
         }
-        diff = group_any<G>(diff, base);
-        if (diff) {
-            int32_t slot = -1;
-            if (any) {
-                if (age == 0) {
-                    slot = atomicAdd(&I.fx_count, 1);
-                }
-                slot = __shfl(slot, base);
-                if (slot < FX_SLOTS) {
-#pragma unroll
-                    for (int i = 0; i < NC; ++i) {
-                        pool[(size_t(slot) * G + age) * NC + i] = m[i];
-                    }
-                }
-                else {
-                    slot = -1;
-                    if (age == 0) {
-                        I.fx_state = 2; // record pool full: resolve this phase with the sequential replay
-                    }
-                }
-            }
-            if (age == 0) {
-                FxRec* r        = recs + 2 * k;
-                const int older = (r[0].tag <= r[1].tag) ? 0 : 1;
-                r[older]        = FxRec{tag, slot};
-                dirty_out[seg_node(I, e.nbr)] = tag; // the source re-walks in the next pass
-            }
-            changed = true;
-        }
-#pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            y[i] -= m[i];
-        }
+        wave_sync();
+        return t;
     };
-    for (int k = in_b; k < in_s; ++k) {
-        in_edge(k);
+    k0 = total(k0);
+    if (icu) {
+        k10 = total(k10);
+        k12 = total(k12);
     }
-    if (out_b < out_e) {
-        double sv[SNAP_STRIDE];
-        load_row(c.snap, lane_off, sv);
-        const double D_v = c.out_d ? c.out_d[lane_off] : 0.0;
-        for (int k = out_b; k < out_e; ++k) {
-            const EdgeEnt e = oute[k];
-            double m[NC];
-            const int32_t ps = FIRST ? -1 : record_slot(recs + 2 * e.peer, lo, tag - 1);
-            if (ps >= 0) {
+    homecoming<G>(c, I, es, v, own, age, D_v, k0, k10, k12, home);
+    if (pass > 0) {
+        // out-edges whose travelers a destination changed: their record instead of the unfixed vector
+        for (int kb = out_b; kb < out_e; kb += WAVE) {
+            const int k      = kb + lane;
+            const int32_t ps = k < out_e ? record_slot(recs + 2 * es.out_ent[k].peer, lo, tag - 1) : -1;
+            for (unsigned long long left = __ballot(ps >= 0); left; left &= left - 1) {
+                const int b       = __ffsll(left) - 1;
+                const int slot    = __shfl(ps, b);
+                const EdgeEnt e   = es.out_ent[kb + b];
+                const EdgeCoef ec = edge_coef(es, e, es.out_min, kb + b, D_v, G, age);
+                double m[NC];
+                load_planes(c.dep, np, own, m);
+                lane_rates(c, icu, src_base + size_t(e.nbr) * src_step, rates);
+                edge_return(ec, rates, h, m);
 #pragma unroll
                 for (int i = 0; i < NC; ++i) {
-                    m[i] = pool[(size_t(ps) * G + age) * NC + i];
+                    home[i] += pool[(size_t(slot) * G + age) * NC + i] - m[i];
                 }
-            }
-            else {
-                traveler_vector(es, e, es.out_min, k, D_v, sv, G, age, true, m);
-                return_euler(c.rc + (src_base + size_t(e.nbr) * src_step) * RC_STRIDE, h, m);
-            }
-#pragma unroll
-            for (int i = 0; i < NC; ++i) {
-                y[i] += m[i];
             }
         }
     }
-    for (int k = in_s; k < in_e; ++k) {
-        in_edge(k);
-    }
-    if (changed && age == 0) {
-        I.fx_changed = 1; // every writer stores 1
-    }
-    double* yp = c.y + lane_off * NC;
+    lane_rates(c, icu, own, rates);
+    load_planes(c.ypre, np, own, y);
+    int result    = 0;
+    auto in_edges = [&](int first, int last) {
+        for (int kb = first; kb < last; kb += NPW) {
+            const int k = kb + grp;
+            int32_t ps  = -1;
+            if (act && k < last) {
+                const EdgeEnt e   = es.in_ent[k];
+                const size_t sl   = src_base + size_t(e.nbr) * src_step;
+                const EdgeCoef ec = edge_coef(es, e, es.in_min, k, c.out_d ? c.out_d[sl] : 0.0, G, age);
+                double m[NC];
+                load_planes(c.dep, np, sl, m);
+                edge_return(ec, rates, h, m);
+#pragma unroll
+                for (int i = 0; i < NC; ++i) {
+                    buf[i * WAVE + lane] = m[i];
+                }
+                if (pass > 0) {
+                    ps = record_slot(recs + 2 * k, lo, tag - 1);
+                }
+            }
+            wave_sync();
+            const int n = min(NPW, last - kb);
+            for (int j = 0; j < n; ++j) {
+                double m[NC];
+#pragma unroll
+                for (int i = 0; i < NC; ++i) {
+                    m[i] = buf[i * WAVE + j * G + age];
+                }
+                const bool any    = __any(act && fixup_negative(y, m));
+                const int32_t psj = __shfl(ps, j * G);
+                bool diff         = (psj >= 0) != any;
+                if (any && !diff) {
+                    bool d = false;
+#pragma unroll
+                    for (int i = 0; i < NC; ++i) {
+                        d = d || (pool[(size_t(psj) * G + age) * NC + i] != m[i]);
+                    }
+                    diff = __any(act && d);
+                }
+                if (diff) {
+                    int32_t slot = -1;
+                    if (any) {
+                        if (lane == 0) {
+                            slot = atomicAdd(&I.fx_count, 1);
+                        }
+                        slot = __shfl(slot, 0);
+                        if (slot < FX_SLOTS) {
+                            if (grp == 0) {
+#pragma unroll
+                                for (int i = 0; i < NC; ++i) {
+                                    pool[(size_t(slot) * G + age) * NC + i] = m[i];
+                                }
+                            }
+                        }
+                        else {
+                            slot = -1;
+                            result |= WALK_FULL; // the sequential replay resolves this phase
+                        }
+                    }
+                    if (lane == 0) {
+                        FxRec* r        = recs + 2 * (kb + j);
+                        const int older = (r[0].tag <= r[1].tag) ? 0 : 1;
+                        r[older]        = FxRec{tag, slot};
+                        dirty_out[seg_node(I, es.in_ent[kb + j].nbr)] = tag; // the source re-walks in the next pass
+                    }
+                    result |= WALK_CHANGED;
+                }
+#pragma unroll
+                for (int i = 0; i < NC; ++i) {
+                    y[i] -= m[i];
+                }
+            }
+            wave_sync();
+        }
+    };
+    in_edges(in_b, in_s);
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
-        yp[i] = y[i];
+        y[i] += home[i];
     }
-    if (I.c_out_day >= 0) {
-        write_phase_end_day<G>(c, I, lane_off, v, age, y);
+    in_edges(in_s, in_e);
+    if (grp == 0) {
+        double* yp = c.y + own * NC;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            yp[i] = y[i];
+        }
+        if (I.c_out_day >= 0) {
+            write_phase_end_day<G>(c, I, own, v, age, y);
+        }
     }
+    return result;
 }
 
-// After a return pass: settle the instance, schedule another pass, or hand it to the sequential replay.
-static __global__ void fixup_check(LaunchDev ld, InstDev* inst)
+// pass 0 of the instances whose returns walk their edges (InstDev::general): every node, one wavefront each
+template <int G>
+__device__ __forceinline__ void walk_body(const LaunchDev& ld, InstDev* __restrict__ inst, double* buf)
 {
-    const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= ld.num_inst) {
+    if (ld.cyc && !ld.cyc[CYC_RETURN]) {
         return;
     }
-    InstDev& I = inst[ld.inst_ids[i]];
-    if (!I.c_active || I.c_action != 2 || I.fx_state >= 2) {
+    const int lb = xcd_block();
+    if (lb >= ld.num_blocks || ld.block_seg[lb] < 0) {
         return;
     }
-    if (!I.fx_changed) {
-        I.fx_state = 3;
-        return;
-    }
-    if (I.fx_sequential || I.fx_pass + 1 >= FX_MAX_PASSES) {
-        I.fx_state = 2;
-        return;
-    }
-    I.fx_state   = 1;
-    I.fx_pass    = I.fx_pass + 1;
-    I.fx_changed = 0;
-    I.fx_passes += 1;
-    if (ld.cyc) {
-        ld.cyc[CYC_PASS0 + I.fx_pass] = 1; // fx_pass < FX_MAX_PASSES here
+    const int seg   = ld.block_seg[lb];
+    Seg& c = *segment(ld, seg);
+    constexpr int NPW = WAVE / G;
+    const int wave    = (lb - ld.block_first[seg]) * (BLOCK / WAVE) + int(threadIdx.x) / WAVE;
+    for (int node = wave * NPW; node < min(c.num_nodes, (wave + 1) * NPW); ++node) {
+        InstDev& I = inst[c.nodep[node].inst];
+        if (I.c_active && I.c_action == 2 && I.general) {
+            const int r = walk_node<G>(c, I, node, 0, buf + (threadIdx.x / WAVE) * (WAVE * NC));
+            if (r != 0 && threadIdx.x % WAVE == 0) {
+                I.fx_changed = 1; // every writer stores the same value
+                if (r & WALK_FULL) {
+                    I.fx_state = 2;
+                }
+            }
+        }
     }
 }
 
-// ------------------------------------------------------------------------------- exact replay
+// ------------------------------------------------------------------------------- settling the fix-ups
 // Sequential return pass of one instance in the reference's edge order with the negative-value fix-up
 // (metapopulation_mobility_instant.h:568-603). Fallback for the rare return phases whose fix-up records
 // did not settle within FX_MAX_PASSES passes or overflowed the record pool; lanes = age groups.
 template <int G>
-__device__ __forceinline__ void replay_body(const LaunchDev& ld, InstDev* __restrict__ inst)
+__device__ __forceinline__ void replay(Seg& c, InstDev& I)
 {
-    const int ii = ld.inst_ids[blockIdx.x];
-    InstDev& I   = inst[ii];
-    if (!I.c_active || I.c_action != 2 || I.fx_state != 2) {
-        return;
-    }
-    const SegDev& c = ld.segs[I.seg];
-    const int a = int(threadIdx.x);
+    const int a     = int(threadIdx.x);
+    const size_t np = size_t(c.num_nodes) * G;
     // restore the pre-return state of every node
-    for (int v = 0; v < I.num_nodes; ++v) {
-        if (a < G) {
-            const size_t off = (seg_node(I, v) * G + a) * NC;
-            for (int i = 0; i < NC; ++i) {
-                c.y[off + i] = c.ypre[off + i];
-            }
+    for (int k = int(threadIdx.x); k < I.num_nodes * G; k += int(blockDim.x)) {
+        const size_t lane = seg_node(I, k / G) * G + size_t(k % G);
+        double y[NC];
+        load_planes(c.ypre, np, lane, y);
+        for (int i = 0; i < NC; ++i) {
+            c.y[lane * NC + i] = y[i];
         }
     }
     __syncthreads();
-    const EdgeStructDev& es = c.estructs[I.estruct];
+    Est& es = edge_struct(c, I.estruct);
     const int32_t* seq      = es.seq;
     const EdgeEnt* oute     = es.out_ent;
     const double h          = I.c_step;
+    const bool icu          = I.icu != 0;
     if (a < G) {
         for (int k = 0; k < es.num_edges; ++k) {
             const EdgeEnt e   = oute[seq[3 * k + 2]];
             const size_t soff = seg_node(I, seq[3 * k]) * G + a;
             const size_t doff = seg_node(I, seq[3 * k + 1]) * G + a;
-            double row[SNAP_STRIDE];
-            load_row(c.snap, soff, row);
-            double m[NC];
-            traveler_vector(es, e, es.out_min, seq[3 * k + 2], c.out_d ? c.out_d[soff] : 0.0, row, G, a, true, m);
-            return_euler(c.rc + doff * RC_STRIDE, h, m);
+            const EdgeCoef ec = edge_coef(es, e, es.out_min, seq[3 * k + 2], c.out_d ? c.out_d[soff] : 0.0, G, a);
+            double m[NC], dm[NC], w[NFLOW];
+            load_planes(c.dep, np, soff, m);
+            lane_rates(c, icu, doff, w);
+            for (int i = 0; i < NC; ++i) {
+                m[i] = m[i] * coef_of(ec, i);
+            }
+            euler_change(m, w, h, dm);
             double* yd = c.y + doff * NC;
             double* ys = c.y + soff * NC;
             double yl[NC];
             for (int i = 0; i < NC; ++i) {
+                m[i]  = m[i] + dm[i];
                 yl[i] = yd[i];
             }
             fixup_negative(yl, m);
@@ -1522,7 +1986,6 @@ __device__ __forceinline__ void replay_body(const LaunchDev& ld, InstDev* __rest
     __syncthreads();
     if (a == 0) {
         I.replays += 1;
-        I.fx_state = 3;
     }
     if (I.c_out_day >= 0 && a < G) {
         for (int v = 0; v < I.num_nodes; ++v) {
@@ -1533,6 +1996,70 @@ __device__ __forceinline__ void replay_body(const LaunchDev& ld, InstDev* __rest
             }
             write_phase_end_day<G>(c, I, lane, v, a, yv);
         }
+    }
+}
+
+// One block per instance: the passes of walk_node over the marked nodes until no record changes. All of an
+// instance's walks run in its block, so a pass ends at a barrier instead of a kernel boundary (seven pairs of
+// launches per cycle before, most of them idle).
+template <int G>
+__device__ __forceinline__ void settle_body(const LaunchDev& ld, InstDev* __restrict__ inst, int32_t* list,
+                                            double* buf)
+{
+    constexpr int CAP = SETTLE_LIST; // marked nodes of one chunk
+    InstDev& I        = inst[ld.inst_ids[blockIdx.x]];
+    if (!I.c_active || I.c_action != 2 || !I.fx_changed) {
+        return;
+    }
+    Seg& c = *segment(ld, I.seg);
+    const int wave  = int(threadIdx.x) / WAVE;
+    // list[CAP]: number of marked nodes, list[CAP + 1]: results of the pass's walks
+    bool sequential = I.fx_sequential != 0 || I.fx_state == 2;
+    int pass        = 1;
+    for (; !sequential; ++pass) {
+        if (threadIdx.x == 0) {
+            list[CAP + 1] = 0;
+        }
+        const int32_t* marks = c.fx_dirty + size_t((pass - 1) & 1) * c.num_nodes;
+        for (int first = 0; first < I.num_nodes; first += CAP) {
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                list[CAP] = 0;
+            }
+            __syncthreads();
+            const int last = min(I.num_nodes, first + CAP);
+            for (int v = first + int(threadIdx.x); v < last; v += int(blockDim.x)) {
+                const int node = int(seg_node(I, v));
+                if (marks[node] == I.fx_epoch + pass - 1) {
+                    list[atomicAdd(&list[CAP], 1)] = node;
+                }
+            }
+            __syncthreads();
+            const int n = list[CAP];
+            for (int k = wave; k < n; k += int(blockDim.x) / WAVE) {
+                const int r = walk_node<G>(c, I, list[k], pass, buf + wave * (WAVE * NC));
+                if (r != 0 && threadIdx.x % WAVE == 0) {
+                    atomicOr(&list[CAP + 1], r);
+                }
+            }
+        }
+        // marks, records and record vectors of this pass are read by the other wavefronts in the next one
+        __threadfence();
+        __syncthreads();
+        __threadfence();
+        const int r = list[CAP + 1];
+        __syncthreads(); // everyone has read it before the next pass clears it
+        if (!(r & WALK_CHANGED)) {
+            break;
+        }
+        sequential = (r & WALK_FULL) || pass + 1 >= FX_MAX_PASSES;
+    }
+    if (threadIdx.x == 0) {
+        I.fx_passes += pass;
+    }
+    if (sequential) {
+        __syncthreads();
+        replay<G>(c, I);
     }
 }
 
@@ -1578,48 +2105,64 @@ __global__ void __launch_bounds__(BLOCK) node_phase_mixed(LaunchDev ld, InstDev*
 }
 
 template <int G>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) depart_phase(LaunchDev ld,
-                                                                                       InstDev* __restrict__ inst)
+__global__ void __launch_bounds__(BLOCK) depart_phase(LaunchDev ld, InstDev* __restrict__ inst)
 {
     depart_body<G>(ld, inst);
 }
 
-#if MGO_SHARD == 13
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) depart_phase_mixed(LaunchDev ld,
-                                                                                             InstDev* __restrict__ inst)
+template <int G>
+__global__ void __launch_bounds__(BLOCK) weights_phase(LaunchDev ld, InstDev* __restrict__ inst, int inst_offset)
 {
-    MGO_DISPATCH_G(block_groups(ld), (depart_body<GG>(ld, inst)))
-}
-#endif
-
-template <int G, bool FIRST>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) return_phase(LaunchDev ld,
-                                                                                       InstDev* __restrict__ inst,
-                                                                                       int pass)
-{
-    return_body<G, FIRST>(ld, inst, pass);
-}
-
-template <bool FIRST>
-__global__ void __launch_bounds__(BLOCK) return_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst, int pass)
-{
-    MGO_DISPATCH_G(block_groups(ld), (return_body<GG, FIRST>(ld, inst, pass)))
+    weights_body<G>(ld, inst, inst_offset);
 }
 
 template <int G>
-__global__ void __launch_bounds__(WAVE) replay_phase(LaunchDev ld, InstDev* __restrict__ inst)
+__global__ void __launch_bounds__(BLOCK) return_phase(LaunchDev ld, InstDev* __restrict__ inst)
 {
-    replay_body<G>(ld, inst);
+    return_body<G>(ld, inst);
+}
+
+template <int G>
+__global__ void __launch_bounds__(BLOCK) walk_phase(LaunchDev ld, InstDev* __restrict__ inst)
+{
+    __shared__ double buf[BLOCK * NC];
+    walk_body<G>(ld, inst, buf);
+}
+
+template <int G>
+__global__ void __launch_bounds__(SETTLE_BLOCK) settle_phase(LaunchDev ld, InstDev* __restrict__ inst)
+{
+    __shared__ int32_t list[SETTLE_LIST + 2];
+    __shared__ double buf[SETTLE_BLOCK * NC];
+    settle_body<G>(ld, inst, list, buf);
 }
 
 #if MGO_SHARD == 13
-__global__ void __launch_bounds__(WAVE) replay_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
+__global__ void __launch_bounds__(BLOCK) depart_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
 {
+    MGO_DISPATCH_G(block_groups(ld), (depart_body<GG>(ld, inst)))
+}
+
+__global__ void __launch_bounds__(BLOCK) return_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
+{
+    MGO_DISPATCH_G(block_groups(ld), (return_body<GG>(ld, inst)))
+}
+
+__global__ void __launch_bounds__(BLOCK) walk_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
+{
+    __shared__ double buf[BLOCK * NC];
+    MGO_DISPATCH_G(block_groups(ld), (walk_body<GG>(ld, inst, buf)))
+}
+
+__global__ void __launch_bounds__(SETTLE_BLOCK) settle_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
+{
+    __shared__ int32_t list[SETTLE_LIST + 2];
+    __shared__ double buf[SETTLE_BLOCK * NC];
     const InstDev& I = inst[ld.inst_ids[blockIdx.x]];
-    if (!I.c_active || I.c_action != 2 || I.fx_state != 2) {
+    if (!I.c_active || I.c_action != 2 || !I.fx_changed) {
         return;
     }
-    MGO_DISPATCH_G(ld.segs[I.seg].G, (replay_body<GG>(ld, inst)))
+    MGO_DISPATCH_G(ld.segs[I.seg].G, (settle_body<GG>(ld, inst, list, buf)))
 }
 #endif
 
@@ -1659,21 +2202,20 @@ hipError_t launch_edge_g(const LaunchDev& c, InstDev* inst, hipStream_t s)
 {
     const int nb = c.num_blocks;
     hipLaunchKernelGGL((depart_phase<G>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
-    hipLaunchKernelGGL((return_phase<G, true>), dim3(nb), dim3(BLOCK), 0, s, c, inst, 0);
-    hipError_t err = hipGetLastError();
-    const int ni   = (c.num_inst + 255) / 256;
-    for (int p = 1; p < FX_MAX_PASSES && err == hipSuccess; ++p) {
-        hipLaunchKernelGGL(fixup_check, dim3(ni), dim3(256), 0, s, c, inst);
-        hipLaunchKernelGGL((return_phase<G, false>), dim3(nb), dim3(BLOCK), 0, s, c, inst, p);
-        err = hipGetLastError();
+    hipLaunchKernelGGL((return_phase<G>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
+    if (c.general) {
+        hipLaunchKernelGGL((walk_phase<G>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
     }
-    if (err != hipSuccess) {
-        return err;
-    }
-    hipLaunchKernelGGL(fixup_check, dim3(ni), dim3(256), 0, s, c, inst);
     if (c.num_inst > 0) {
-        hipLaunchKernelGGL((replay_phase<G>), dim3(c.num_inst), dim3(WAVE), 0, s, c, inst);
+        hipLaunchKernelGGL((settle_phase<G>), dim3(c.num_inst), dim3(SETTLE_BLOCK), 0, s, c, inst);
     }
+    return hipGetLastError();
+}
+
+template <int G>
+hipError_t launch_weights_g(const LaunchDev& c, InstDev* inst, int inst_offset, hipStream_t s)
+{
+    hipLaunchKernelGGL((weights_phase<G>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst, inst_offset);
     return hipGetLastError();
 }
 
@@ -1690,6 +2232,7 @@ hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s);
 #if MGO_SHARD >= 1 && MGO_SHARD <= 8
 template hipError_t launch_node_g<MGO_SHARD>(const LaunchDev&, InstDev*, hipStream_t);
 template hipError_t launch_edge_g<MGO_SHARD>(const LaunchDev&, InstDev*, hipStream_t);
+template hipError_t launch_weights_g<MGO_SHARD>(const LaunchDev&, InstDev*, int, hipStream_t);
 #elif MGO_SHARD >= 9 && MGO_SHARD <= 12
 template hipError_t launch_node_mixed<MGO_SHARD - 9>(const LaunchDev&, InstDev*, hipStream_t);
 #elif MGO_SHARD == 13
@@ -1697,27 +2240,20 @@ hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s)
 {
     const int nb = c.num_blocks;
     hipLaunchKernelGGL(depart_phase_mixed, dim3(nb), dim3(BLOCK), 0, s, c, inst);
-    hipLaunchKernelGGL((return_phase_mixed<true>), dim3(nb), dim3(BLOCK), 0, s, c, inst, 0);
-    hipError_t err = hipGetLastError();
-    const int ni   = (c.num_inst + 255) / 256;
-    for (int p = 1; p < FX_MAX_PASSES && err == hipSuccess; ++p) {
-        hipLaunchKernelGGL(fixup_check, dim3(ni), dim3(256), 0, s, c, inst);
-        hipLaunchKernelGGL((return_phase_mixed<false>), dim3(nb), dim3(BLOCK), 0, s, c, inst, p);
-        err = hipGetLastError();
+    hipLaunchKernelGGL(return_phase_mixed, dim3(nb), dim3(BLOCK), 0, s, c, inst);
+    if (c.general) {
+        hipLaunchKernelGGL(walk_phase_mixed, dim3(nb), dim3(BLOCK), 0, s, c, inst);
     }
-    if (err != hipSuccess) {
-        return err;
-    }
-    hipLaunchKernelGGL(fixup_check, dim3(ni), dim3(256), 0, s, c, inst);
     if (c.num_inst > 0) {
-        hipLaunchKernelGGL(replay_phase_mixed, dim3(c.num_inst), dim3(WAVE), 0, s, c, inst);
+        hipLaunchKernelGGL(settle_phase_mixed, dim3(c.num_inst), dim3(SETTLE_BLOCK), 0, s, c, inst);
     }
     return hipGetLastError();
 }
 #else // MGO_SHARD == 0
 #define MGO_EXTERN_G(GG)                                                                                       \
     extern template hipError_t launch_node_g<GG>(const LaunchDev&, InstDev*, hipStream_t);                     \
-    extern template hipError_t launch_edge_g<GG>(const LaunchDev&, InstDev*, hipStream_t);
+    extern template hipError_t launch_edge_g<GG>(const LaunchDev&, InstDev*, hipStream_t);                     \
+    extern template hipError_t launch_weights_g<GG>(const LaunchDev&, InstDev*, int, hipStream_t);
 MGO_EXTERN_G(1)
 MGO_EXTERN_G(2)
 MGO_EXTERN_G(3)
@@ -1742,8 +2278,6 @@ hipError_t launch_clock(InstDev* inst, int n, int32_t* cyc, hipStream_t s)
 // Serving keeps every resident request's instance record in one table of slots. Admission and retirement
 // write whole records (table[ids[k]] = src[k]), class rebuilds renumber the segments (table[ids[k]].seg = k);
 // one launch each per loop iteration instead of one copy per request.
-static_assert(sizeof(InstDev) % 8 == 0, "instance records are copied as 8-byte words");
-
 static __global__ void scatter_slots_kernel(InstDev* __restrict__ table, const InstDev* __restrict__ src,
                                      const int32_t* __restrict__ ids, int n)
 {
@@ -1839,6 +2373,30 @@ hipError_t launch_edge(const LaunchDev& c, InstDev* inst, hipStream_t s)
         return launch_edge_g<7>(c, inst, s);
     case 8:
         return launch_edge_g<8>(c, inst, s);
+    default:
+        return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launch_weights(const LaunchDev& c, InstDev* inst, int inst_offset, hipStream_t s)
+{
+    switch (c.G) {
+    case 1:
+        return launch_weights_g<1>(c, inst, inst_offset, s);
+    case 2:
+        return launch_weights_g<2>(c, inst, inst_offset, s);
+    case 3:
+        return launch_weights_g<3>(c, inst, inst_offset, s);
+    case 4:
+        return launch_weights_g<4>(c, inst, inst_offset, s);
+    case 5:
+        return launch_weights_g<5>(c, inst, inst_offset, s);
+    case 6:
+        return launch_weights_g<6>(c, inst, inst_offset, s);
+    case 7:
+        return launch_weights_g<7>(c, inst, inst_offset, s);
+    case 8:
+        return launch_weights_g<8>(c, inst, inst_offset, s);
     default:
         return hipErrorInvalidValue;
     }

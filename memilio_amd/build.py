@@ -20,7 +20,7 @@ def _stale(obj, deps):
 
 
 # translation units: (source, object, extra flags, further dependencies); the kernels compile as shards
-UNITS = [("mgo_kernels.hip", f"mgo_kernels_{k}.o", [f"-DMGO_SHARD={k}"], []) for k in range(14)]
+UNITS = [("mgo_kernels.hip", f"mgo_kernels_{k}.o", [f"-DMGO_SHARD={k}"], []) for k in range(15)]
 UNITS.append(("mgo_host.cpp", "mgo_host.o", ["-x", "hip", "-ffp-contract=off"], ["mgo_serve.inc"]))
 
 
@@ -39,7 +39,7 @@ def build(verbose=False, only_changed=False):
             continue
         cmds.append([HIPCC, *COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj])
     # the largest shards first
-    cmds.sort(key=lambda c: not any(f"MGO_SHARD={k}" in " ".join(c) for k in (9, 10, 11, 12)))
+    cmds.sort(key=lambda c: not any(f"MGO_SHARD={k}" in " ".join(c) for k in (9, 10, 11, 12, 14)))
 
     def compile_one(cmd):
         if verbose:

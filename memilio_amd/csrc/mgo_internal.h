@@ -267,6 +267,8 @@ struct SegDev {
     double* out_d;                 // [node][g]
 };
 
+constexpr int MAX_SORT_RUNS = 4096; // percentiles: runs whose values one wavefront sorts in its registers
+
 // One kernel launch over the segments of a class.
 struct LaunchDev {
     const SegDev* segs;

@@ -1039,6 +1039,7 @@ struct Batch {
         int64_t pool_slots = 0;
         int wplanes        = 5;
         bool any_icu = false, any_general = false;
+        bool features = false; // some node has a feature that the plain node kernel leaves out (see NodeMode)
         for (int ii : C.insts) {
             RunSpec& r    = runs[size_t(ii)];
             InstHost& I   = inst[size_t(ii)];
@@ -1092,6 +1093,10 @@ struct Batch {
                 }
                 std::copy(g->populations + size_t(v) * G * NC, g->populations + size_t(v + 1) * G * NC,
                           y.begin() + long(node * G * NC));
+                for (int a = 0; a < G; ++a) {
+                    const double* y0 = &y[(node * G + size_t(a)) * NC];
+                    features         = features || y0[INSC] != 0.0 || y0[ISYC] != 0.0;
+                }
                 tnode[node]  = r.cfg.t0;
                 dtnode[node] = r.cfg.dt_node;
                 // damping cache
@@ -1145,6 +1150,9 @@ struct Batch {
                     dtime.insert(dtime.end(), tt.begin(), tt.end());
                     dmat.insert(dmat.end(), mm.begin(), mm.end());
                 }
+            }
+            for (int v = 0; v < g->num_nodes && !features; ++v) {
+                features = nodep[size_t(I.node_base) + size_t(v) * size_t(I.node_stride)].flags != 0;
             }
             // edge structure (shared between runs that pass the same edge arrays)
             InstDev& D = idev[size_t(ii)];
@@ -1432,7 +1440,7 @@ struct Batch {
         ld.num_blocks  = int(bseg.size());
         ld.G           = G;
         ld.kind        = C.kind;
-        ld.npi         = (C.npi.nodes0.empty() && C.oute.nodes0.empty()) ? 0 : 1;
+        ld.mode        = !(C.npi.nodes0.empty() && C.oute.nodes0.empty()) ? NPIS : features ? FEATURES : PLAIN;
         ld.general     = any_general ? 1 : 0;
         ld.cyc         = cyc.as<int32_t>();
     }

@@ -269,6 +269,12 @@ struct SegDev {
 
 constexpr int MAX_SORT_RUNS = 4096; // percentiles: runs whose values one wavefront sorts in its registers
 
+// Instantiations of the node kernel. PLAIN: no node of the launch has an optional feature (test-and-trace or ICU
+// limit, contact dampings, commuter detection, confirmed cases); eight compartments change (INSC and ISYC stay
+// zero: only commuter detection and initial values fill them) and every coefficient is constant. FEATURES: all
+// ten compartments, features by node flag. NPIS: FEATURES with the dynamic NPI checks.
+enum NodeMode : int { PLAIN = 0, FEATURES = 1, NPIS = 2 };
+
 // One kernel launch over the segments of a class.
 struct LaunchDev {
     const SegDev* segs;
@@ -279,7 +285,7 @@ struct LaunchDev {
     int32_t num_blocks;         // launched blocks (multiple of 8)
     int32_t G;                  // age groups of every segment, or 0: segments differ (mixed kernels)
     int32_t kind;
-    int32_t npi;                // some node has dynamic NPIs (per-G kernels only)
+    int32_t mode;               // NodeMode of the class's node kernel
     int32_t general;            // some instance's returns walk the edges (InstDev::general)
     int32_t* cyc;               // [CYC_FLAGS] cycle flags of the batch (or NULL: every phase runs its checks)
 };

@@ -2,8 +2,8 @@
 //
 // One lane per (node, age group): a wavefront holds 64/G nodes; a node's 10 compartments of one age
 // group live in the lane's registers. Cross-age-group terms (force of infection, test-and-trace demand,
-// ICU occupancy, the step's error norm) are group reductions over the node's G consecutive lanes with
-// ds_bpermute shuffles; the G x G contact row of the lane stays in registers. There is no dense
+// ICU occupancy, the step's error norm) are group reductions over the node's G consecutive lanes through LDS
+// slots and shuffles; the G x G contact row of the lane stays in registers. There is no dense
 // contraction, so everything runs on the FP64 vector ALUs.
 //
 // Kernels per half-day cycle (GraphSimulation::advance, cpp/memilio/mobility/graph_simulation.h:101-120):
@@ -37,6 +37,11 @@ namespace mgo
 {
 
 #define MGO_PI 3.14159265358979323846
+
+// Fused multiply-adds are written out: every instantiation of a body (age groups, with or without the optional
+// model features, per-G or mixed) then rounds alike, and a run's results do not depend on the kernel that a
+// batch's other runs bring with them.
+#pragma clang fp contract(off)
 
 // Segment and edge-structure descriptors do not change during a launch and are read from the constant address
 // space: the pointers they hold are then known to be global. Read as ordinary memory they are generic, and every
@@ -72,7 +77,7 @@ __device__ __forceinline__ double smoother_cosine(double x, double xl, double xr
     if (x >= xr) {
         return yr;
     }
-    return 0.5 * (yl - yr) * cos(MGO_PI / (xr - xl) * (x - xl)) + 0.5 * (yl + yr);
+    return fma(0.5 * (yl - yr), cospi((x - xl) / (xr - xl)), 0.5 * (yl + yr));
 }
 
 // Blocks are dispatched round-robin over the 8 XCDs; map the hardware block id so that each XCD gets a
@@ -144,86 +149,133 @@ __device__ __forceinline__ double recip_pop(double x)
     return fma(r, e, r);
 }
 
+// compartments of a lane in registers
+template <int M>
+struct Comps {
+    static constexpr int N = M == PLAIN ? 8 : NC;
+    static constexpr int S = 0, E = 1, INS = 2;
+    static constexpr int INSC = 3; // FEATURES and NPIS only, like ISYC
+    static constexpr int ISY  = M == PLAIN ? 3 : 4;
+    static constexpr int ISYC = 5;
+    static constexpr int ISEV = M == PLAIN ? 4 : 6;
+    static constexpr int ICR  = M == PLAIN ? 5 : 7;
+    static constexpr int R    = M == PLAIN ? 6 : 8;
+    static constexpr int D    = M == PLAIN ? 7 : 9;
+    // register of compartment i of the state layout, or -1
+    __device__ static constexpr int of(int i)
+    {
+        return M != PLAIN ? i : (i < mgo::INSC) ? i : (i == mgo::INSC || i == mgo::ISYC) ? -1 : (i == mgo::ISY) ? 3 : i - 2;
+    }
+};
+
 // Per-lane context of one node lane, loaded once per kernel.
-template <int G>
+template <int G, int M>
 struct Lane {
-    double c[NUM_LC];
-    double crow[G];   // contact row at the last evaluated time (constant without dampings)
-    NodeP np;
+    // rates (see LaneCoef); isev: the sum of ISev's
+    double e, ins_isy, ins_r, isy_isev, isy_r, isev_icr, isev_r, isev_d, isev, icr_d, icr_r;
+    double rel, risk, tp;
+    double crow[G]; // contact row times tp at the last evaluated time (constant without dampings)
+    // features
+    double ttr, maxrisk, cps, dps, tisev, ttc, ttc_hi, icu_cap;
+    const gdouble* damp_time;
+    const gdouble* damp_mat;
+    int damp_cnt;
+    double row_lo, row_hi; // crow holds for row_lo <= t <= row_hi (dampings)
+    int flags;
     int node;
     int age;
     int base;         // first lane of the node's group
+    int inst;
     double* wx;       // LDS: the wavefront's exchange slots, one double per lane (force of infection, error norm)
     double* ws;       // LDS: the wavefront's stage-season slots, (5 + G - 1) / G planes of BLOCK doubles
+    double* cold;     // LDS: the lane's Cold values, planes of BLOCK doubles
 };
 
-// Effective contact row C(t)_age,. = B - D(t) o (B - M) (contact_matrix.h:190-194, damping.h:381-396)
+// Scalars of a lane that a step attempt reads at most a few times: kept in LDS, since the registers of two
+// wavefronts per SIMD hold the stage vectors (in registers, 25 values per attempt went through scratch memory).
+enum Cold : int {
+    COLD_ABS = 0,
+    COLD_REL,
+    COLD_DT_MAX,
+    COLD_DT_MIN,
+    COLD_DT_RESTORE,
+    COLD_TMAX,   // end of the piece
+    COLD_SPAN,   // its length
+    COLD_SEASON, // season of the next k1
+    COLD_START_DAY,
+    COLD_SEASONALITY,
+    COLD_DAYS,   // two integers: next output day, end of the output days (both counted from day0)
+    COLD_COUNTS, // two integers: steps, attempts
+    NUM_COLD
+};
+
+// LDS of a node kernel: exchange slots, stage-season planes, cold planes
 template <int G>
-__device__ __forceinline__ void contact_row(Seg& c, Lane<G>& L, double t)
+constexpr int node_lds()
 {
-    const double* B = c.cbase + (size_t(L.node) * G + L.age) * G;
-    if (!(L.np.flags & NF_DAMPED)) {
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-            L.crow[j] = B[j];
-        }
+    return BLOCK * (1 + (5 + G - 1) / G + NUM_COLD);
+}
+
+// Effective contact row C(t)_age,. = B - D(t) o (B - M) (contact_matrix.h:190-194, damping.h:381-396), times tp, of
+// a node with dampings. D changes only within the day before a damping's time: outside of it the row and its
+// interval are kept, so that most right-hand sides do without the chain of loads from the damping cache (their
+// latency, in every right-hand side, was most of the node kernel's time on damped nodes).
+template <int G, int M>
+__device__ __forceinline__ void contact_row(Seg& c, Lane<G, M>& L, double t)
+{
+    if (t >= L.row_lo && t <= L.row_hi) {
         return;
     }
-    const gdouble* tk = (const gdouble*)L.np.damp_time;
+    const double* B   = c.cbase + (size_t(L.node) * G + L.age) * G;
+    const gdouble* tk = L.damp_time;
     int k             = 1;
-    while (k < L.np.damp_cnt - 1 && !(tk[k] > t)) {
+    while (k < L.damp_cnt - 1 && !(tk[k] > t)) {
         ++k;
     }
     const double xr    = tk[k];
     const double xl    = xr - 1.0;
-    const gdouble* Dl  = (const gdouble*)L.np.damp_mat + (size_t(k - 1) * G + L.age) * G;
-    const gdouble* Dr  = (const gdouble*)L.np.damp_mat + (size_t(k) * G + L.age) * G;
+    const gdouble* Dl  = L.damp_mat + (size_t(k - 1) * G + L.age) * G;
+    const gdouble* Dr  = L.damp_mat + (size_t(k) * G + L.age) * G;
     const double* Dd   = c.cdelta + (size_t(L.node) * G + L.age) * G;
     const bool left    = t <= xl;
     const bool right   = t >= xr;
-    const double cs    = (left || right) ? 0.0 : cos(MGO_PI / (xr - xl) * (t - xl));
+    const double cs    = (left || right) ? 0.0 : cospi((t - xl) / (xr - xl));
+    L.row_lo           = left ? tk[k - 1] : INFINITY;
+    L.row_hi           = left ? xl : -INFINITY;
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-        const double d = left ? Dl[j] : (right ? Dr[j] : 0.5 * (Dl[j] - Dr[j]) * cs + 0.5 * (Dl[j] + Dr[j]));
-        L.crow[j]      = B[j] - d * Dd[j];
+        const double d = left ? Dl[j] : (right ? Dr[j] : fma(0.5 * (Dl[j] - Dr[j]), cs, 0.5 * (Dl[j] + Dr[j])));
+        L.crow[j]      = L.tp * fma(-d, Dd[j], B[j]);
     }
 }
 
 // Seasonal factor 1 + k sin(pi ((StartDay + t) / 182.5 + 0.5)) of the lane's node at time t
-// (model.h:115-117).
-template <int G>
-__device__ __forceinline__ double season_at(const Lane<G>& L, double t)
+// (model.h:115-117). sinpi reduces its argument exactly; sin needs a reduction by pi whose code (and registers)
+// was a tenth of the kernel.
+template <int G, int M>
+__device__ __forceinline__ double season_at(const Lane<G, M>& L, double t)
 {
-    return 1.0 + L.np.seasonality * sin(MGO_PI * ((L.np.start_day + t) / 182.5 + 0.5));
+    return fma(L.cold[COLD_SEASONALITY * BLOCK], sinpi(fma(L.cold[COLD_START_DAY * BLOCK] + t, 1.0 / 182.5, 0.5)), 1.0);
 }
 
 // Seasonal factors of the five later stages of a step, spread over the node's G lanes: lane a evaluates
 // stages j = a, a + G, ... (j < 5) at t + c_j h, and every lane reads a stage's factor from the lane that
 // owns it (one sin per lane and step attempt for G >= 5 instead of five).
-template <int G>
-struct StageSeasons {
-    static constexpr int N = (5 + G - 1) / G;
-    double v[N];
-};
-
-template <int G>
-__device__ __forceinline__ StageSeasons<G> stage_seasons(const Lane<G>& L, double t, double h, double c2, double c3,
-                                                         double c4, double c5, double c6)
+template <int G, int M>
+__device__ __forceinline__ void stage_seasons(const Lane<G, M>& L, double t, double h, double c2, double c3,
+                                              double c4, double c5, double c6)
 {
-    StageSeasons<G> s;
 #pragma unroll
-    for (int q = 0; q < StageSeasons<G>::N; ++q) {
+    for (int q = 0; q < (5 + G - 1) / G; ++q) {
         const int j    = L.age + q * G;
         const double c = (j == 0) ? c2 : (j == 1) ? c3 : (j == 2) ? c4 : (j == 3) ? c5 : c6;
-        s.v[q]         = (j < 5) ? season_at<G>(L, t + c * h) : 1.0;
-        L.ws[q * BLOCK + threadIdx.x % WAVE] = s.v[q]; // read by the node's lanes from the wavefront's slots
+        L.ws[q * BLOCK + threadIdx.x % WAVE] = (j < 5) ? season_at(L, fma(c, h, t)) : 1.0;
     }
-    __builtin_amdgcn_wave_barrier();
-    return s;
+    wave_sync();
 }
 
-template <int G, int J>
-__device__ __forceinline__ double stage_season(const Lane<G>& L, const StageSeasons<G>&)
+template <int J, int G, int M>
+__device__ __forceinline__ double stage_season(const Lane<G, M>& L)
 {
     return L.ws[(J / G) * BLOCK + L.base + J % G];
 }
@@ -231,84 +283,88 @@ __device__ __forceinline__ double stage_season(const Lane<G>& L, const StageSeas
 // Force-of-infection coefficient of the lane's age group: season * tp * sum_j C_gj(t) w_j(pop),
 // w_j = divN_j * (rel_j pop[INS_j] + risk_j pop[ISy_j]) (model.h:99-145, factored over j). Also returns
 // the ICU-adjusted ISev->ICr / ISev->D coefficients (model.h:147-152, 196-204).
-template <int G>
-__device__ __forceinline__ double force_of_infection(Seg& c, Lane<G>& L, const double (&pop)[NC], double t,
+template <int G, int M>
+__device__ __forceinline__ double force_of_infection(Seg& c, Lane<G, M>& L, const double (&pop)[Comps<M>::N], double t,
                                                      double season, double& c_icr, double& c_d)
 {
-    double risk = L.c[LC_RISK];
-    if (L.np.flags & NF_TTC_ACTIVE) {
-        const double ttr = group_sum<G>(L.c[LC_TTR] * pop[INS], L.base);
-        risk             = smoother_cosine(ttr, L.np.ttc, L.np.ttc_hi, L.c[LC_RISK], L.c[LC_MAXRISK]);
+    using X     = Comps<M>;
+    double risk = L.risk;
+    if (M != PLAIN && (L.flags & NF_TTC_ACTIVE)) {
+        const double ttr = group_sum<G>(L.ttr * pop[X::INS], L.base);
+        risk             = smoother_cosine(ttr, L.ttc, L.ttc_hi, L.risk, L.maxrisk);
     }
-    const double Nj   = pop[S] + pop[E] + pop[INS] + pop[ISY] + pop[ISEV] + pop[ICR] + pop[R];
+    const double Nj = ((pop[X::S] + pop[X::E]) + (pop[X::INS] + pop[X::ISY])) + ((pop[X::ISEV] + pop[X::ICR]) + pop[X::R]);
     const double divN = (Nj < 1e-12) ? 0.0 : recip_pop(Nj);
-    const double w    = divN * (L.c[LC_REL] * pop[INS] + risk * pop[ISY]);
-    if (L.np.flags & NF_DAMPED) {
-        contact_row<G>(c, L, t);
+    const double w    = divN * fma(L.rel, pop[X::INS], risk * pop[X::ISY]);
+    if (M != PLAIN && (L.flags & NF_DAMPED)) {
+        contact_row(c, L, t);
     }
     // w of the node's G lanes through the wavefront's LDS slots: one write, G reads (a wavefront's LDS
     // instructions complete in order; the lanes of a node are active together)
     L.wx[threadIdx.x % WAVE] = w;
-    __builtin_amdgcn_wave_barrier();
-    double lam = 0.0;
+    wave_sync();
+    double wg[G];
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-        lam += L.crow[j] * L.wx[L.base + j];
+        wg[j] = L.wx[L.base + j];
     }
-    __builtin_amdgcn_wave_barrier();
-    c_icr = L.c[LC_ISEV_ICR];
-    c_d   = L.c[LC_ISEV_D];
-    if (L.np.flags & NF_ICU_ACTIVE) {
-        const double icu  = group_sum<G>(pop[ICR], L.base);
-        const double crit = smoother_cosine(icu, 0.90 * L.np.icu, L.np.icu, L.c[LC_CPS], 0.0);
-        c_icr             = crit / L.c[LC_TISEV];
-        c_d               = (L.c[LC_DPS] + (L.c[LC_CPS] - crit)) / L.c[LC_TISEV];
+    wave_sync();
+    double lam = L.crow[0] * wg[0], lam1 = 0.0; // two chains: half the latency
+    if constexpr (G > 1) {
+        lam1 = L.crow[1] * wg[1];
     }
-    return season * L.c[LC_TP] * lam;
+#pragma unroll
+    for (int j = 2; j < G; ++j) {
+        double& l = (j & 1) ? lam1 : lam;
+        l         = fma(L.crow[j], wg[j], l);
+    }
+    lam += lam1;
+    c_icr = L.isev_icr;
+    c_d   = L.isev_d;
+    if (M != PLAIN && (L.flags & NF_ICU_ACTIVE)) {
+        const double icu  = group_sum<G>(pop[X::ICR], L.base);
+        const double crit = smoother_cosine(icu, 0.90 * L.icu_cap, L.icu_cap, L.cps, 0.0);
+        c_icr             = crit / L.tisev;
+        c_d               = (L.dps + (L.cps - crit)) / L.tisev;
+    }
+    return season * lam;
 }
 
-// flows of one age group -> derivative (flow_model.h:112-125,219-235 with the osecir Flows order)
-__device__ __forceinline__ void flows_to_dydt(const double (&y)[NC], double kappa, double cE, double cINS_ISY,
-                                              double cINS_R, double cISY_ISEV, double cISY_R, double cISEV_ICR,
-                                              double cISEV_R, double cISEV_D, double cICR_D, double cICR_R,
-                                              double (&dy)[NC])
+// Right-hand side of the node ODE, pop == y (osecir::Model::get_flows + FlowModel::get_derivatives,
+// flow_model.h:112-125,219-235). A flow that leaves one compartment and enters another is computed once where two
+// uses need it and fused into the sums elsewhere.
+template <int G, int M>
+__device__ __forceinline__ void rhs(Seg& c, Lane<G, M>& L, const double (&y)[Comps<M>::N], double t, double season,
+                                    double (&dy)[Comps<M>::N])
 {
-    const double f0  = y[S] * kappa;
-    const double f1  = cE * y[E];
-    const double f2  = cINS_ISY * y[INS];
-    const double f3  = cINS_R * y[INS];
-    const double f4  = cINS_ISY * y[INSC];
-    const double f5  = cINS_R * y[INSC];
-    const double f6  = cISY_ISEV * y[ISY];
-    const double f7  = cISY_R * y[ISY];
-    const double f8  = cISY_ISEV * y[ISYC];
-    const double f9  = cISY_R * y[ISYC];
-    const double f10 = cISEV_ICR * y[ISEV];
-    const double f11 = cISEV_R * y[ISEV];
-    const double f12 = cISEV_D * y[ISEV];
-    const double f13 = cICR_D * y[ICR];
-    const double f14 = cICR_R * y[ICR];
-    dy[S]    = -f0;
-    dy[E]    = f0 - f1;
-    dy[INS]  = (f1 - f2) - f3;
-    dy[INSC] = -f4 - f5;
-    dy[ISY]  = (f2 - f6) - f7;
-    dy[ISYC] = (f4 - f8) - f9;
-    dy[ISEV] = (((f6 + f8) - f10) - f11) - f12;
-    dy[ICR]  = (f10 - f13) - f14;
-    dy[R]    = ((((f3 + f5) + f7) + f9) + f11) + f14;
-    dy[D]    = f12 + f13;
-}
-
-// Right-hand side of the node ODE, pop == y (osecir::Model::get_flows + FlowModel::get_derivatives)
-template <int G>
-__device__ __forceinline__ void rhs(Seg& c, Lane<G>& L, const double (&y)[NC], double t, double season,
-                                    double (&dy)[NC])
-{
+    using X = Comps<M>;
     double c_icr, c_d;
-    const double kappa = force_of_infection<G>(c, L, y, t, season, c_icr, c_d);
-    flows_to_dydt(y, kappa, L.c[LC_E], L.c[LC_INS_ISY], L.c[LC_INS_R], L.c[LC_ISY_ISEV], L.c[LC_ISY_R], c_icr,
-                  L.c[LC_ISEV_R], c_d, L.c[LC_ICR_D], L.c[LC_ICR_R], dy);
+    const double f0   = y[X::S] * force_of_infection(c, L, y, t, season, c_icr, c_d);
+    const double f1   = L.e * y[X::E];
+    const double f2   = L.ins_isy * y[X::INS];
+    const double f6   = L.isy_isev * y[X::ISY];
+    double isev       = L.isev;
+    double to_isev    = f6;
+    double to_r       = fma(L.ins_r, y[X::INS], fma(L.isy_r, y[X::ISY], fma(L.isev_r, y[X::ISEV], L.icr_r * y[X::ICR])));
+    if constexpr (M != PLAIN) {
+        if (L.flags & NF_ICU_ACTIVE) {
+            isev = (c_icr + L.isev_r) + c_d;
+        }
+        const double f4 = L.ins_isy * y[X::INSC];
+        const double f8 = L.isy_isev * y[X::ISYC];
+        to_isev += f8;
+        to_r        = fma(L.ins_r, y[X::INSC], fma(L.isy_r, y[X::ISYC], to_r));
+        dy[X::INSC] = fma(-L.ins_r, y[X::INSC], -f4);
+        dy[X::ISYC] = fma(-L.isy_r, y[X::ISYC], f4 - f8);
+    }
+    dy[X::S]    = -f0;
+    dy[X::E]    = f0 - f1;
+    dy[X::INS]  = fma(-L.ins_r, y[X::INS], f1 - f2);
+    dy[X::ISY]  = fma(-L.isy_r, y[X::ISY], f2 - f6);
+    dy[X::ISEV] = fma(-isev, y[X::ISEV], to_isev);
+    dy[X::ICR]  = fma(-L.icr_r, y[X::ICR], fma(-L.icr_d, y[X::ICR], c_icr * y[X::ISEV]));
+    dy[X::R]    = to_r;
+    dy[X::D]    = fma(c_d, y[X::ISEV], L.icr_d * y[X::ICR]);
 }
 
 // ------------------------------------------------------------------------------- Cash-Karp 5(4)
@@ -328,50 +384,67 @@ constexpr double E1 = 37.0 / 378.0 - 2825.0 / 27648.0, E3 = 250.0 / 621.0 - 1857
 } // namespace ck
 
 // One Cash-Karp step from (y, k1 = f(y, t)) with step h: 5th-order solution in yo, embedded error in er.
-template <int G>
-__device__ __forceinline__ void cash_karp_stages(Seg& c, Lane<G>& L, const double (&y)[NC],
-                                                 const double (&k1)[NC], double t, double h, double (&yo)[NC],
-                                                 double (&er)[NC], bool want_err, double& season_end)
+template <int G, int M>
+__device__ __forceinline__ void cash_karp_stages(Seg& c, Lane<G, M>& L, const double (&y)[Comps<M>::N],
+                                                 const double (&k1)[Comps<M>::N], double t, double h,
+                                                 double (&yo)[Comps<M>::N], double (&er)[Comps<M>::N], bool want_err)
 {
-    const StageSeasons<G> ss = stage_seasons<G>(L, t, h, ck::C2, ck::C3, ck::C4, ck::C5, ck::C6);
-    double k2[NC], k3[NC], k4[NC], k5[NC], yt[NC];
+    constexpr int N = Comps<M>::N;
+    stage_seasons(L, t, h, ck::C2, ck::C3, ck::C4, ck::C5, ck::C6);
+    double k2[N], k3[N], k4[N], k5[N], yt[N];
+    {
+        const double a1 = ck::A21 * h;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (ck::A21 * h) * k1[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a1, k1[i], y[i]);
+        }
     }
-    rhs<G>(c, L, yt, t + ck::C2 * h, stage_season<G, 0>(L, ss), k2);
+    rhs(c, L, yt, fma(ck::C2, h, t), stage_season<0>(L), k2);
+    {
+        const double a1 = ck::A31 * h, a2 = ck::A32 * h;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (ck::A31 * h) * k1[i] + (ck::A32 * h) * k2[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a2, k2[i], fma(a1, k1[i], y[i]));
+        }
     }
-    rhs<G>(c, L, yt, t + ck::C3 * h, stage_season<G, 1>(L, ss), k3);
+    rhs(c, L, yt, fma(ck::C3, h, t), stage_season<1>(L), k3);
+    {
+        const double a1 = ck::A41 * h, a2 = ck::A42 * h, a3 = ck::A43 * h;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (ck::A41 * h) * k1[i] + (ck::A42 * h) * k2[i] + (ck::A43 * h) * k3[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a3, k3[i], fma(a2, k2[i], fma(a1, k1[i], y[i])));
+        }
     }
-    rhs<G>(c, L, yt, t + ck::C4 * h, stage_season<G, 2>(L, ss), k4);
+    rhs(c, L, yt, fma(ck::C4, h, t), stage_season<2>(L), k4);
+    {
+        const double a1 = ck::A51 * h, a2 = ck::A52 * h, a3 = ck::A53 * h, a4 = ck::A54 * h;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (ck::A51 * h) * k1[i] + (ck::A52 * h) * k2[i] + (ck::A53 * h) * k3[i] + (ck::A54 * h) * k4[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a4, k4[i], fma(a3, k3[i], fma(a2, k2[i], fma(a1, k1[i], y[i]))));
+        }
     }
-    season_end = stage_season<G, 3>(L, ss); // C5 = 1: the season at t + h, the next step's k1 time
-    rhs<G>(c, L, yt, t + ck::C5 * h, season_end, k5);
+    rhs(c, L, yt, fma(ck::C5, h, t), stage_season<3>(L), k5);
+    {
+        const double a1 = ck::A61 * h, a2 = ck::A62 * h, a3 = ck::A63 * h, a4 = ck::A64 * h, a5 = ck::A65 * h;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (ck::A61 * h) * k1[i] + (ck::A62 * h) * k2[i] + (ck::A63 * h) * k3[i] + (ck::A64 * h) * k4[i] +
-                (ck::A65 * h) * k5[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a5, k5[i], fma(a4, k4[i], fma(a3, k3[i], fma(a2, k2[i], fma(a1, k1[i], y[i])))));
+        }
     }
-    double k6[NC];
-    rhs<G>(c, L, yt, t + ck::C6 * h, stage_season<G, 4>(L, ss), k6);
+    double(&k6)[N] = k2; // k2 is no longer needed
+    rhs(c, L, yt, fma(ck::C6, h, t), stage_season<4>(L), k6);
+    {
+        const double b1 = ck::B1 * h, b3 = ck::B3 * h, b4 = ck::B4 * h, b6 = ck::B6 * h;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yo[i] = y[i] + (ck::B1 * h) * k1[i] + (ck::B3 * h) * k3[i] + (ck::B4 * h) * k4[i] + (ck::B6 * h) * k6[i];
+        for (int i = 0; i < N; ++i) {
+            yo[i] = fma(b6, k6[i], fma(b4, k4[i], fma(b3, k3[i], fma(b1, k1[i], y[i]))));
+        }
     }
     if (want_err) {
+        const double e1 = ck::E1 * h, e3 = ck::E3 * h, e4 = ck::E4 * h, e5 = ck::E5 * h, e6 = ck::E6 * h;
 #pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            er[i] = (ck::E1 * h) * k1[i] + (ck::E3 * h) * k3[i] + (ck::E4 * h) * k4[i] + (ck::E5 * h) * k5[i] +
-                    (ck::E6 * h) * k6[i];
+        for (int i = 0; i < N; ++i) {
+            er[i] = fma(e6, k6[i], fma(e5, k5[i], fma(e4, k4[i], fma(e3, k3[i], e1 * k1[i]))));
         }
     }
 }
@@ -391,55 +464,72 @@ constexpr double BH1 = 16 / 135.0, BH3 = 6656 / 12825.0, BH4 = 28561 / 56430.0, 
 constexpr double D1 = BH1 - BL1, D3 = BH3 - BL3, D4 = BH4 - BL4, D5 = BH5 - BL5, D6 = BH6 - 0.0;
 } // namespace rkf
 
-template <int G>
-__device__ __forceinline__ void rkf45_stages(Seg& c, Lane<G>& L, const double (&y)[NC],
-                                             const double (&k1)[NC], double t, double h, double (&yo)[NC],
-                                             double (&er)[NC], double& season_end)
+template <int G, int M>
+__device__ __forceinline__ void rkf45_stages(Seg& c, Lane<G, M>& L, const double (&y)[Comps<M>::N],
+                                             const double (&k1)[Comps<M>::N], double t, double h,
+                                             double (&yo)[Comps<M>::N], double (&er)[Comps<M>::N])
 {
-    const StageSeasons<G> ss = stage_seasons<G>(L, t, h, rkf::C2, rkf::C3, rkf::C4, rkf::C5, rkf::C6);
-    double k2[NC], k3[NC], k4[NC], k5[NC], k6[NC], yt[NC];
+    constexpr int N = Comps<M>::N;
+    stage_seasons(L, t, h, rkf::C2, rkf::C3, rkf::C4, rkf::C5, rkf::C6);
+    double k2[N], k3[N], k4[N], k5[N], yt[N];
+    {
+        const double a1 = h * rkf::A21;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (h * rkf::A21) * k1[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a1, k1[i], y[i]);
+        }
     }
-    rhs<G>(c, L, yt, t + rkf::C2 * h, stage_season<G, 0>(L, ss), k2);
+    rhs(c, L, yt, fma(rkf::C2, h, t), stage_season<0>(L), k2);
+    {
+        const double a1 = h * rkf::A31, a2 = h * rkf::A32;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (h * rkf::A31) * k1[i] + (h * rkf::A32) * k2[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a2, k2[i], fma(a1, k1[i], y[i]));
+        }
     }
-    rhs<G>(c, L, yt, t + rkf::C3 * h, stage_season<G, 1>(L, ss), k3);
+    rhs(c, L, yt, fma(rkf::C3, h, t), stage_season<1>(L), k3);
+    {
+        const double a1 = h * rkf::A41, a2 = h * rkf::A42, a3 = h * rkf::A43;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (h * rkf::A41) * k1[i] + (h * rkf::A42) * k2[i] + (h * rkf::A43) * k3[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a3, k3[i], fma(a2, k2[i], fma(a1, k1[i], y[i])));
+        }
     }
-    rhs<G>(c, L, yt, t + rkf::C4 * h, stage_season<G, 2>(L, ss), k4);
+    rhs(c, L, yt, fma(rkf::C4, h, t), stage_season<2>(L), k4);
+    {
+        const double a1 = h * rkf::A51, a2 = h * rkf::A52, a3 = h * rkf::A53, a4 = h * rkf::A54;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (h * rkf::A51) * k1[i] + (h * rkf::A52) * k2[i] + (h * rkf::A53) * k3[i] + (h * rkf::A54) * k4[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a4, k4[i], fma(a3, k3[i], fma(a2, k2[i], fma(a1, k1[i], y[i]))));
+        }
     }
-    season_end = stage_season<G, 3>(L, ss); // C5 = 1: the season at t + h, the next step's k1 time
-    rhs<G>(c, L, yt, t + rkf::C5 * h, season_end, k5);
+    rhs(c, L, yt, fma(rkf::C5, h, t), stage_season<3>(L), k5);
+    {
+        const double a1 = h * rkf::A61, a2 = h * rkf::A62, a3 = h * rkf::A63, a4 = h * rkf::A64, a5 = h * rkf::A65;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        yt[i] = y[i] + (h * rkf::A61) * k1[i] + (h * rkf::A62) * k2[i] + (h * rkf::A63) * k3[i] +
-                (h * rkf::A64) * k4[i] + (h * rkf::A65) * k5[i];
+        for (int i = 0; i < N; ++i) {
+            yt[i] = fma(a5, k5[i], fma(a4, k4[i], fma(a3, k3[i], fma(a2, k2[i], fma(a1, k1[i], y[i])))));
+        }
     }
-    rhs<G>(c, L, yt, t + rkf::C6 * h, stage_season<G, 4>(L, ss), k6);
+    double(&k6)[N] = k2; // k2 is no longer needed
+    rhs(c, L, yt, fma(rkf::C6, h, t), stage_season<4>(L), k6);
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
+    for (int i = 0; i < N; ++i) {
         // y + dt * (K * b_low) and dt * |K * (b_high - b_low)| (adapt_rk.h:268-271)
-        const double sl = k1[i] * rkf::BL1 + k3[i] * rkf::BL3 + k4[i] * rkf::BL4 + k5[i] * rkf::BL5;
-        yo[i]           = y[i] + sl * h;
-        const double sd = k1[i] * rkf::D1 + k3[i] * rkf::D3 + k4[i] * rkf::D4 + k5[i] * rkf::D5 + k6[i] * rkf::D6;
-        er[i]           = h * fabs(sd);
+        const double sl = fma(k5[i], rkf::BL5, fma(k4[i], rkf::BL4, fma(k3[i], rkf::BL3, k1[i] * rkf::BL1)));
+        yo[i]           = fma(sl, h, y[i]);
+        const double sd =
+            fma(k6[i], rkf::D6, fma(k5[i], rkf::D5, fma(k4[i], rkf::D4, fma(k3[i], rkf::D3, k1[i] * rkf::D1))));
+        er[i] = h * fabs(sd);
     }
 }
 
-template <int G>
-__device__ __forceinline__ Seg* load_lane(const LaunchDev& ld, Lane<G>& L, double* wx)
+template <int G, int M>
+__device__ __forceinline__ Seg* load_lane(const LaunchDev& ld, Lane<G, M>& L, double* wx)
 {
     L.wx = wx + (threadIdx.x / WAVE) * WAVE;
     L.ws = wx + BLOCK + (threadIdx.x / WAVE) * WAVE;
+    L.cold = wx + BLOCK * (1 + (5 + G - 1) / G) + threadIdx.x;
     constexpr int NPW = WAVE / G;
     const int lb      = xcd_block();
     if (lb >= ld.num_blocks) {
@@ -462,16 +552,52 @@ __device__ __forceinline__ Seg* load_lane(const LaunchDev& ld, Lane<G>& L, doubl
     if (c->node_order) {
         L.node = c->node_order[L.node]; // same graph node of consecutive runs in one wavefront
     }
-    L.np            = c->nodep[L.node];
-    const double* p = c->lcoef + (size_t(L.node) * G + L.age) * NUM_LC;
+    const NodeP& np = c->nodep[L.node];
+    L.flags         = np.flags;
+    L.inst          = np.inst;
+    L.cold[COLD_START_DAY * BLOCK]   = np.start_day;
+    L.cold[COLD_SEASONALITY * BLOCK] = np.seasonality;
+    double lc[NUM_LC];
+    const double2* p = reinterpret_cast<const double2*>(c->lcoef + (size_t(L.node) * G + L.age) * NUM_LC);
 #pragma unroll
-    for (int k = 0; k < NUM_LC; ++k) {
-        L.c[k] = p[k];
+    for (int k = 0; k < NUM_LC / 2; ++k) {
+        const double2 v = p[k];
+        lc[2 * k]       = v.x;
+        lc[2 * k + 1]   = v.y;
+    }
+    L.e        = lc[LC_E];
+    L.ins_isy  = lc[LC_INS_ISY];
+    L.ins_r    = lc[LC_INS_R];
+    L.isy_isev = lc[LC_ISY_ISEV];
+    L.isy_r    = lc[LC_ISY_R];
+    L.isev_icr = lc[LC_ISEV_ICR];
+    L.isev_r   = lc[LC_ISEV_R];
+    L.isev_d   = lc[LC_ISEV_D];
+    L.isev     = (lc[LC_ISEV_ICR] + lc[LC_ISEV_R]) + lc[LC_ISEV_D];
+    L.icr_d    = lc[LC_ICR_D];
+    L.icr_r    = lc[LC_ICR_R];
+    L.tp       = lc[LC_TP];
+    L.rel      = lc[LC_REL];
+    L.risk     = lc[LC_RISK];
+    if constexpr (M != PLAIN) {
+        L.maxrisk   = lc[LC_MAXRISK];
+        L.ttr       = lc[LC_TTR];
+        L.cps       = lc[LC_CPS];
+        L.dps       = lc[LC_DPS];
+        L.tisev     = lc[LC_TISEV];
+        L.ttc       = np.ttc;
+        L.ttc_hi    = np.ttc_hi;
+        L.icu_cap   = np.icu;
+        L.damp_time = (const gdouble*)np.damp_time;
+        L.damp_mat  = (const gdouble*)np.damp_mat;
+        L.damp_cnt  = np.damp_cnt;
+        L.row_lo    = INFINITY;
+        L.row_hi    = -INFINITY;
     }
     const double* B = c->cbase + (size_t(L.node) * G + L.age) * G;
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-        L.crow[j] = B[j];
+        L.crow[j] = L.tp * B[j];
     }
     return c;
 }
@@ -483,14 +609,14 @@ __device__ __forceinline__ double detect_nondetection(const NodeP& np, double t)
 }
 
 // mobility factor of the ISy compartment of the lane's age group (model.h:687-715)
-template <int G>
-__device__ __forceinline__ double mobility_factor(const Lane<G>& L, const double (&y)[NC])
+template <int G, int M>
+__device__ __forceinline__ double mobility_factor(const Lane<G, M>& L, double y_ins)
 {
-    if (!(L.np.flags & NF_TTC_ACTIVE)) {
-        return L.c[LC_RISK];
+    if (M == PLAIN || !(L.flags & NF_TTC_ACTIVE)) {
+        return L.risk;
     }
-    const double ttr = group_sum<G>(L.c[LC_TTR] * y[INS], L.base);
-    return smoother_cosine(ttr, L.np.ttc, L.np.ttc_hi, L.c[LC_RISK], L.c[LC_MAXRISK]);
+    const double ttr = group_sum<G>(L.ttr * y_ins, L.base);
+    return smoother_cosine(ttr, L.ttc, L.ttc_hi, L.risk, L.maxrisk);
 }
 
 // ------------------------------------------------------------------------------- clock
@@ -647,12 +773,12 @@ __device__ __forceinline__ void store_planes(double2* p, size_t stride, size_t l
 // metapopulation_mobility_instant.h:460-471): the force of infection and the ICU-adjusted rates of the state
 // pop at the departure time, frozen for the Euler step of the returning travelers (the other rates are lane
 // constants).
-template <int G>
-__device__ __forceinline__ void return_coefficients(Seg& c, Lane<G>& L, const InstDev& I,
-                                                    const double (&pop)[NC])
+template <int G, int M>
+__device__ __forceinline__ void return_coefficients(Seg& c, Lane<G, M>& L, const InstDev& I,
+                                                    const double (&pop)[Comps<M>::N])
 {
     double c_icr, c_d;
-    const double kappa = force_of_infection<G>(c, L, pop, I.c_tdep, season_at<G>(L, I.c_tdep), c_icr, c_d);
+    const double kappa = force_of_infection(c, L, pop, I.c_tdep, season_at(L, I.c_tdep), c_icr, c_d);
     const size_t lane  = size_t(L.node) * G + L.age;
     c.kap[lane]        = kappa;
     if (c.kicu) {
@@ -673,8 +799,8 @@ __device__ __forceinline__ double damped(double b, double m, double D)
 // commuter nondetection factor), and the node's state without all its travelers. Every out-edge takes the same
 // row times its coefficient, so the sum over the out-edges is the row times the sum of the coefficients (a
 // constant of the graph): no walk over the out-edges.
-template <int G>
-__device__ __forceinline__ void leave(Seg& c, const Lane<G>& L, InstDev& I, double fac, double nd, double D,
+template <int G, int M>
+__device__ __forceinline__ void leave(Seg& c, const Lane<G, M>& L, InstDev& I, double fac, double nd, double D,
                                       double (&y)[NC])
 {
 #pragma clang fp contract(off)
@@ -687,7 +813,7 @@ __device__ __forceinline__ void leave(Seg& c, const Lane<G>& L, InstDev& I, doub
     }
     row[ISY] = row[ISY] * fac;
     double gone[NC];
-    const int v = L.np.local;
+    const int v = c.nodep[L.node].local;
     if (es.out_sum) {
         double sum = es.out_sum[v];
         if (D != 0.0) {
@@ -738,8 +864,8 @@ __device__ __forceinline__ void leave(Seg& c, const Lane<G>& L, InstDev& I, doub
 // ending at the active NPI's end). Every lane of the node reaches the same decision; the first lane of the
 // group implements the NPI on the node's damping list and cache (mgo_npi.h). Returns true in `changed`
 // when the contact matrix changed.
-template <int G>
-__device__ double npi_piece(Seg& c, Lane<G>& L, InstDev& I, const double (&y)[NC], double t, double tmax,
+template <int G, int M>
+__device__ double npi_piece(Seg& c, Lane<G, M>& L, InstDev& I, const double (&y)[NC], double t, double tmax,
                             bool& changed)
 {
     NpiNode* nn         = c.npi + L.node;
@@ -796,7 +922,9 @@ __device__ double npi_piece(Seg& c, Lane<G>& L, InstDev& I, const double (&y)[NC
     }
     if (changed) {
         __threadfence(); // the group's other lanes read the new cache written by its first lane
-        L.np.damp_cnt = __shfl(*static_cast<volatile int32_t*>(&nn->cache_count), L.base);
+        L.damp_cnt = __shfl(*static_cast<volatile int32_t*>(&nn->cache_count), L.base);
+        L.row_lo   = INFINITY; // the kept contact row is of the old cache
+        L.row_hi   = -INFINITY;
     }
     double dt_eff = (tmax - t < 1.0) ? tmax - t : 1.0;
     if (t < t_end) {
@@ -809,8 +937,8 @@ __device__ double npi_piece(Seg& c, Lane<G>& L, InstDev& I, const double (&y)[NC
 // metapopulation_mobility_instant.h:549-566): the edge NPI check on the node's last state (no delay, no
 // directive; begin t, end t + duration, per-group mobility dampings), then on a departure the damping factor
 // D of the lane's age group at t (Dampings::get_matrix_at, damping.h:381-396) for the edge kernels.
-template <int G>
-__device__ double out_damping(Seg& c, Lane<G>& L, InstDev& I, const double (&y)[NC])
+template <int G, int M>
+__device__ double out_damping(Seg& c, Lane<G, M>& L, InstDev& I, const double (&y)[NC])
 {
     NpiNode* od    = c.out_npi + L.node;
     const double t = I.c_t1;
@@ -871,7 +999,7 @@ __device__ double out_damping(Seg& c, Lane<G>& L, InstDev& I, const double (&y)[
             d = Dr;
         }
         else {
-            d = 0.5 * (Dl - Dr) * cos(MGO_PI / (xr - xl) * (t - xl)) + 0.5 * (Dl + Dr);
+            d = fma(0.5 * (Dl - Dr), cospi((t - xl) / (xr - xl)), 0.5 * (Dl + Dr));
         }
         c.out_d[size_t(L.node) * G + L.age] = d;
         return d;
@@ -883,82 +1011,118 @@ __device__ double out_damping(Seg& c, Lane<G>& L, InstDev& I, const double (&y)[
 // SystemIntegrator::advance (integrator.h:184-249) of every node to the cycle's end time with the
 // integrator core K: odeint Cash-Karp controller (stepper_wrapper.h:112-163), RKIntegratorCore
 // (adapt_rk.h:217-298), fixed Cash-Karp (stepper_wrapper.h:240-255) or Euler (euler.h:54-62).
-// Loop is flattened to one try_step attempt per iteration so that a rejected node only idles through
-// the k1 evaluation of its neighbours in the wavefront.
+// Loop is flattened to one try_step attempt per iteration so that a rejected node stays in step with its
+// neighbours in the wavefront.
+//
+// Bound by the FP64 issue rate and, with few wavefronts, by the chain of dependent operations of one attempt (six
+// right-hand sides with an LDS exchange each). The plain instantiation fits 256 registers without scratch, two
+// wavefronts per SIMD: eight compartments, no feature code (the arguments of sin, cos and pow alone took a third
+// of 107 KB of code, above the 64 KB instruction cache; 15 KB now), the scalars of a step in LDS (Cold). 512 runs x
+// 400 nodes x 6 groups at 1e-10: 580 us per half-day against 1030 us for ten compartments at one wavefront per
+// SIMD; a single 400-node graph 39 us against 50 us. Two wavefronts with the cold scalars in registers spilled 25
+// values per attempt: 768 us and 51 us.
 constexpr uint32_t kMaxAttemptsPerPhase = 1u << 20;
 
-template <int G, int K, bool NPI = false>
+template <int G, int K, int M>
 __device__ __forceinline__ void node_body(const LaunchDev& ld, InstDev* __restrict__ inst, double* wx)
 {
-    Lane<G> L;
-    Seg* cp = load_lane<G>(ld, L, wx);
+    using X         = Comps<M>;
+    constexpr int N = X::N;
+    Lane<G, M> L;
+    Seg* cp = load_lane(ld, L, wx);
     if (!cp) {
         return;
     }
-    Seg& c = *cp;
-    InstDev& I = inst[L.np.inst];
+    Seg& c     = *cp;
+    InstDev& I = inst[L.inst];
     if (!I.c_active) {
         return;
     }
     double* yp = c.y + (size_t(L.node) * G + L.age) * NC;
-    double y[NC];
+    double y[N];
+    {
+        const double2* y2 = reinterpret_cast<const double2*>(yp);
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        y[i] = yp[i];
+        for (int q = 0; q < NC / 2; ++q) {
+            const double2 v = y2[q];
+            if (X::of(2 * q) >= 0) {
+                y[X::of(2 * q)] = v.x;
+            }
+            if (X::of(2 * q + 1) >= 0) {
+                y[X::of(2 * q + 1)] = v.y;
+            }
+        }
     }
     double t            = c.tnode[L.node];
     double dt           = c.dtnode[L.node];
     const double t_phase = I.c_t1;
     // Without dynamic NPIs the phase is one SystemIntegrator::advance to c_t1; with them it is the pieces of
     // osecir::Simulation::advance (at most a day each, ending at NPI ends), each starting with the NPI check
-    const bool npi      = NPI && (L.np.flags & NF_NPI) != 0; // NPI: instantiation for classes with NPIs
+    const bool npi      = M == NPIS && (L.flags & NF_NPI) != 0;
     double t_loop       = t; // osecir::Simulation::advance's loop time (model.h:301)
-    double tmax         = t_phase;
-    double t0           = t;
-    const double dt_max = I.dt_max;
-    double dt_min       = I.dt_min;
-    double dt_restore   = 0.0;
-    const double eps    = 1e-12;
+    auto cold           = [&](Cold k) -> double& {
+        return L.cold[k * BLOCK];
+    };
+    auto cold_int = [&](Cold k) {
+        return reinterpret_cast<int32_t*>(&L.cold[k * BLOCK]);
+    };
+    cold(COLD_ABS)        = I.abs_tol;
+    cold(COLD_REL)        = I.rel_tol;
+    cold(COLD_DT_MAX)     = I.dt_max;
+    cold(COLD_DT_MIN)     = I.dt_min;
+    cold(COLD_DT_RESTORE) = 0.0;
+    cold(COLD_TMAX)       = t_phase;
+    // season of the next k1: an accepted step ends at t + h, where its fifth stage (c5 = 1 in both tableaus)
+    // evaluated the season already
+    cold(COLD_SEASON) = season_at(L, t);
     // output days strictly inside this phase are interpolated here; a day at the phase end is written
     // after the edge action
     // (the first is the day after the node's own time: a fixed-step node can end a phase just below the day
     // the phase ended on, and then its first step here encloses that day)
-    const int ndays  = I.ndays;
-    int next_day     = max(0, int(floor(t)) + 1 - I.day0);
-    const double tde = I.c_t1 - 1e-10;
+    cold_int(COLD_DAYS)[0]   = max(0, int(floor(t)) + 1 - I.day0);
+    cold_int(COLD_DAYS)[1]   = I.ndays;
+    cold_int(COLD_COUNTS)[0] = 0;
+    cold_int(COLD_COUNTS)[1] = 0;
+    const double eps = 1e-12;
 
-    bool active  = false;
-    bool need_k1 = true;
-    // season of the next k1: an accepted step ends at t + h, where its fifth stage evaluated the season already
-    bool have_season   = false;
-    double season_next = 0.0, season_end = 0.0;
-    bool fail = true, valid = true, first = true, stalled = false;
-    uint32_t nsteps = 0, natt = 0;
-    double k1[NC];
+    bool active = false;
+    bool fresh  = true; // the next attempt begins a step
+    bool valid = true, first = true, stalled = false;
+    double k1[N];
     for (;;) { // pieces of the node advance (one without dynamic NPIs)
         bool changed = false;
-        if (npi) {
-            tmax = t_loop + npi_piece<G>(c, L, I, y, t_loop, t_phase, changed);
+        if constexpr (M == NPIS) {
+            if (npi) {
+                cold(COLD_TMAX) = t_loop + npi_piece(c, L, I, y, t_loop, t_phase, changed);
+            }
         }
         if (I.c_action == 2 && (first || changed)) {
             // return coefficients of this node as a destination: its state after the departures, at the
             // departure time (the `pop` of calculate_mobility_returns, metapopulation_mobility_instant.h:460-471),
             // with the contact matrix as it is after the node's NPI checks of this phase
-            double pop[NC];
+            if constexpr (M == NPIS) {
+                double pop[N];
 #pragma unroll
-            for (int i = 0; i < NC; ++i) {
-                pop[i] = first ? y[i] : c.npi[L.node].y0[L.age * NC + i];
-                if (first && npi) {
-                    c.npi[L.node].y0[L.age * NC + i] = y[i];
+                for (int i = 0; i < N; ++i) {
+                    pop[i] = first ? y[i] : c.npi[L.node].y0[L.age * NC + i];
+                    if (first && npi) {
+                        c.npi[L.node].y0[L.age * NC + i] = y[i];
+                    }
                 }
+                return_coefficients(c, L, I, pop);
             }
-            return_coefficients<G>(c, L, I, pop);
+            else {
+                return_coefficients(c, L, I, y);
+            }
         }
-        first  = false;
-        t0     = t;
-        active = fabs((tmax - t) / (tmax - t0)) > eps;
+        first           = false;
+        cold(COLD_SPAN) = cold(COLD_TMAX) - t;
+        active          = fabs((cold(COLD_TMAX) - t) / cold(COLD_SPAN)) > eps;
+        fresh           = true;
+        rhs(c, L, y, t, cold(COLD_SEASON), k1);
         while (active) {
-            if (natt >= kMaxAttemptsPerPhase) {
+            int32_t* counts = cold_int(COLD_COUNTS);
+            if (uint32_t(counts[1]) >= kMaxAttemptsPerPhase) {
                 // a step size driven below any progress (dt_min ~ DBL_MIN with a persistent error): stop this
                 // node and report instead of spinning; the reference would not terminate here
                 if (L.age == 0) {
@@ -967,144 +1131,151 @@ __device__ __forceinline__ void node_body(const LaunchDev& ld, InstDev* __restri
                 stalled = true;
                 break;
             }
-            if (need_k1) {
-                if (dt > tmax - t) {
-                    dt_restore = dt;
-                    dt         = tmax - t;
-                    dt_min     = fmin(tmax - t, dt_min);
+            if (fresh) {
+                const double left = cold(COLD_TMAX) - t;
+                if (dt > left) {
+                    cold(COLD_DT_RESTORE) = dt;
+                    dt                    = left;
+                    cold(COLD_DT_MIN)     = fmin(left, cold(COLD_DT_MIN));
                 }
-                rhs<G>(c, L, y, t, have_season ? season_next : season_at<G>(L, t), k1);
-                have_season = false;
-                need_k1 = false;
-                fail    = true;
-                valid   = true;
+                fresh = false;
+                valid = true;
                 if (K == MGO_INTEGRATOR_RKF45) {
-                    dt = fmin(dt, dt_max);
+                    dt = fmin(dt, cold(COLD_DT_MAX));
                 }
             }
-            double yo[NC], er[NC];
-            bool done       = false;
+            double yo[N], er[N];
+            bool done       = true;
             const double ta = t;
-            ++natt;
+            // scale of the next step size is factor (clamped below by factor_min), or 1
+            double base = 1.0, power = 0.0, factor_min = 0.0;
+            bool scale = false;
+            ++counts[1];
             if (K == MGO_INTEGRATOR_CASH_KARP54) {
-                if (dt < dt_min) {
+                if (dt < cold(COLD_DT_MIN)) {
                     valid = false;
-                    dt    = dt_min;
+                    dt    = cold(COLD_DT_MIN);
                 }
-                if (!(dt - dt_max <= DBL_EPSILON)) {
-                    dt   = dt_max; // check_step_size_limit: rejected without a step
-                    fail = true;
+                if (!(dt - cold(COLD_DT_MAX) <= DBL_EPSILON)) {
+                    dt = cold(COLD_DT_MAX); // check_step_size_limit: rejected without a step
+                    continue;
                 }
-                else {
-                    cash_karp_stages<G>(c, L, y, k1, t, dt, yo, er, true, season_end);
-                    // max_i |err_i| / (abs + rel (|y_i| + dt |k1_i|)) (odeint default_error_checker): the index of
-                    // the largest quotient by cross-multiplied comparison, then one division
-                    double en = 0.0, ed = 1.0;
+                cash_karp_stages(c, L, y, k1, t, dt, yo, er, true);
+                // max_i |err_i| / (abs + rel (|y_i| + dt |k1_i|)) (odeint default_error_checker): the index of
+                // the largest quotient by cross-multiplied comparison, then one division
+                double en = 0.0, ed = 1.0;
+                const double abs_tol = cold(COLD_ABS), rel_tol = cold(COLD_REL);
 #pragma unroll
-                    for (int i = 0; i < NC; ++i) {
-                        const double n = fabs(er[i]);
-                        const double d = I.abs_tol + I.rel_tol * (fabs(y[i]) + dt * fabs(k1[i]));
-                        if (n * ed > en * d) {
-                            en = n;
-                            ed = d;
-                        }
-                    }
-                    double e = en / ed;
-                    // maximum over the node's lanes through the wavefront's slots (the same fmax order)
-                    L.wx[threadIdx.x % WAVE] = e;
-                    __builtin_amdgcn_wave_barrier();
-                    e = L.wx[L.base];
-#pragma unroll
-                    for (int j = 1; j < G; ++j) {
-                        e = fmax(e, L.wx[L.base + j]);
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                    if (e > 1.0) {
-                        dt *= fmax(0.9 * step_pow(e, -1.0 / 3.0), 0.2);
-                        dt   = fmin(dt, dt_max);
-                        fail = true;
-                    }
-                    else {
-                        t += dt;
-                        have_season = true;
-                        season_next = season_end;
-                        if (e < 0.5) {
-                            e = fmax(1.0 / 3125.0, e);
-                            dt *= 0.9 * step_pow(e, -0.2);
-                            dt = fmin(dt, dt_max);
-                        }
-                        fail = false;
+                for (int i = 0; i < N; ++i) {
+                    const double n = fabs(er[i]);
+                    const double d = fma(rel_tol, fma(dt, fabs(k1[i]), fabs(y[i])), abs_tol);
+                    if (n * ed > en * d) {
+                        en = n;
+                        ed = d;
                     }
                 }
-                done = !(fail && valid);
-                if (done) {
-                    dt = fmax(dt, dt_min);
-                    if (fail) {
-                        t += dt_min;
-                    }
+                double e = en / ed;
+                // maximum over the node's lanes through the wavefront's slots (the same fmax order)
+                L.wx[threadIdx.x % WAVE] = e;
+                wave_sync();
+                e = L.wx[L.base];
+#pragma unroll
+                for (int j = 1; j < G; ++j) {
+                    e = fmax(e, L.wx[L.base + j]);
+                }
+                wave_sync();
+                // rejected: dt *= max(0.9 e^(-1/3), 0.2); accepted below 0.5: dt *= 0.9 max(5^-5, e)^(-1/5)
+                const bool rejected = e > 1.0;
+                base                = rejected ? e : fmax(1.0 / 3125.0, e);
+                power               = rejected ? -1.0 / 3.0 : -0.2;
+                factor_min          = rejected ? 0.2 : 0.0;
+                scale               = rejected || e < 0.5;
+                done                = !(rejected && valid);
+                if (!rejected) {
+                    t += dt;
+                    cold(COLD_SEASON) = stage_season<3>(L);
+                }
+                else if (done) {
+                    t += cold(COLD_DT_MIN);
+                    cold(COLD_SEASON) = season_at(L, t);
                 }
             }
             else if (K == MGO_INTEGRATOR_RKF45) {
-                if (dt < dt_min) {
+                if (dt < cold(COLD_DT_MIN)) {
                     valid = false;
-                    dt    = dt_min;
+                    dt    = cold(COLD_DT_MIN);
                 }
-                rkf45_stages<G>(c, L, y, k1, t, dt, yo, er, season_end);
+                rkf45_stages(c, L, y, k1, t, dt, yo, er);
+                const double abs_tol = cold(COLD_ABS), rel_tol = cold(COLD_REL);
                 bool conv = true;
                 double q  = INFINITY;
 #pragma unroll
-                for (int i = 0; i < NC; ++i) {
-                    const double ep = I.abs_tol + fabs(yo[i]) * I.rel_tol;
+                for (int i = 0; i < N; ++i) {
+                    const double ep = fma(fabs(yo[i]), rel_tol, abs_tol);
                     conv            = conv && (er[i] <= ep);
                     q               = fmin(q, ep / er[i]);
                 }
-                conv = group_all<G>(conv, L.base);
-                q    = group_min<G>(q, L.base);
-                if (conv || !valid) {
-                    t += dt;
-                    have_season = true;
-                    season_next = season_end;
-                }
-                double dt_new = dt * step_pow(q, 1.0 / 5.0);
-                dt_new *= 0.9;
-                dt   = fmin(dt_new, dt_max);
-                done = conv || !valid;
+                conv  = group_all<G>(conv, L.base);
+                base  = group_min<G>(q, L.base);
+                power = 1.0 / 5.0;
+                scale = true;
+                done  = conv || !valid;
                 if (done) {
-                    dt = fmax(dt, dt_min);
+                    t += dt;
+                    cold(COLD_SEASON) = stage_season<3>(L);
                 }
             }
             else if (K == MGO_INTEGRATOR_CASH_KARP54_FIXED) {
-                cash_karp_stages<G>(c, L, y, k1, t, dt, yo, er, false, season_end);
+                cash_karp_stages(c, L, y, k1, t, dt, yo, er, false);
                 t += dt;
-                have_season = true;
-                season_next = season_end;
-                done = true;
+                cold(COLD_SEASON) = stage_season<3>(L);
             }
             else { // Euler
 #pragma unroll
-                for (int i = 0; i < NC; ++i) {
-                    yo[i] = y[i] + dt * k1[i];
+                for (int i = 0; i < N; ++i) {
+                    yo[i] = fma(dt, k1[i], y[i]);
                 }
                 t += dt;
-                done = true;
+                cold(COLD_SEASON) = season_at(L, t);
+            }
+            // k1 of the next attempt, before its step size is known: independent of the power below, whose chain of
+            // dependent operations it overlaps (after a rejection it is the same k1 again)
+            double yn[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                yn[i] = done ? yo[i] : y[i];
+            }
+            rhs(c, L, yn, t, cold(COLD_SEASON), k1);
+            if (K == MGO_INTEGRATOR_CASH_KARP54 || K == MGO_INTEGRATOR_RKF45) {
+                const double factor = 0.9 * step_pow(base, power);
+                const double scaled = fmin(dt * fmax(factor, factor_min), cold(COLD_DT_MAX));
+                dt                  = scale ? scaled : dt;
+                if (done) {
+                    dt = fmax(dt, cold(COLD_DT_MIN));
+                }
             }
             if (done) {
-                ++nsteps;
+                ++counts[0];
                 // interpolate_simulation_result (analyze_result.h:235-252): days in (ta, t] strictly inside
                 // the phase
-                while (next_day < ndays && double(next_day + I.day0) <= t && double(next_day + I.day0) < tde) {
-                    const double dd = double(next_day + I.day0);
+                int32_t* days = cold_int(COLD_DAYS);
+                while (days[0] < days[1]) {
+                    const double dd = double(days[0] + I.day0);
+                    if (!(dd <= t && dd < I.c_t1 - 1e-10)) {
+                        break;
+                    }
                     if (dd > ta) {
                         const double w = (dd - ta) / (t - ta);
-                        gdouble* op     = out_ptr(I, L.np.local, L.age, G, next_day);
+                        gdouble* op    = out_ptr(I, c.nodep[L.node].local, L.age, G, days[0]);
 #pragma unroll
                         for (int i = 0; i < NC; ++i) {
-                            op[i] = lerp_ref(y[i], yo[i], w);
+                            const int x = X::of(i);
+                            op[i]       = x < 0 ? 0.0 : lerp_ref(y[x < 0 ? 0 : x], yo[x < 0 ? 0 : x], w);
                         }
                     }
-                    ++next_day;
+                    ++days[0];
                 }
-                active = fabs((tmax - t) / (tmax - t0)) > eps;
+                active = fabs((cold(COLD_TMAX) - t) / cold(COLD_SPAN)) > eps;
                 if (!active && I.c_out_day >= 0) {
                     // the last step of the phase (so far): the phase-end day is interpolated from it after the
                     // edge action (write_phase_end_day)
@@ -1112,56 +1283,62 @@ __device__ __forceinline__ void node_body(const LaunchDev& ld, InstDev* __restri
                     double* pr      = c.yint + (size_t(L.node) * G + L.age) * YINT_STRIDE;
 #pragma unroll
                     for (int i = 0; i < NC; ++i) {
-                        pr[i] = y[i];
+                        pr[i] = X::of(i) < 0 ? 0.0 : y[X::of(i) < 0 ? 0 : X::of(i)];
                     }
                     pr[YINT_W] = (t >= dd) ? (dd - ta) / (t - ta) : -1.0;
                 }
 #pragma unroll
-                for (int i = 0; i < NC; ++i) {
+                for (int i = 0; i < N; ++i) {
                     y[i] = yo[i];
                 }
-                need_k1 = true;
+                fresh = true;
             }
         }
         if (!npi || stalled) {
             break;
         }
         // end of a piece: SystemIntegrator::advance's exit (integrator.h:244-248), then the next piece
-        dt         = fmax(dt, dt_restore);
-        dt_restore = 0.0;
-        dt_min     = I.dt_min;
-        t_loop     = tmax;
+        dt                    = fmax(dt, cold(COLD_DT_RESTORE));
+        cold(COLD_DT_RESTORE) = 0.0;
+        cold(COLD_DT_MIN)     = I.dt_min;
+        t_loop                = cold(COLD_TMAX);
         if (!(t_loop < t_phase)) {
             break;
         }
-        need_k1 = true;
     }
-    dt = fmax(dt, dt_restore);
+    dt = fmax(dt, cold(COLD_DT_RESTORE));
     if (L.age == 0) {
         c.tnode[L.node]  = t;
         c.dtnode[L.node] = dt;
-        c.steps[L.node] += nsteps;
-        c.attempts[L.node] += natt;
+        c.steps[L.node] += uint32_t(cold_int(COLD_COUNTS)[0]);
+        c.attempts[L.node] += uint32_t(cold_int(COLD_COUNTS)[1]);
+    }
+    double ye[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        ye[i] = X::of(i) < 0 ? 0.0 : y[X::of(i) < 0 ? 0 : X::of(i)];
     }
     double D = 0.0;
-    if (NPI && (L.np.flags & NF_OUT_DAMP) && I.c_action != 0) {
-        D = out_damping<G>(c, L, I, y);
+    if constexpr (M == NPIS) {
+        if ((L.flags & NF_OUT_DAMP) && I.c_action != 0) {
+            D = out_damping(c, L, I, ye);
+        }
     }
     if (I.c_action == 2) {
-        store_planes(c.ypre, size_t(c.num_nodes) * G, size_t(L.node) * G + L.age, y);
+        store_planes(c.ypre, size_t(c.num_nodes) * G, size_t(L.node) * G + L.age, ye);
         return; // the return phase writes the state and the day
     }
     if (I.c_action == 1) {
         // the departure phase adds the arrivals and writes the day
-        leave<G>(c, L, I, mobility_factor<G>(L, y),
-                 (L.np.flags & NF_DETECTION) ? detect_nondetection(L.np, I.c_t1) : 1.0, D, y);
+        const double nd = (M != PLAIN && (L.flags & NF_DETECTION)) ? detect_nondetection(c.nodep[L.node], t_phase) : 1.0;
+        leave(c, L, I, mobility_factor(L, ye[INS]), nd, D, ye);
     }
     else if (I.c_out_day >= 0) {
-        write_phase_end_day<G>(c, I, size_t(L.node) * G + L.age, L.np.local, L.age, y);
+        write_phase_end_day<G>(c, I, size_t(L.node) * G + L.age, c.nodep[L.node].local, L.age, ye);
     }
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
-        yp[i] = y[i];
+        yp[i] = ye[i];
     }
 }
 
@@ -2090,18 +2267,19 @@ __device__ __forceinline__ int block_groups(const LaunchDev& ld)
     default: break;                                                                                            \
     }
 
-template <int G, int K, bool NPI>
-__global__ void __launch_bounds__(BLOCK) node_phase(LaunchDev ld, InstDev* __restrict__ inst)
+// the plain kernel's registers are allocated for two wavefronts per SIMD
+template <int G, int K, int M>
+__global__ void __launch_bounds__(BLOCK, M == PLAIN ? 2 : 1) node_phase(LaunchDev ld, InstDev* __restrict__ inst)
 {
-    __shared__ double wx[BLOCK * (1 + (5 + G - 1) / G)]; // exchange slots, then the stage-season planes
-    node_body<G, K, NPI>(ld, inst, wx);
+    __shared__ double wx[node_lds<G>()];
+    node_body<G, K, M>(ld, inst, wx);
 }
 
-template <int K>
-__global__ void __launch_bounds__(BLOCK) node_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
+template <int K, int M>
+__global__ void __launch_bounds__(BLOCK, M == PLAIN ? 2 : 1) node_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
 {
-    __shared__ double wx[BLOCK * 6]; // exchange slots and up to five stage-season planes (G = 1)
-    MGO_DISPATCH_G(block_groups(ld), (node_body<GG, K>(ld, inst, wx)))
+    __shared__ double wx[node_lds<1>()]; // G = 1 has the most stage-season planes
+    MGO_DISPATCH_G(block_groups(ld), (node_body<GG, K, M>(ld, inst, wx)))
 }
 
 template <int G>
@@ -2173,11 +2351,14 @@ hipError_t launch_node_g(const LaunchDev& c, InstDev* inst, hipStream_t s)
 {
     const int nb = c.num_blocks;
 #define MGO_NODE_LAUNCH(KIND)                                                                                  \
-    if (c.npi) {                                                                                               \
-        hipLaunchKernelGGL((node_phase<G, KIND, true>), dim3(nb), dim3(BLOCK), 0, s, c, inst);                 \
+    if (c.mode == PLAIN) {                                                                                     \
+        hipLaunchKernelGGL((node_phase<G, KIND, PLAIN>), dim3(nb), dim3(BLOCK), 0, s, c, inst);                \
+    }                                                                                                          \
+    else if (c.mode == FEATURES) {                                                                             \
+        hipLaunchKernelGGL((node_phase<G, KIND, FEATURES>), dim3(nb), dim3(BLOCK), 0, s, c, inst);             \
     }                                                                                                          \
     else {                                                                                                     \
-        hipLaunchKernelGGL((node_phase<G, KIND, false>), dim3(nb), dim3(BLOCK), 0, s, c, inst);                \
+        hipLaunchKernelGGL((node_phase<G, KIND, NPIS>), dim3(nb), dim3(BLOCK), 0, s, c, inst);                 \
     }
     switch (c.kind) {
     case MGO_INTEGRATOR_CASH_KARP54:
@@ -2222,7 +2403,12 @@ hipError_t launch_weights_g(const LaunchDev& c, InstDev* inst, int inst_offset, 
 template <int K>
 hipError_t launch_node_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s)
 {
-    hipLaunchKernelGGL((node_phase_mixed<K>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+    if (c.mode == PLAIN) {
+        hipLaunchKernelGGL((node_phase_mixed<K, PLAIN>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+    }
+    else {
+        hipLaunchKernelGGL((node_phase_mixed<K, FEATURES>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+    }
     return hipGetLastError();
 }
 

@@ -1501,6 +1501,9 @@ __device__ __forceinline__ bool fixup_negative(const double (&y)[NC], double (&m
     return neg;
 }
 
+constexpr int DEPART_ROWS  = 4; // departure rows in flight per lane
+constexpr int RETURN_EDGES = 8; // forces of infection in flight per lane
+
 // Arrivals at c_t1 (metapopulation_mobility_instant.h:605-621): every edge (s, d) adds its source's departure
 // row times its coefficient to d. The lane sums its age group over the node's in-edges, in the reference's
 // order; the sum is kept for the returns (return_body).
@@ -1508,7 +1511,9 @@ __device__ __forceinline__ bool fixup_negative(const double (&y)[NC], double (&m
 // Bound by the gathered rows: 80 B per lane and edge, 4.9 GB per launch for 512 runs of a 400-node, 20k-edge
 // graph with 6 groups. The rows lie in planes of compartment pairs: a wavefront that holds one graph node of
 // several runs reads one contiguous kilobyte per pair, where rows of 96 B touched every line of the rows five
-// times. Measured there: 300 us (16 TB/s from the L2 caches) against 470 us for the walk over rows and out-edges.
+// times. Measured there: 300 us (16 TB/s from the L2 caches) against 470 us for the walk over rows and out-edges; one
+// run alone, bound by the gathers' latency: 25 us with the entries a batch ahead, 33 us without (6 or 8 rows in
+// flight are no faster).
 template <int G>
 __device__ __forceinline__ void depart_body(const LaunchDev& ld, InstDev* __restrict__ inst)
 {
@@ -1535,43 +1540,65 @@ __device__ __forceinline__ void depart_body(const LaunchDev& ld, InstDev* __rest
     const double2* dep    = c.dep;
     double M[NC] = {};
     if (es.out_sum) {
-        const int32_t* src = es.in_src;
-        const double* cf   = es.in_c;
-        const double* mn   = es.in_min;
-        constexpr int U    = 4; // rows in flight per lane
-        int k              = in_b;
-        auto rows          = [&](auto n) {
-            double2 r[decltype(n)::value][NC / 2];
-            double w[decltype(n)::value];
+        const double* mn = es.in_min;
+        constexpr int U  = DEPART_ROWS;
+        // U edges: their sources and coefficients (loaded a batch ahead), the rows, the sums in edge order
+        int32_t src[U];
+        double w[U];
+        auto entries = [&](int k) {
 #pragma unroll
-            for (int u = 0; u < decltype(n)::value; ++u) {
-                const size_t sl = src_base + size_t(src[k + u]) * src_step;
-                w[u]            = cf[k + u];
-                if (c.out_d) {
-                    const double D = c.out_d[sl];
-                    if (D != 0.0) {
-                        w[u] = damped(w[u], mn ? mn[k + u] : 0.0, D);
-                    }
-                }
+            for (int u = 0; u < U; ++u) {
+                const int ku = min(k + u, in_e - 1);
+                src[u]       = es.in_src[ku];
+                w[u]         = es.in_c[ku];
+            }
+        };
+        auto batch = [&](int k, auto full) {
+            double2 r[U][NC / 2];
+            double wk[U];
+            size_t sl[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) { // no branch between the loads
+                sl[u] = src_base + size_t(src[u]) * src_step;
+                wk[u] = w[u];
 #pragma unroll
                 for (int q = 0; q < NC / 2; ++q) {
-                    r[u][q] = dep[size_t(q) * np + sl];
+                    r[u][q] = dep[size_t(q) * np + sl[u]];
                 }
             }
+            if (c.out_d) {
 #pragma unroll
-            for (int u = 0; u < decltype(n)::value; ++u) {
+                for (int u = 0; u < U; ++u) {
+                    const double D = c.out_d[sl[u]];
+                    if (D != 0.0) {
+                        wk[u] = damped(wk[u], mn ? mn[min(k + u, in_e - 1)] : 0.0, D);
+                    }
+                }
+            }
+            if (decltype(full)::value) {
+                entries(k + U);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (!decltype(full)::value && k + u >= in_e) {
+                    continue;
+                }
 #pragma unroll
                 for (int q = 0; q < NC / 2; ++q) {
-                    M[2 * q]     = fma(w[u], r[u][q].x, M[2 * q]);
-                    M[2 * q + 1] = fma(w[u], r[u][q].y, M[2 * q + 1]);
+                    M[2 * q]     = fma(wk[u], r[u][q].x, M[2 * q]);
+                    M[2 * q + 1] = fma(wk[u], r[u][q].y, M[2 * q + 1]);
                 }
             }
         };
-        for (; k + U <= in_e; k += U) {
-            rows(std::integral_constant<int, U>{});
-        }
-        for (; k < in_e; ++k) {
-            rows(std::integral_constant<int, 1>{});
+        if (in_b < in_e) {
+            entries(in_b);
+            int k = in_b;
+            for (; k + U <= in_e; k += U) {
+                batch(k, std::true_type{});
+            }
+            if (k < in_e) {
+                batch(k, std::false_type{});
+            }
         }
     }
     else {
@@ -1759,7 +1786,8 @@ __device__ __forceinline__ void edge_return(const EdgeCoef& ec, const double (&r
 // out-edges of coefficient times rate: those of the constant rates are kept per lane (weights_body), the
 // force of infection (and, with ICU limits, two more) is summed here, 8 B per lane and edge instead of the
 // 2 x 96 B per lane and edge that a walk over all edges gathers. Measured (512 runs, 400 nodes, 20k edges, 6
-// groups): 350 us per launch against 1315 us for the walk.
+// groups): 304 us per launch against 1315 us for the walk (350 us, and 30 instead of 17 us for one run, with a
+// branch on the ICU limits between the loads, which then waited for each other).
 //
 // The fix-up acts where a compartment of a destination falls below zero while its in-edges are taken off one
 // by one. With nonnegative returning travelers every partial difference is at least the full one, ypre - arrivals
@@ -1801,20 +1829,45 @@ __device__ __forceinline__ void return_body(const LaunchDev& ld, InstDev* __rest
     double k0 = 0.0, k10 = 0.0, k12 = 0.0, k_min = 0.0;
     const int out_b = es.out_ptr[v], out_e = es.out_ptr[v + 1];
     if (es.out_sum) {
-#pragma unroll 4
-        for (int k = out_b; k < out_e; ++k) {
-            const size_t dl = src_base + size_t(es.out_dst[k]) * src_step;
-            double cf       = es.out_c[k];
-            if (D_v != 0.0) {
-                cf = damped(cf, es.out_min ? es.out_min[k] : 0.0, D_v);
+        // U edges at a time, their loads in flight together; the sums in edge order
+        constexpr int U = RETURN_EDGES;
+        for (int k = out_b; k < out_e; k += U) {
+            double cf[U], kd[U];
+            size_t dl[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int ku = min(k + u, out_e - 1);
+                dl[u]        = src_base + size_t(es.out_dst[ku]) * src_step;
+                cf[u]        = es.out_c[ku];
             }
-            const double kd = c.kap[dl];
-            k0              = fma(cf, kd, k0);
-            k_min           = fmin(k_min, kd);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                kd[u] = c.kap[dl[u]];
+            }
+            if (D_v != 0.0) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    cf[u] = damped(cf[u], es.out_min ? es.out_min[min(k + u, out_e - 1)] : 0.0, D_v);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const bool in = k + u < out_e;
+                k0            = in ? fma(cf[u], kd[u], k0) : k0;
+                k_min         = fmin(k_min, kd[u]); // the last edge again past the end
+            }
             if (icu) {
-                const double2 r = c.kicu[dl];
-                k10             = fma(cf, r.x, k10);
-                k12             = fma(cf, r.y, k12);
+                double2 ri[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    ri[u] = c.kicu[dl[u]];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const bool in = k + u < out_e;
+                    k10           = in ? fma(cf[u], ri[u].x, k10) : k10;
+                    k12           = in ? fma(cf[u], ri[u].y, k12) : k12;
+                }
             }
         }
     }

@@ -31,11 +31,11 @@
 
 namespace mgo
 {
-hipError_t launch_clock(InstDev* inst, int n, int32_t* cyc, hipStream_t s);
+hipError_t launch_clock(InstDev* inst, int n, hipStream_t s);
 hipError_t launch_scatter_slots(InstDev* table, const InstDev* src, const int32_t* ids, int n, hipStream_t s);
 hipError_t launch_set_segments(InstDev* table, const int32_t* ids, int n, hipStream_t s);
 hipError_t launch_node(const LaunchDev& c, InstDev* inst, hipStream_t s);
-hipError_t launch_edge(const LaunchDev& c, InstDev* inst, hipStream_t s);
+hipError_t launch_edge(const LaunchDev& c, InstDev* inst, bool clock, hipStream_t s);
 hipError_t launch_weights(const LaunchDev& c, InstDev* inst, int inst_offset, hipStream_t s);
 hipError_t launch_ensemble_mean(const double* out, const int64_t* base, int runs, int64_t positions, double* mean,
                                 hipStream_t s);
@@ -774,7 +774,14 @@ struct Batch {
     std::deque<ClassHost> classes;
     std::vector<InstHost> inst;
     DevBuf inst_dev;
-    DevBuf cyc; // [CYC_FLAGS] cycle flags (clock kernel, fixup_check), shared by the classes' launches
+    // Launches over several classes of one integrator kind and node mode (mixed G): one chain of launches per
+    // cycle for all of them, see merge_classes
+    struct Merged {
+        DevBuf segs, block_seg, block_first, inst_ids;
+        LaunchDev launch{};
+    };
+    std::deque<Merged> merged;
+    std::vector<const LaunchDev*> launches; // of a cycle: merged classes, the others per G
     int64_t cycles_run = 0;
     double last_ms     = 0;
     hipGraphExec_t graph_exec = nullptr;
@@ -785,6 +792,8 @@ struct Batch {
     size_t device_bytes       = 0;
     std::vector<InstDev> inst0; // instance table at creation (tmax set), for reset
     std::deque<std::vector<double>> staging; // host sources of uploads in flight during build
+    std::deque<std::vector<SegDev>> staging_segs;
+    std::deque<std::vector<int32_t>> staging_ints;
     // kernel timing of the last run (profile mode)
     double node_ms = 0, edge_ms = 0;
     int node_launches = 0, edge_launches = 0;
@@ -876,13 +885,12 @@ struct Batch {
             place_nodes(C, runs);
         }
         // sources of the asynchronous uploads below; they outlive the handler
-        const std::vector<int32_t> cyc_init(CYC_FLAGS, 0);
         std::vector<InstDev> idev(runs.size());
         try {
-            cyc.upload(cyc_init, stream);
             for (size_t ci = 0; ci < classes.size(); ++ci) {
                 build_class(ci, runs, idev);
             }
+            merge_classes(idev);
             inst_dev.upload(idev, stream);
             for (ClassHost& C : classes) {
                 if (C.wst.p) {
@@ -899,6 +907,8 @@ struct Batch {
         device_bytes += inst_dev.bytes;
         hip_check(hipStreamSynchronize(stream), "batch upload");
         staging.clear();
+        staging_segs.clear();
+        staging_ints.clear();
     }
 
     // Segment node indices of a class: runs that share a graph (same edge arrays and node count) are
@@ -1442,45 +1452,93 @@ struct Batch {
         ld.kind        = C.kind;
         ld.mode        = !(C.npi.nodes0.empty() && C.oute.nodes0.empty()) ? NPIS : features ? FEATURES : PLAIN;
         ld.general     = any_general ? 1 : 0;
-        ld.cyc         = cyc.as<int32_t>();
-    }
-
-    // launch tables of a cycle: one per class. (Batches keep per-G kernels so that a run's arithmetic is
-    // the same compiled code alone and in any batch; mixed tables serve the request loop.)
-    void launch_tables(std::vector<const LaunchDev*>& node_ld, std::vector<const LaunchDev*>& edge_ld) const
-    {
-        node_ld.clear();
-        edge_ld.clear();
-        for (const ClassHost& C : classes) {
-            node_ld.push_back(&C.launch);
-            bool any_edges = false;
-            for (int ii : C.insts) {
-                any_edges = any_edges || inst[size_t(ii)].has_edges;
-            }
-            if (any_edges) {
-                edge_ld.push_back(&C.launch);
-            }
+        ld.edges       = 0;
+        for (int ii : C.insts) {
+            ld.edges = ld.edges || inst[size_t(ii)].has_edges;
         }
     }
 
-    // enqueue one half-day cycle for every instance; with ev != nullptr, events bracket the node and the
-    // edge launches (ev[0..1] node, ev[2..3] edge)
+    // Launch tables of a cycle. Small classes that differ in G alone share one chain of launches whose blocks
+    // dispatch on their segment's G: a cycle of eight classes was bound by its 33 launches (240 us for 48 graphs of up
+    // to 1000 nodes; 8 concurrent streams included). The kernels' arithmetic is the same for a G in either (fused
+    // multiply-adds are written out), and segments are ordered by G so that neighbouring blocks run the same code.
+    // Uneven batches, shared chain against a stream per class: 237 blocks 58 / 107 ms, 1095 blocks 111 / 144 ms, 2479
+    // blocks 198 / 210 ms, 4842 blocks 332 / 316 ms, 9871 blocks 641 / 539 ms.
+    static constexpr int MERGE_BLOCKS = 3072;
+    void merge_classes(std::vector<InstDev>& idev)
+    {
+        std::map<std::pair<int, int>, std::vector<ClassHost*>> groups;
+        for (ClassHost& C : classes) {
+            groups[{C.launch.mode, C.kind}].push_back(&C);
+        }
+        for (auto& kv : groups) {
+            auto& group = kv.second;
+            int blocks  = 0;
+            for (ClassHost* C : group) {
+                blocks += segment_blocks(C->num_nodes, C->G);
+            }
+            // (the NPI checks are in the per-G kernels only)
+            if (group.size() < 2 || blocks > MERGE_BLOCKS || kv.first.first == NPIS) {
+                for (ClassHost* C : group) {
+                    launches.push_back(&C->launch);
+                }
+                continue;
+            }
+            std::sort(group.begin(), group.end(), [](const ClassHost* a, const ClassHost* b) {
+                return a->G < b->G;
+            });
+            merged.emplace_back();
+            Merged& m = merged.back();
+            m.launch  = group[0]->launch;
+            std::vector<SegDev> segs;
+            std::vector<int> nodes, gs;
+            std::vector<int32_t> ids, bseg, bfirst;
+            for (ClassHost* C : group) {
+                for (int ii : C->insts) {
+                    ids.push_back(ii);
+                    idev[size_t(ii)].seg = int32_t(segs.size());
+                }
+                segs.push_back(C->seg_host);
+                nodes.push_back(C->num_nodes);
+                gs.push_back(C->G);
+                m.launch.edges   = m.launch.edges || C->launch.edges;
+                m.launch.general = m.launch.general || C->launch.general;
+            }
+            block_tables_mixed(nodes, gs, bseg, bfirst);
+            auto up = [&](DevBuf& b, auto&& v, auto& keep) {
+                keep.push_back(std::move(v));
+                b.upload(keep.back(), stream);
+                device_bytes += b.bytes;
+            };
+            up(m.segs, std::move(segs), staging_segs);
+            up(m.block_seg, std::move(bseg), staging_ints);
+            up(m.block_first, std::move(bfirst), staging_ints);
+            m.launch.num_inst = int(ids.size());
+            up(m.inst_ids, std::move(ids), staging_ints);
+            m.launch.segs        = m.segs.as<SegDev>();
+            m.launch.block_seg   = m.block_seg.as<int32_t>();
+            m.launch.block_first = m.block_first.as<int32_t>();
+            m.launch.inst_ids    = m.inst_ids.as<int32_t>();
+            m.launch.num_blocks  = int(m.block_seg.bytes / sizeof(int32_t));
+            m.launch.G           = 0;
+            launches.push_back(&m.launch);
+        }
+    }
+
+    // enqueue one half-day cycle for every instance (its clock record is set: by the clock kernel at the start of a
+    // run, then by the previous cycle); with ev != nullptr, events bracket the node and the edge launches (ev[0..1]
+    // node, ev[2..3] edge)
     void enqueue_cycle(hipEvent_t* ev = nullptr)
     {
-        std::vector<const LaunchDev*> node_ld, edge_ld;
-        launch_tables(node_ld, edge_ld);
         InstDev* id = inst_dev.as<InstDev>();
-        hip_check(launch_clock(id, int(inst.size()), cyc.as<int32_t>(), stream), "clock kernel");
-        if (!ev && concurrent_classes && node_ld.size() > 1) {
-            // classes share no data: each runs its node and edge kernels on its own stream
-            make_side_streams(node_ld.size());
+        if (!ev && concurrent_classes && launches.size() > 1) {
+            // the launches share no data: each runs its node and edge kernels on its own stream
+            make_side_streams(launches.size());
             hip_check(hipEventRecord(fork_ev, stream), "fork");
-            for (size_t k = 0; k < node_ld.size(); ++k) {
+            for (size_t k = 0; k < launches.size(); ++k) {
                 hip_check(hipStreamWaitEvent(side[k], fork_ev, 0), "fork wait");
-                hip_check(launch_node(*node_ld[k], id, side[k]), "node kernel");
-                if (std::find(edge_ld.begin(), edge_ld.end(), node_ld[k]) != edge_ld.end()) {
-                    hip_check(launch_edge(*node_ld[k], id, side[k]), "edge kernel");
-                }
+                hip_check(launch_node(*launches[k], id, side[k]), "node kernel");
+                hip_check(launch_edge(*launches[k], id, true, side[k]), "edge kernel");
                 hip_check(hipEventRecord(side_done[k], side[k]), "join");
                 hip_check(hipStreamWaitEvent(stream, side_done[k], 0), "join wait");
             }
@@ -1489,15 +1547,15 @@ struct Batch {
         if (ev) {
             hip_check(hipEventRecord(ev[0], stream), "event");
         }
-        for (const LaunchDev* ld : node_ld) {
+        for (const LaunchDev* ld : launches) {
             hip_check(launch_node(*ld, id, stream), "node kernel");
         }
         if (ev) {
             hip_check(hipEventRecord(ev[1], stream), "event");
             hip_check(hipEventRecord(ev[2], stream), "event");
         }
-        for (const LaunchDev* ld : edge_ld) {
-            hip_check(launch_edge(*ld, id, stream), "edge kernel");
+        for (const LaunchDev* ld : launches) {
+            hip_check(launch_edge(*ld, id, true, stream), "edge kernel");
         }
         if (ev) {
             hip_check(hipEventRecord(ev[3], stream), "event");
@@ -1540,6 +1598,9 @@ struct Batch {
         std::vector<hipEvent_t> evs;
         node_ms = edge_ms = 0;
         node_launches = edge_launches = 0;
+        if (n > 0) {
+            hip_check(launch_clock(inst_dev.as<InstDev>(), int(inst.size()), stream), "clock kernel");
+        }
         if (n > 0 && profile) {
             evs.resize(size_t(4 * n));
             for (auto& e : evs) {
@@ -1583,10 +1644,10 @@ struct Batch {
             edge_ms += b;
         }
         if (!evs.empty()) {
-            std::vector<const LaunchDev*> node_ld, edge_ld;
-            launch_tables(node_ld, edge_ld);
-            node_launches = int(n) * int(node_ld.size());
-            edge_launches = int(n) * int(edge_ld.size());
+            node_launches = int(n) * int(launches.size());
+            for (const LaunchDev* ld : launches) {
+                edge_launches += ld->edges ? int(n) : 0;
+            }
         }
         for (auto& e : evs) {
             (void)hipEventDestroy(e);

@@ -157,7 +157,7 @@ struct InstDev {
     int32_t node_stride;  // segment index of local node v = node_base + v * node_stride (see Tiling)
     int32_t icu;          // some node has an ICU limit: the ISev rates of the returns depend on the state
     int32_t general;      // every return walks the edges: some edge coefficient or rate is negative, or a rate
-                          // exceeds 1 / dt_graph (see return_body)
+                          // exceeds 1 / dt_graph (see come_home)
     int32_t pad3;
 };
 static_assert(sizeof(InstDev) % 8 == 0, "instance records are copied as 8-byte words");
@@ -177,13 +177,6 @@ constexpr int FX_EPOCH_STEP = 16;   // > FX_MAX_PASSES
 
 constexpr int SETTLE_BLOCK  = 512;  // threads of an instance's block (eight walks at a time)
 constexpr int SETTLE_LIST   = 1024; // marked nodes an instance's block holds in LDS at a time
-
-// Cycle flags, written by the clock kernel (cleared, then set by the instances): which phases of this half-day
-// cycle have work anywhere in the batch, so that the launches of idle phases (the departure kernel in a return
-// cycle) exit at once.
-constexpr int CYC_DEPART = 0; // some instance departs
-constexpr int CYC_RETURN = 1; // some instance returns
-constexpr int CYC_FLAGS  = 2;
 
 // CSR edge structure of one graph (node indices local to the instance). In-edges of node v are sorted
 // by source; in_split[v] = number of in-edges whose source < v, so walking
@@ -287,7 +280,8 @@ struct LaunchDev {
     int32_t kind;
     int32_t mode;               // NodeMode of the class's node kernel
     int32_t general;            // some instance's returns walk the edges (InstDev::general)
-    int32_t* cyc;               // [CYC_FLAGS] cycle flags of the batch (or NULL: every phase runs its checks)
+    int32_t edges;              // some instance has edges
+    int32_t pad;
 };
 
 } // namespace mgo

@@ -7,17 +7,16 @@
 // contraction, so everything runs on the FP64 vector ALUs.
 //
 // Kernels per half-day cycle (GraphSimulation::advance, cpp/memilio/mobility/graph_simulation.h:101-120):
-//   clock_kernel       per instance: step size, edge action and output day of this cycle
 //   node_phase<G,K>    per node lane: SystemIntegrator::advance to t+dt with integrator K; writes the
 //                      departure row and takes the departing travelers off (departure cycles) or writes the
 //                      pre-return state and the return coefficients (return cycles)
-//   depart_phase<G>    per node lane: the arriving travelers, one sum over the node's in-edges in the
-//                      reference's edge order (deterministic, no atomics)
-//   return_phase<G>    per node lane: the returns in closed form; marks the nodes on which the negative-value
-//                      fix-up can act
+//   edge_phase<G>      per node lane: the arriving travelers, one sum over the node's in-edges in the
+//                      reference's edge order (deterministic, no atomics); or the returns in closed form,
+//                      marking the nodes on which the negative-value fix-up can act
 //   walk_phase<G>      per node lane of the instances whose returns need the edge walk (see InstDev::general)
 //   settle_phase<G>    per instance: marked nodes walk their edges with the fix-up, in passes over the nodes
-//                      whose inputs changed; sequential replay where these do not settle
+//                      whose inputs changed; sequential replay where these do not settle. Then the instance's
+//                      next cycle: step size, edge action and output day
 //
 // The file is compiled once per shard (MGO_SHARD, see memilio_amd/build.py), in parallel: shard 0 holds the
 // launch dispatch and the kernels without a G, shards 1..8 the kernels of that G, shards 9..12 the node kernel
@@ -682,25 +681,12 @@ __device__ __forceinline__ void clock_one(InstDev& I)
     }
 }
 
-// One block: the first threads clear the cycle flags, then every instance advances its clock and flags the
-// phases it needs (every writer stores 1).
-static __global__ void __launch_bounds__(1024) clock_kernel(InstDev* inst, int n, int32_t* cyc)
+// First clock of a run; later ones are advanced at the end of the settling kernel.
+static __global__ void __launch_bounds__(256) clock_kernel(InstDev* inst, int n)
 {
-    if (cyc) {
-        if (threadIdx.x < CYC_FLAGS) {
-            cyc[threadIdx.x] = 0;
-        }
-        __syncthreads();
-    }
-    for (int i = int(threadIdx.x); i < n; i += int(blockDim.x)) {
-        InstDev& I = inst[i];
-        clock_one(I);
-        if (cyc && I.c_action == 1) {
-            cyc[CYC_DEPART] = 1;
-        }
-        if (cyc && I.c_action == 2) {
-            cyc[CYC_RETURN] = 1;
-        }
+    const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i < n) {
+        clock_one(inst[i]);
     }
 }
 
@@ -1501,12 +1487,13 @@ __device__ __forceinline__ bool fixup_negative(const double (&y)[NC], double (&m
     return neg;
 }
 
+constexpr int EDGE_WAVES   = 3; // wavefronts per SIMD of the edge kernel
 constexpr int DEPART_ROWS  = 4; // departure rows in flight per lane
 constexpr int RETURN_EDGES = 8; // forces of infection in flight per lane
 
 // Arrivals at c_t1 (metapopulation_mobility_instant.h:605-621): every edge (s, d) adds its source's departure
 // row times its coefficient to d. The lane sums its age group over the node's in-edges, in the reference's
-// order; the sum is kept for the returns (return_body).
+// order; the sum is kept for the returns (come_home).
 //
 // Bound by the gathered rows: 80 B per lane and edge, 4.9 GB per launch for 512 runs of a 400-node, 20k-edge
 // graph with 6 groups. The rows lie in planes of compartment pairs: a wavefront that holds one graph node of
@@ -1515,21 +1502,8 @@ constexpr int RETURN_EDGES = 8; // forces of infection in flight per lane
 // run alone, bound by the gathers' latency: 25 us with the entries a batch ahead, 33 us without (6 or 8 rows in
 // flight are no faster).
 template <int G>
-__device__ __forceinline__ void depart_body(const LaunchDev& ld, InstDev* __restrict__ inst)
+__device__ __forceinline__ void arrive(Seg& c, InstDev& I, int node, int age)
 {
-    if (ld.cyc && !ld.cyc[CYC_DEPART]) {
-        return; // nobody departs in this cycle
-    }
-    int node, age, base;
-    Seg* cp = lane_map<G>(ld, node, age, base);
-    if (!cp) {
-        return;
-    }
-    Seg& c = *cp;
-    InstDev& I      = inst[c.nodep[node].inst];
-    if (!I.c_active || I.c_action != 1) {
-        return;
-    }
     Est& es = edge_struct(c, I.estruct);
     const int v             = c.nodep[node].local;
     const int in_b = es.in_ptr[v], in_e = es.in_ptr[v + 1];
@@ -1799,22 +1773,8 @@ __device__ __forceinline__ void edge_return(const EdgeCoef& ec, const double (&r
 // so all in-edges of a node change it in one direction and its extremes are at the ends of the sequence and at
 // the homecomings: ypre, ypre - arrivals and both with the homecomings added.
 template <int G>
-__device__ __forceinline__ void return_body(const LaunchDev& ld, InstDev* __restrict__ inst)
+__device__ __forceinline__ void come_home(Seg& c, InstDev& I, int node, int age, int base)
 {
-#pragma clang fp contract(off)
-    if (ld.cyc && !ld.cyc[CYC_RETURN]) {
-        return; // nobody returns in this cycle
-    }
-    int node, age, base;
-    Seg* cp = lane_map<G>(ld, node, age, base);
-    if (!cp) {
-        return;
-    }
-    Seg& c = *cp;
-    InstDev& I      = inst[c.nodep[node].inst];
-    if (!I.c_active || I.c_action != 2 || I.general) {
-        return;
-    }
     Est& es = edge_struct(c, I.estruct);
     const int v             = c.nodep[node].local;
     const size_t lane       = size_t(node) * G + age;
@@ -1918,6 +1878,29 @@ __device__ __forceinline__ void return_body(const LaunchDev& ld, InstDev* __rest
     }
     if (I.c_out_day >= 0) {
         write_phase_end_day<G>(c, I, lane, v, age, y);
+    }
+}
+
+// Edge action of the cycle: arrivals or returns, one launch for both (a cycle has one or the other, or some runs
+// each; an idle launch costs about 4.5 us).
+template <int G>
+__device__ __forceinline__ void edge_body(const LaunchDev& ld, InstDev* __restrict__ inst)
+{
+    int node, age, base;
+    Seg* cp = lane_map<G>(ld, node, age, base);
+    if (!cp) {
+        return;
+    }
+    Seg& c     = *cp;
+    InstDev& I = inst[c.nodep[node].inst];
+    if (!I.c_active) {
+        return;
+    }
+    if (I.c_action == 1) {
+        arrive<G>(c, I, node, age);
+    }
+    else if (I.c_action == 2 && !I.general) {
+        come_home<G>(c, I, node, age, base);
     }
 }
 
@@ -2135,9 +2118,6 @@ __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass,
 template <int G>
 __device__ __forceinline__ void walk_body(const LaunchDev& ld, InstDev* __restrict__ inst, double* buf)
 {
-    if (ld.cyc && !ld.cyc[CYC_RETURN]) {
-        return;
-    }
     const int lb = xcd_block();
     if (lb >= ld.num_blocks || ld.block_seg[lb] < 0) {
         return;
@@ -2238,11 +2218,8 @@ __device__ __forceinline__ void settle_body(const LaunchDev& ld, InstDev* __rest
 {
     constexpr int CAP = SETTLE_LIST; // marked nodes of one chunk
     InstDev& I        = inst[ld.inst_ids[blockIdx.x]];
-    if (!I.c_active || I.c_action != 2 || !I.fx_changed) {
-        return;
-    }
-    Seg& c = *segment(ld, I.seg);
-    const int wave  = int(threadIdx.x) / WAVE;
+    Seg& c            = *segment(ld, I.seg);
+    const int wave    = int(threadIdx.x) / WAVE;
     // list[CAP]: number of marked nodes, list[CAP + 1]: results of the pass's walks
     bool sequential = I.fx_sequential != 0 || I.fx_state == 2;
     int pass        = 1;
@@ -2336,9 +2313,9 @@ __global__ void __launch_bounds__(BLOCK, M == PLAIN ? 2 : 1) node_phase_mixed(La
 }
 
 template <int G>
-__global__ void __launch_bounds__(BLOCK) depart_phase(LaunchDev ld, InstDev* __restrict__ inst)
+__global__ void __launch_bounds__(BLOCK, EDGE_WAVES) edge_phase(LaunchDev ld, InstDev* __restrict__ inst)
 {
-    depart_body<G>(ld, inst);
+    edge_body<G>(ld, inst);
 }
 
 template <int G>
@@ -2348,35 +2325,42 @@ __global__ void __launch_bounds__(BLOCK) weights_phase(LaunchDev ld, InstDev* __
 }
 
 template <int G>
-__global__ void __launch_bounds__(BLOCK) return_phase(LaunchDev ld, InstDev* __restrict__ inst)
-{
-    return_body<G>(ld, inst);
-}
-
-template <int G>
 __global__ void __launch_bounds__(BLOCK) walk_phase(LaunchDev ld, InstDev* __restrict__ inst)
 {
     __shared__ double buf[BLOCK * NC];
     walk_body<G>(ld, inst, buf);
 }
 
+// Last kernel of a cycle: settles the fix-ups and, with clock, begins the run's next cycle (its other blocks read
+// only their own runs' records).
+__device__ __forceinline__ bool unsettled(const InstDev& I)
+{
+    return I.c_active && I.c_action == 2 && I.fx_changed;
+}
+
+__device__ __forceinline__ void next_cycle(const LaunchDev& ld, InstDev* __restrict__ inst, bool clock)
+{
+    __syncthreads(); // every thread is done with the cycle's record
+    if (clock && threadIdx.x == 0) {
+        clock_one(inst[ld.inst_ids[blockIdx.x]]);
+    }
+}
+
 template <int G>
-__global__ void __launch_bounds__(SETTLE_BLOCK) settle_phase(LaunchDev ld, InstDev* __restrict__ inst)
+__global__ void __launch_bounds__(SETTLE_BLOCK) settle_phase(LaunchDev ld, InstDev* __restrict__ inst, bool clock)
 {
     __shared__ int32_t list[SETTLE_LIST + 2];
     __shared__ double buf[SETTLE_BLOCK * NC];
-    settle_body<G>(ld, inst, list, buf);
+    if (unsettled(inst[ld.inst_ids[blockIdx.x]])) {
+        settle_body<G>(ld, inst, list, buf);
+    }
+    next_cycle(ld, inst, clock);
 }
 
 #if MGO_SHARD == 13
-__global__ void __launch_bounds__(BLOCK) depart_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
+__global__ void __launch_bounds__(BLOCK, EDGE_WAVES) edge_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
 {
-    MGO_DISPATCH_G(block_groups(ld), (depart_body<GG>(ld, inst)))
-}
-
-__global__ void __launch_bounds__(BLOCK) return_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
-{
-    MGO_DISPATCH_G(block_groups(ld), (return_body<GG>(ld, inst)))
+    MGO_DISPATCH_G(block_groups(ld), (edge_body<GG>(ld, inst)))
 }
 
 __global__ void __launch_bounds__(BLOCK) walk_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
@@ -2385,15 +2369,15 @@ __global__ void __launch_bounds__(BLOCK) walk_phase_mixed(LaunchDev ld, InstDev*
     MGO_DISPATCH_G(block_groups(ld), (walk_body<GG>(ld, inst, buf)))
 }
 
-__global__ void __launch_bounds__(SETTLE_BLOCK) settle_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
+__global__ void __launch_bounds__(SETTLE_BLOCK) settle_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst, bool clock)
 {
     __shared__ int32_t list[SETTLE_LIST + 2];
     __shared__ double buf[SETTLE_BLOCK * NC];
     const InstDev& I = inst[ld.inst_ids[blockIdx.x]];
-    if (!I.c_active || I.c_action != 2 || !I.fx_changed) {
-        return;
+    if (unsettled(I)) {
+        MGO_DISPATCH_G(ld.segs[I.seg].G, (settle_body<GG>(ld, inst, list, buf)))
     }
-    MGO_DISPATCH_G(ld.segs[I.seg].G, (settle_body<GG>(ld, inst, list, buf)))
+    next_cycle(ld, inst, clock);
 }
 #endif
 
@@ -2431,17 +2415,18 @@ hipError_t launch_node_g(const LaunchDev& c, InstDev* inst, hipStream_t s)
     return hipGetLastError();
 }
 
+// Edge phase and settling of one cycle; with clock, the runs' next cycle begins.
 template <int G>
-hipError_t launch_edge_g(const LaunchDev& c, InstDev* inst, hipStream_t s)
+hipError_t launch_edge_g(const LaunchDev& c, InstDev* inst, bool clock, hipStream_t s)
 {
-    const int nb = c.num_blocks;
-    hipLaunchKernelGGL((depart_phase<G>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
-    hipLaunchKernelGGL((return_phase<G>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
-    if (c.general) {
-        hipLaunchKernelGGL((walk_phase<G>), dim3(nb), dim3(BLOCK), 0, s, c, inst);
+    if (c.edges) {
+        hipLaunchKernelGGL((edge_phase<G>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        if (c.general) {
+            hipLaunchKernelGGL((walk_phase<G>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        }
     }
-    if (c.num_inst > 0) {
-        hipLaunchKernelGGL((settle_phase<G>), dim3(c.num_inst), dim3(SETTLE_BLOCK), 0, s, c, inst);
+    if (c.num_inst > 0 && (c.edges || clock)) {
+        hipLaunchKernelGGL((settle_phase<G>), dim3(c.num_inst), dim3(SETTLE_BLOCK), 0, s, c, inst, clock);
     }
     return hipGetLastError();
 }
@@ -2676,32 +2661,33 @@ hipError_t launch_ensemble_sort(const double* out, const int64_t* base, int runs
 }
 #endif
 
-hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s);
+hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, bool clock, hipStream_t s);
 
 #if MGO_SHARD >= 1 && MGO_SHARD <= 8
 template hipError_t launch_node_g<MGO_SHARD>(const LaunchDev&, InstDev*, hipStream_t);
-template hipError_t launch_edge_g<MGO_SHARD>(const LaunchDev&, InstDev*, hipStream_t);
+template hipError_t launch_edge_g<MGO_SHARD>(const LaunchDev&, InstDev*, bool, hipStream_t);
 template hipError_t launch_weights_g<MGO_SHARD>(const LaunchDev&, InstDev*, int, hipStream_t);
 #elif MGO_SHARD >= 9 && MGO_SHARD <= 12
 template hipError_t launch_node_mixed<MGO_SHARD - 9>(const LaunchDev&, InstDev*, hipStream_t);
 #elif MGO_SHARD == 13
-hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s)
+hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, bool clock, hipStream_t s)
 {
-    const int nb = c.num_blocks;
-    hipLaunchKernelGGL(depart_phase_mixed, dim3(nb), dim3(BLOCK), 0, s, c, inst);
-    hipLaunchKernelGGL(return_phase_mixed, dim3(nb), dim3(BLOCK), 0, s, c, inst);
-    if (c.general) {
-        hipLaunchKernelGGL(walk_phase_mixed, dim3(nb), dim3(BLOCK), 0, s, c, inst);
+    if (c.edges) {
+        hipLaunchKernelGGL(edge_phase_mixed, dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        if (c.general) {
+            hipLaunchKernelGGL(walk_phase_mixed, dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        }
     }
-    if (c.num_inst > 0) {
-        hipLaunchKernelGGL(settle_phase_mixed, dim3(c.num_inst), dim3(SETTLE_BLOCK), 0, s, c, inst);
+    if (c.num_inst > 0 && (c.edges || clock)) {
+        hipLaunchKernelGGL(settle_phase_mixed, dim3(c.num_inst), dim3(SETTLE_BLOCK), 0, s, c, inst, clock);
     }
     return hipGetLastError();
 }
+
 #elif MGO_SHARD == 0
 #define MGO_EXTERN_G(GG)                                                                                       \
     extern template hipError_t launch_node_g<GG>(const LaunchDev&, InstDev*, hipStream_t);                     \
-    extern template hipError_t launch_edge_g<GG>(const LaunchDev&, InstDev*, hipStream_t);                     \
+    extern template hipError_t launch_edge_g<GG>(const LaunchDev&, InstDev*, bool, hipStream_t);               \
     extern template hipError_t launch_weights_g<GG>(const LaunchDev&, InstDev*, int, hipStream_t);
 MGO_EXTERN_G(1)
 MGO_EXTERN_G(2)
@@ -2717,9 +2703,9 @@ extern template hipError_t launch_node_mixed<MGO_INTEGRATOR_RKF45>(const LaunchD
 extern template hipError_t launch_node_mixed<MGO_INTEGRATOR_CASH_KARP54_FIXED>(const LaunchDev&, InstDev*, hipStream_t);
 extern template hipError_t launch_node_mixed<MGO_INTEGRATOR_EULER>(const LaunchDev&, InstDev*, hipStream_t);
 
-hipError_t launch_clock(InstDev* inst, int n, int32_t* cyc, hipStream_t s)
+hipError_t launch_clock(InstDev* inst, int n, hipStream_t s)
 {
-    hipLaunchKernelGGL(clock_kernel, dim3(1), dim3(1024), 0, s, inst, n, cyc);
+    hipLaunchKernelGGL(clock_kernel, dim3(unsigned(n + 255) / 256), dim3(256), 0, s, inst, n);
     return hipGetLastError();
 }
 
@@ -2801,27 +2787,27 @@ hipError_t launch_node(const LaunchDev& c, InstDev* inst, hipStream_t s)
     }
 }
 
-hipError_t launch_edge(const LaunchDev& c, InstDev* inst, hipStream_t s)
+hipError_t launch_edge(const LaunchDev& c, InstDev* inst, bool clock, hipStream_t s)
 {
     switch (c.G) {
     case 0:
-        return launch_edge_mixed(c, inst, s);
+        return launch_edge_mixed(c, inst, clock, s);
     case 1:
-        return launch_edge_g<1>(c, inst, s);
+        return launch_edge_g<1>(c, inst, clock, s);
     case 2:
-        return launch_edge_g<2>(c, inst, s);
+        return launch_edge_g<2>(c, inst, clock, s);
     case 3:
-        return launch_edge_g<3>(c, inst, s);
+        return launch_edge_g<3>(c, inst, clock, s);
     case 4:
-        return launch_edge_g<4>(c, inst, s);
+        return launch_edge_g<4>(c, inst, clock, s);
     case 5:
-        return launch_edge_g<5>(c, inst, s);
+        return launch_edge_g<5>(c, inst, clock, s);
     case 6:
-        return launch_edge_g<6>(c, inst, s);
+        return launch_edge_g<6>(c, inst, clock, s);
     case 7:
-        return launch_edge_g<7>(c, inst, s);
+        return launch_edge_g<7>(c, inst, clock, s);
     case 8:
-        return launch_edge_g<8>(c, inst, s);
+        return launch_edge_g<8>(c, inst, clock, s);
     default:
         return hipErrorInvalidValue;
     }

@@ -1967,13 +1967,15 @@ __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass,
     const double D_v      = c.out_d ? c.out_d[own] : 0.0;
     double rates[NFLOW], y[NC], home[NC];
     // homecomings: sums over the out-edges, in 64 / G parts
-    double k0 = 0.0, k10 = 0.0, k12 = 0.0;
+    double k0 = 0.0, k10 = 0.0, k12 = 0.0, k_min = 0.0;
     if (act) {
         for (int k = out_b + grp; k < out_e; k += NPW) {
             const EdgeEnt e   = es.out_ent[k];
             const size_t dl   = src_base + size_t(e.nbr) * src_step;
             const EdgeCoef ec = edge_coef(es, e, es.out_min, k, D_v, G, age);
-            k0                = fma(coef_of(ec, S), c.kap[dl], k0);
+            const double kd   = c.kap[dl];
+            k0                = fma(coef_of(ec, S), kd, k0);
+            k_min             = fmin(k_min, kd);
             if (icu) {
                 const double2 r = c.kicu[dl];
                 k10             = fma(coef_of(ec, ISEV), r.x, k10);
@@ -2020,11 +2022,51 @@ __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass,
     }
     lane_rates(c, icu, own, rates);
     load_planes(c.ypre, np, own, y);
+    auto finish = [&]() {
+        if (grp == 0) {
+            double* yp = c.y + own * NC;
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                yp[i] = y[i];
+            }
+            if (I.c_out_day >= 0) {
+                write_phase_end_day<G>(c, I, own, v, age, y);
+            }
+        }
+    };
+    if (!I.general) {
+        // A node that walks because a homecoming changed (its travelers were fixed up elsewhere) is mostly done with
+        // the closed form of come_home and the new sum, if no fix-up of its own can act and none did so far.
+        double m[NC], dm[NC], y1[NC];
+        load_planes(c.arr, np, own, m);
+        euler_change(m, rates, h, dm);
+        bool full = I.fx_neg != 0 || !(rates[0] >= 0.0) || !(k_min >= 0.0);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            y1[i]            = y[i] - (m[i] + dm[i]);
+            const double low = fmin(home[i], 0.0);
+            full             = full || !(y1[i] >= 0.0) || !(y1[i] + low >= 0.0) || !(y[i] + low >= 0.0);
+        }
+        if (pass > 1) {
+            for (int k = in_b + lane; k < in_e; k += WAVE) {
+                full = full || record_slot(recs + 2 * k, lo, tag - 1) >= 0;
+            }
+        }
+        if (!__any(full)) {
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                y[i] = y1[i] + home[i];
+            }
+            finish();
+            return 0;
+        }
+    }
     int result    = 0;
     auto in_edges = [&](int first, int last) {
         for (int kb = first; kb < last; kb += NPW) {
             const int k = kb + grp;
             int32_t ps  = -1;
+            bool slow   = false; // negative travelers or a record among these edges
             if (act && k < last) {
                 const EdgeEnt e   = es.in_ent[k];
                 const size_t sl   = src_base + size_t(e.nbr) * src_step;
@@ -2035,13 +2077,40 @@ __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass,
 #pragma unroll
                 for (int i = 0; i < NC; ++i) {
                     buf[i * WAVE + lane] = m[i];
+                    slow                 = slow || !(m[i] >= 0.0);
                 }
                 if (pass > 0) {
-                    ps = record_slot(recs + 2 * k, lo, tag - 1);
+                    ps   = record_slot(recs + 2 * k, lo, tag - 1);
+                    slow = slow || ps >= 0;
                 }
             }
             wave_sync();
             const int n = min(NPW, last - kb);
+            // all of them at once, in order: with nonnegative travelers no compartment fell below zero on the way if
+            // none is below zero after them
+            double z[NC];
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                z[i] = y[i];
+            }
+            for (int j = 0; j < n; ++j) {
+#pragma unroll
+                for (int i = 0; i < NC; ++i) {
+                    z[i] -= buf[i * WAVE + j * G + age];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                slow = slow || !(z[i] >= 0.0);
+            }
+            if (!__any(slow)) {
+#pragma unroll
+                for (int i = 0; i < NC; ++i) {
+                    y[i] = z[i];
+                }
+                wave_sync();
+                continue;
+            }
             for (int j = 0; j < n; ++j) {
                 double m[NC];
 #pragma unroll
@@ -2101,16 +2170,7 @@ __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass,
         y[i] += home[i];
     }
     in_edges(in_s, in_e);
-    if (grp == 0) {
-        double* yp = c.y + own * NC;
-#pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            yp[i] = y[i];
-        }
-        if (I.c_out_day >= 0) {
-            write_phase_end_day<G>(c, I, own, v, age, y);
-        }
-    }
+    finish();
     return result;
 }
 

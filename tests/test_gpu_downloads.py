@@ -1,0 +1,31 @@
+"""Downloads in chunks by several threads: sizes around the size from which they are used (8 MiB) and around a chunk
+(1 MiB), every value in its place, bitwise (the mean of one run is the run itself)."""
+import numpy as np
+import pytest
+
+from memilio_amd import synthetic
+from memilio_amd.engine import Batch, Context
+
+pytestmark = pytest.mark.gpu
+MIB = 1 << 17   # doubles
+
+
+@pytest.mark.parametrize("n", [1, 8 * MIB - 1, 8 * MIB, 8 * MIB + 1, 9 * MIB - 1, 9 * MIB + 1, 30 * MIB + 12345])
+def test_large_results_arrive_whole(n):
+    v = np.random.default_rng(n).normal(size=(1, n))
+    with Context() as ctx:
+        for _ in range(2):
+            assert np.array_equal(ctx.ensemble_mean_values(v), v[0])
+
+
+def test_runs_of_different_size_arrive_in_place():
+    specs = [synthetic.graph(num_nodes=n, G=g, seed=n, mean_degree=3.0) for n, g in ((300, 6), (1, 1), (333, 8), (7, 2))]
+    cfgs, tmaxs = [synthetic.ck_cfg(1e-6)] * 4, [60.0, 31.0, 45.0, 30.0]
+    with Context() as ctx:
+        batch = Batch(ctx, specs, cfgs, tmaxs)
+        batch.run()
+        whole = batch.read_daily()
+        assert sum(x.nbytes for x in whole) > 8 << 20
+        for k in range(4):
+            assert np.array_equal(batch.read_daily(k, 1)[0], whole[k])
+        batch.close()

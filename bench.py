@@ -430,7 +430,7 @@ def main():
         "max_rel_err_vs_oracle": max_rel,
         "accuracy_ok": None if max_rel is None else bool(max_rel <= 1e-6),
         "roofline": {"bound": "fp64-valu", "roof": "FP64 vector ALU (78.6 TFLOP/s = FP64 peak of MI355X; no MFMA "
-                                                   "is used), latency-limited at one wavefront per SIMD",
+                                                   "is used), two wavefronts per SIMD",
                      "kernel": f"node_phase<G={G},CashKarp54>", "achieved": achieved, "peak": FP64_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": achieved / FP64_PEAK_TFLOPS, "traffic": traffic,
                      "traffic_source": traffic_src, "avg_launch_ms": node_ms, "launches": launches,

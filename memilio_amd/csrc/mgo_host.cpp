@@ -1200,7 +1200,7 @@ struct Batch {
                 for (int a = 0; a < G; ++a) {
                     double* lc = &lcoef[(node * G + size_t(a)) * NUM_LC];
                     lane_coefficients(g, v, a, lc);
-                    // closed-form returns need nonnegative travelers (see return_body)
+                    // closed-form returns need nonnegative travelers (see come_home)
                     for (int k = LC_E; k <= LC_ICR_R; ++k) {
                         general = general || !(lc[k] >= 0.0);
                     }

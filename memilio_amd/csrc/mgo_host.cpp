@@ -534,6 +534,7 @@ struct InstHost {
     int64_t out_base;
     bool has_edges;
     bool single;
+    int launch = 0; // index into Batch::launches
 };
 
 int day_floor(double t)
@@ -897,7 +898,7 @@ struct Batch {
         LaunchDev launch{};
     };
     std::deque<Merged> merged;
-    std::vector<const LaunchDev*> launches; // of a cycle: merged classes, the others per G
+    std::vector<LaunchDev*> launches; // of a cycle: merged classes, the others per G
     int64_t cycles_run = 0;
     double last_ms     = 0;
     hipGraphExec_t graph_exec = nullptr;
@@ -906,7 +907,8 @@ struct Batch {
     bool profile              = false;
     bool sequential_fixup     = false;
     size_t device_bytes       = 0;
-    std::vector<InstDev> inst0; // instance table at creation (tmax set), for reset
+    std::vector<InstDev> inst0;     // instance table at creation (tmax set), for reset
+    std::vector<InstDev> end_table; // instance table at the end of the last run
     std::deque<std::vector<double>> staging; // host sources of uploads in flight during build
     std::deque<std::vector<SegDev>> staging_segs;
     std::deque<std::vector<int32_t>> staging_ints;
@@ -1570,7 +1572,8 @@ struct Batch {
         ld.general     = any_general ? 1 : 0;
         ld.edges       = 0;
         for (int ii : C.insts) {
-            ld.edges = ld.edges || inst[size_t(ii)].has_edges;
+            ld.edges               = ld.edges || inst[size_t(ii)].has_edges;
+            idev[size_t(ii)].plain = ld.mode == PLAIN ? 1 : 0;
         }
     }
 
@@ -1596,6 +1599,9 @@ struct Batch {
             // (the NPI checks are in the per-G kernels only)
             if (group.size() < 2 || blocks > MERGE_BLOCKS || kv.first.first == NPIS) {
                 for (ClassHost* C : group) {
+                    for (int ii : C->insts) {
+                        inst[size_t(ii)].launch = int(launches.size());
+                    }
                     launches.push_back(&C->launch);
                 }
                 continue;
@@ -1612,7 +1618,8 @@ struct Batch {
             for (ClassHost* C : group) {
                 for (int ii : C->insts) {
                     ids.push_back(ii);
-                    idev[size_t(ii)].seg = int32_t(segs.size());
+                    idev[size_t(ii)].seg     = int32_t(segs.size());
+                    inst[size_t(ii)].launch = int(launches.size());
                 }
                 segs.push_back(C->seg_host);
                 nodes.push_back(C->num_nodes);
@@ -1683,30 +1690,112 @@ struct Batch {
     {
         int64_t mx = 0;
         for (size_t i = 0; i < inst.size(); ++i) {
-            const InstHost& I = inst[i];
-            double t          = I.t;
-            int64_t n         = 0;
-            while (t < I.tmax) {
-                double step = I.dt_graph;
-                if (t + step > I.tmax) {
-                    step = I.tmax - t;
-                }
-                t = (I.single && step != I.dt_graph) ? I.tmax : t + step;
-                ++n;
-            }
-            mx = std::max(mx, n);
+            double t = 0;
+            mx       = std::max(mx, cycles_to(inst[i].t, i, &t));
             if (t_after) {
                 t_after->push_back(t);
             }
         }
         return mx;
     }
+    // the same for one instance whose clock is at t
+    int64_t cycles_to(double t, size_t i, double* t_after) const
+    {
+        const InstHost& I = inst[i];
+        int64_t n         = 0;
+        while (t < I.tmax) {
+            double step = I.dt_graph;
+            if (t + step > I.tmax) {
+                step = I.tmax - t;
+            }
+            t = (I.single && step != I.dt_graph) ? I.tmax : t + step;
+            ++n;
+        }
+        if (t_after) {
+            *t_after = t;
+        }
+        return n;
+    }
+
+    // enqueue n cycles; with evs, four events per cycle bracket its node and edge launches
+    void enqueue_cycles(int64_t n, std::vector<hipEvent_t>* evs)
+    {
+        if (n <= 0) {
+            return;
+        }
+        hip_check(launch_clock(inst_dev.as<InstDev>(), int(inst.size()), stream), "clock kernel");
+        if (evs) {
+            const size_t first = evs->size();
+            evs->resize(first + size_t(4 * n));
+            for (size_t k = first; k < evs->size(); ++k) {
+                hip_check(hipEventCreate(&(*evs)[k]), "event");
+            }
+            for (int64_t k = 0; k < n; ++k) {
+                enqueue_cycle(&(*evs)[first + size_t(4 * k)]);
+            }
+        }
+        else if (use_graph) {
+            if (!graph_exec) {
+                hipGraph_t g;
+                hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "begin capture");
+                enqueue_cycle();
+                hip_check(hipStreamEndCapture(stream, &g), "end capture");
+                hip_check(hipGraphInstantiate(&graph_exec, g, nullptr, nullptr, 0), "graph instantiate");
+                (void)hipGraphDestroy(g);
+            }
+            for (int64_t k = 0; k < n; ++k) {
+                hip_check(hipGraphLaunch(graph_exec, stream), "graph launch");
+            }
+        }
+        else {
+            for (int64_t k = 0; k < n; ++k) {
+                enqueue_cycle();
+            }
+        }
+    }
+
+    // Instances that wait with confirmed cases (PLAIN_LOST): their launches change to the node kernel with all
+    // compartments. Returns the cycles that they have left. The device is idle; end_table is the instance table.
+    int64_t leave_plain()
+    {
+        std::vector<char> change(launches.size(), 0);
+        int64_t left = 0;
+        for (size_t i = 0; i < end_table.size(); ++i) {
+            const InstDev& D = end_table[i];
+            if (D.plain == PLAIN_LOST) {
+                change[size_t(inst[i].launch)] = 1;
+                left = std::max(left, D.status == MGO_OK ? cycles_to(D.t, i, nullptr) : 0);
+            }
+        }
+        const int32_t zero = 0;
+        bool any           = false;
+        for (size_t i = 0; i < inst.size(); ++i) {
+            if (!change[size_t(inst[i].launch)]) {
+                continue;
+            }
+            any                               = true;
+            launches[size_t(inst[i].launch)]->mode = FEATURES;
+            if (i < inst0.size()) {
+                inst0[i].plain = 0; // a reset run would come to the same
+            }
+            hip_check(hipMemcpyAsync(&inst_dev.as<InstDev>()[i].plain, &zero, sizeof(zero), hipMemcpyHostToDevice, stream),
+                      "node kernel change");
+        }
+        if (any) {
+            hip_check(hipStreamSynchronize(stream), "node kernel change");
+            if (graph_exec) {
+                (void)hipGraphExecDestroy(graph_exec);
+                graph_exec = nullptr;
+            }
+        }
+        return left;
+    }
 
     // advance every instance to its tmax (already set on host and device)
     void run(double* elapsed_ms)
     {
         std::vector<double> t_after;
-        const int64_t n = cycles_needed(&t_after);
+        int64_t n = cycles_needed(&t_after);
         hipEvent_t e0, e1;
         hip_check(hipEventCreate(&e0), "event");
         hip_check(hipEventCreate(&e1), "event");
@@ -1714,40 +1803,16 @@ struct Batch {
         std::vector<hipEvent_t> evs;
         node_ms = edge_ms = 0;
         node_launches = edge_launches = 0;
-        if (n > 0) {
-            hip_check(launch_clock(inst_dev.as<InstDev>(), int(inst.size()), stream), "clock kernel");
-        }
-        if (n > 0 && profile) {
-            evs.resize(size_t(4 * n));
-            for (auto& e : evs) {
-                hip_check(hipEventCreate(&e), "event");
-            }
-            for (int64_t k = 0; k < n; ++k) {
-                enqueue_cycle(&evs[size_t(4 * k)]);
+        for (int64_t more = n; ; n += more) {
+            enqueue_cycles(more, profile ? &evs : nullptr);
+            hip_check(hipEventRecord(e1, stream), "event record");
+            hip_check(hipEventSynchronize(e1), "run");
+            end_table = read_inst();
+            more      = leave_plain();
+            if (more == 0) {
+                break;
             }
         }
-        else if (n > 0) {
-            if (use_graph) {
-                if (!graph_exec) {
-                    hipGraph_t g;
-                    hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "begin capture");
-                    enqueue_cycle();
-                    hip_check(hipStreamEndCapture(stream, &g), "end capture");
-                    hip_check(hipGraphInstantiate(&graph_exec, g, nullptr, nullptr, 0), "graph instantiate");
-                    (void)hipGraphDestroy(g);
-                }
-                for (int64_t k = 0; k < n; ++k) {
-                    hip_check(hipGraphLaunch(graph_exec, stream), "graph launch");
-                }
-            }
-            else {
-                for (int64_t k = 0; k < n; ++k) {
-                    enqueue_cycle();
-                }
-            }
-        }
-        hip_check(hipEventRecord(e1, stream), "event record");
-        hip_check(hipEventSynchronize(e1), "run");
         float ms = 0;
         hip_check(hipEventElapsedTime(&ms, e0, e1), "elapsed");
         (void)hipEventDestroy(e0);
@@ -1834,7 +1899,7 @@ struct Batch {
 
     void check_status()
     {
-        auto v = read_inst();
+        const auto& v = end_table;
         for (size_t i = 0; i < v.size(); ++i) {
             if (v[i].status == MGO_ERR_UNSUPPORTED) {
                 fail(v[i].status, "run %zu: several pending traveler moves per edge (tmax off the dt grid) are not "

@@ -158,7 +158,8 @@ struct InstDev {
     int32_t icu;          // some node has an ICU limit: the ISev rates of the returns depend on the state
     int32_t general;      // every return walks the edges: some edge coefficient or rate is negative, or a rate
                           // exceeds 1 / dt_graph (see come_home)
-    int32_t pad3;
+    int32_t plain;        // 1: the node kernel is the plain one (see NodeMode); PLAIN_LOST: confirmed cases came up,
+                          // the run waits for the host to change the kernel
 };
 static_assert(sizeof(InstDev) % 8 == 0, "instance records are copied as 8-byte words");
 
@@ -263,10 +264,15 @@ struct SegDev {
 constexpr int MAX_SORT_RUNS = 4096; // percentiles: runs whose values one wavefront sorts in its registers
 
 // Instantiations of the node kernel. PLAIN: no node of the launch has an optional feature (test-and-trace or ICU
-// limit, contact dampings, commuter detection, confirmed cases); eight compartments change (INSC and ISYC stay
-// zero: only commuter detection and initial values fill them) and every coefficient is constant. FEATURES: all
-// ten compartments, features by node flag. NPIS: FEATURES with the dynamic NPI checks.
+// limit, contact dampings, commuter detection, confirmed cases); eight compartments change (INSC and ISYC are zero)
+// and every coefficient is constant. FEATURES: all ten compartments, features by node flag. NPIS: FEATURES with the
+// dynamic NPI checks.
+// Beside commuter detection and initial values, the fix-up of the returns fills INSC where every other compartment
+// of a group is negative (more travelers leave than there are, negative populations). The returns note that in the
+// instance (PLAIN_LOST), whose clock then stands still with the state complete, until the host has changed its launch
+// to FEATURES; both kernels give the same bits, so it does not matter when.
 enum NodeMode : int { PLAIN = 0, FEATURES = 1, NPIS = 2 };
+constexpr int32_t PLAIN_LOST = 2;
 
 // One kernel launch over the segments of a class.
 struct LaunchDev {

@@ -629,7 +629,7 @@ __device__ __forceinline__ void clock_one(InstDev& I)
     I.fx_state  = 0;
     I.fx_changed = 0;
     I.fx_count   = 0;
-    if (I.status != 0 || !(I.t < I.tmax)) {
+    if (I.status != 0 || !(I.t < I.tmax) || I.plain == PLAIN_LOST) {
         return;
     }
     double step = I.dt_graph;
@@ -1935,9 +1935,17 @@ __device__ __forceinline__ int32_t record_slot(const FxRec* r, int32_t lo, int32
 // wavefront). With one group of lanes per node and an edge at a time, a pass over nodes of 50 in- and 50
 // out-edges took 120 us and more.
 //
-// Returns (in every lane) WALK_CHANGED if some record changed and WALK_FULL if the record pool is full.
-constexpr int WALK_CHANGED = 1;
-constexpr int WALK_FULL    = 2;
+// Returns (in every lane) WALK_CHANGED if some record changed, WALK_FULL if the record pool is full and
+// WALK_CONFIRMED if the node ends with confirmed cases: a fix-up moves a shortfall to the group's largest
+// remaining compartment, which is INSC where all others are negative.
+constexpr int WALK_CHANGED   = 1;
+constexpr int WALK_FULL      = 2;
+constexpr int WALK_CONFIRMED = 4;
+
+__device__ __forceinline__ bool confirmed_cases(const double (&y)[NC])
+{
+    return y[INSC] != 0.0 || y[ISYC] != 0.0;
+}
 
 template <int G>
 __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass, double* buf)
@@ -2058,7 +2066,7 @@ __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass,
                 y[i] = y1[i] + home[i];
             }
             finish();
-            return 0;
+            return __any(confirmed_cases(y)) ? WALK_CONFIRMED : 0;
         }
     }
     int result    = 0;
@@ -2171,7 +2179,7 @@ __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass,
     }
     in_edges(in_s, in_e);
     finish();
-    return result;
+    return result | (__any(confirmed_cases(y)) ? WALK_CONFIRMED : 0);
 }
 
 // pass 0 of the instances whose returns walk their edges (InstDev::general): every node, one wavefront each
@@ -2191,9 +2199,15 @@ __device__ __forceinline__ void walk_body(const LaunchDev& ld, InstDev* __restri
         if (I.c_active && I.c_action == 2 && I.general) {
             const int r = walk_node<G>(c, I, node, 0, buf + (threadIdx.x / WAVE) * (WAVE * NC));
             if (r != 0 && threadIdx.x % WAVE == 0) {
-                I.fx_changed = 1; // every writer stores the same value
+                // every writer of a field stores the same value
+                if (r & (WALK_CHANGED | WALK_FULL)) {
+                    I.fx_changed = 1;
+                }
                 if (r & WALK_FULL) {
                     I.fx_state = 2;
+                }
+                if ((r & WALK_CONFIRMED) && I.plain) {
+                    I.plain = PLAIN_LOST;
                 }
             }
         }
@@ -2224,6 +2238,7 @@ __device__ __forceinline__ void replay(Seg& c, InstDev& I)
     const EdgeEnt* oute     = es.out_ent;
     const double h          = I.c_step;
     const bool icu          = I.icu != 0;
+    bool confirmed          = false;
     if (a < G) {
         for (int k = 0; k < es.num_edges; ++k) {
             const EdgeEnt e   = oute[seq[3 * k + 2]];
@@ -2251,11 +2266,16 @@ __device__ __forceinline__ void replay(Seg& c, InstDev& I)
             for (int i = 0; i < NC; ++i) {
                 yd[i] -= m[i];
             }
+            confirmed = confirmed || confirmed_cases(m); // no others without a node that has some
         }
     }
+    confirmed = __any(confirmed);
     __syncthreads();
     if (a == 0) {
         I.replays += 1;
+        if (confirmed && I.plain) {
+            I.plain = PLAIN_LOST;
+        }
     }
     if (I.c_out_day >= 0 && a < G) {
         for (int v = 0; v < I.num_nodes; ++v) {
@@ -2283,6 +2303,7 @@ __device__ __forceinline__ void settle_body(const LaunchDev& ld, InstDev* __rest
     // list[CAP]: number of marked nodes, list[CAP + 1]: results of the pass's walks
     bool sequential = I.fx_sequential != 0 || I.fx_state == 2;
     int pass        = 1;
+    int results     = 0; // of all passes
     for (; !sequential; ++pass) {
         if (threadIdx.x == 0) {
             list[CAP + 1] = 0;
@@ -2315,6 +2336,7 @@ __device__ __forceinline__ void settle_body(const LaunchDev& ld, InstDev* __rest
         __syncthreads();
         __threadfence();
         const int r = list[CAP + 1];
+        results |= r;
         __syncthreads(); // everyone has read it before the next pass clears it
         if (!(r & WALK_CHANGED)) {
             break;
@@ -2323,6 +2345,9 @@ __device__ __forceinline__ void settle_body(const LaunchDev& ld, InstDev* __rest
     }
     if (threadIdx.x == 0) {
         I.fx_passes += pass;
+        if ((results & WALK_CONFIRMED) && I.plain) {
+            I.plain = PLAIN_LOST;
+        }
     }
     if (sequential) {
         __syncthreads();

@@ -1173,7 +1173,7 @@ struct Batch {
             InstHost& I   = inst[size_t(ii)];
             const auto* g = r.g;
             inst_ids.push_back(ii);
-            bool icu = false, general = false;
+            bool icu = false, general = false, steep = false;
             for (int v = 0; v < g->num_nodes; ++v) {
                 const size_t node = size_t(I.node_base) + size_t(v) * size_t(I.node_stride);
                 const double* sc  = g->node_scalars + size_t(v) * MGO_NUM_SCALARS;
@@ -1209,7 +1209,7 @@ struct Batch {
                     const double out[] = {lc[LC_E], lc[LC_INS_ISY] + lc[LC_INS_R], lc[LC_ISY_ISEV] + lc[LC_ISY_R],
                                           (lc[LC_ISEV_ICR] + lc[LC_ISEV_R]) + lc[LC_ISEV_D], lc[LC_ICR_D] + lc[LC_ICR_R]};
                     for (double o : out) {
-                        general = general || !(r.cfg.dt_graph * o <= 1.0);
+                        steep = steep || !(r.cfg.dt_graph * o <= 1.0);
                     }
                     for (int j = 0; j < G; ++j) {
                         const size_t k = (size_t(v) * G + size_t(a)) * G + size_t(j);
@@ -1358,7 +1358,7 @@ struct Batch {
                 }
             }
             D.icu     = icu ? 1 : 0;
-            D.general = (D.estruct >= 0 && general) ? 1 : 0;
+            D.general = D.estruct < 0 ? 0 : general ? GENERAL : steep ? STEEP : 0;
             D.fx_base      = fx_total;
             D.fx_pool_base = int64_t(pool_slots) * FX_SLOTS * G * NC;
             if (D.estruct >= 0) {

@@ -156,11 +156,12 @@ struct InstDev {
     int32_t fx_epoch;     // record tag of pass 0 of the current return phase (grows by FX_EPOCH_STEP)
     int32_t node_stride;  // segment index of local node v = node_base + v * node_stride (see Tiling)
     int32_t icu;          // some node has an ICU limit: the ISev rates of the returns depend on the state
-    int32_t general;      // every return walks the edges: some edge coefficient or rate is negative, or a rate
-                          // exceeds 1 / dt_graph (see come_home)
+    int32_t general;      // GENERAL, STEEP or 0, see come_home
     int32_t plain;        // 1: the node kernel is the plain one (see NodeMode); PLAIN_LOST: confirmed cases came up,
                           // the run waits for the host to change the kernel
 };
+constexpr int32_t GENERAL = 1; // every return walks the edges: some edge coefficient or rate is negative
+constexpr int32_t STEEP   = 2; // a rate exceeds 1 / dt_graph
 static_assert(sizeof(InstDev) % 8 == 0, "instance records are copied as 8-byte words");
 
 // Fix-up records. Each in-edge keeps two tagged versions {tag, slot}; tag = fx_epoch + pass of the pass
@@ -285,7 +286,7 @@ struct LaunchDev {
     int32_t G;                  // age groups of every segment, or 0: segments differ (mixed kernels)
     int32_t kind;
     int32_t mode;               // NodeMode of the class's node kernel
-    int32_t general;            // some instance's returns walk the edges (InstDev::general)
+    int32_t general;            // some instance's returns walk the edges (GENERAL)
     int32_t edges;              // some instance has edges
     int32_t pad;
 };

@@ -1686,6 +1686,28 @@ __device__ __forceinline__ void load_weights(Seg& c, const double2* p, size_t np
     x[14] = g.y;
 }
 
+// Whether a compartment may fall below zero while a node's in-edges are taken off one by one, where some rate exceeds
+// 1 / h. An edge's travelers after the step are what stays of them (negative if the rate is steep) and what flows in,
+// both linear in nonnegative numbers with the node's own rates: no sum over some of the edges exceeds the inflow of
+// all and, unless the rate is steep, what stays of all. y: state before the returns; m: all arrivals, dm: their
+// change, w: the node's rates; home: the homecomings, added at once between two in-edges.
+__device__ __forceinline__ bool falls_short(const double (&y)[NC], const double (&m)[NC], const double (&dm)[NC],
+                                            const double (&w)[NFLOW], double h, const double (&home)[NC])
+{
+    double out[NC] = {};
+#pragma unroll
+    for (int f = 0; f < NFLOW; ++f) {
+        out[flow_src(f)] += w[f];
+    }
+    bool low = false;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const double most = h * out[i] > 1.0 ? fma(h * out[i], m[i], dm[i]) : m[i] + dm[i];
+        low               = low || !((y[i] - most) + fmin(home[i], 0.0) >= 0.0);
+    }
+    return low;
+}
+
 // All travelers that come home to a lane's node, each after its destination's Euler step: the lane's departure
 // row stepped with the sums over the out-edges of coefficient times rate. k0: the sum of the forces of infection;
 // k10, k12: those of the ICU-adjusted rates (used with ICU limits, else the kept constants).
@@ -1771,7 +1793,8 @@ __device__ __forceinline__ void edge_return(const EdgeCoef& ec, const double (&r
 // (InstDev::general), the departure rows as they are written (InstDev::fx_neg). Only S, whose rate is the force
 // of infection, may step below zero in earnest (more than 1 / h infections per day at a peak). It has no inflow,
 // so all in-edges of a node change it in one direction and its extremes are at the ends of the sequence and at
-// the homecomings: ypre, ypre - arrivals and both with the homecomings added.
+// the homecomings: ypre, ypre - arrivals and both with the homecomings added. Runs in which another rate exceeds
+// 1 / h (STEEP) take the bound of falls_short instead.
 template <int G>
 __device__ __forceinline__ void come_home(Seg& c, InstDev& I, int node, int age, int base)
 {
@@ -1862,6 +1885,14 @@ __device__ __forceinline__ void come_home(Seg& c, InstDev& I, int node, int age,
     // travelers coming home
     double home[NC];
     homecoming<G>(c, I, es, v, lane, age, D_v, k0, k10, k12, home);
+    if (I.general == STEEP) {
+        double ypre[NC];
+        load_planes(c.ypre, np, lane, ypre);
+        load_planes(c.arr, np, lane, m);
+        lane_rates(c, icu, lane, w);
+        euler_change(m, w, h, dm);
+        mark = mark || falls_short(ypre, m, dm, w, h, home);
+    }
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
         y[i] = y[i] + home[i];
@@ -1899,7 +1930,7 @@ __device__ __forceinline__ void edge_body(const LaunchDev& ld, InstDev* __restri
     if (I.c_action == 1) {
         arrive<G>(c, I, node, age);
     }
-    else if (I.c_action == 2 && !I.general) {
+    else if (I.c_action == 2 && I.general != GENERAL) {
         come_home<G>(c, I, node, age, base);
     }
 }
@@ -2042,7 +2073,7 @@ __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass,
             }
         }
     };
-    if (!I.general) {
+    if (I.general != GENERAL) {
         // A node that walks because a homecoming changed (its travelers were fixed up elsewhere) is mostly done with
         // the closed form of come_home and the new sum, if no fix-up of its own can act and none did so far.
         double m[NC], dm[NC], y1[NC];
@@ -2054,6 +2085,9 @@ __device__ __forceinline__ int walk_node(Seg& c, InstDev& I, int node, int pass,
             y1[i]            = y[i] - (m[i] + dm[i]);
             const double low = fmin(home[i], 0.0);
             full             = full || !(y1[i] >= 0.0) || !(y1[i] + low >= 0.0) || !(y[i] + low >= 0.0);
+        }
+        if (I.general == STEEP) {
+            full = full || falls_short(y, m, dm, rates, h, home);
         }
         if (pass > 1) {
             for (int k = in_b + lane; k < in_e; k += WAVE) {
@@ -2206,7 +2240,7 @@ __device__ __forceinline__ void walk_body(const LaunchDev& ld, InstDev* __restri
     const int wave    = (lb - ld.block_first[seg]) * (BLOCK / WAVE) + int(threadIdx.x) / WAVE;
     for (int node = wave * NPW + int(blockIdx.y); node < min(c.num_nodes, (wave + 1) * NPW); node += int(gridDim.y)) {
         InstDev& I = inst[c.nodep[node].inst];
-        if (I.c_active && I.c_action == 2 && I.general) {
+        if (I.c_active && I.c_action == 2 && I.general == GENERAL) {
             const int r = walk_node<G>(c, I, node, 0, buf + (threadIdx.x / WAVE) * (WAVE * NC));
             if (r != 0 && threadIdx.x % WAVE == 0) {
                 // every writer of a field stores the same value

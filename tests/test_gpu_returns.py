@@ -1,7 +1,7 @@
 """Departures and returns where their closed form has edges: returns that must walk their edges (rates above one
 per half day, negative travelers), susceptibles stepping below zero on the way (more than one infection per half
 day), coefficient vectors, ICU limits, in-degrees around the walk's 64 / G edges at a time, more marked nodes than
-a block lists at once. Against the oracle, fixed steps.
+a block lists at once, negative coefficients. Against the oracle, fixed steps.
 
 Bar: every value to 1e-12 of its compartment's largest value over the run. A value is reached by at most a few
 hundred edge and step operations of relative error 1.1e-16 on that scale, with observed growth below ten.
@@ -51,10 +51,32 @@ def test_in_degrees_around_a_walk_step(ctx, oracle, G):
 
 
 def test_rates_above_one_per_half_day(ctx, oracle):
-    """Stay times below the graph step: the Euler step of the travelers overshoots, every return walks its edges."""
+    """Stay times below the graph step: the Euler step of the travelers overshoots."""
     sp = setups.fixup_graph(seed=6, n=20, G=3)
     sp.age_params[::2, capi.A_TIME_INFECTED_NO_SYMPTOMS, :] = 0.4
     _check(ctx, oracle, sp, 10, synthetic.fixed_cfg(0.05))
+
+
+@pytest.mark.parametrize("n,G", [(70, 1), (20, 3), (24, 8)])
+@pytest.mark.parametrize("stay", [capi.A_TIME_EXPOSED, capi.A_TIME_INFECTED_NO_SYMPTOMS,
+                                  capi.A_TIME_INFECTED_SYMPTOMS, capi.A_TIME_INFECTED_SEVERE,
+                                  capi.A_TIME_INFECTED_CRITICAL])
+def test_each_rate_above_one_per_half_day(ctx, oracle, stay, n, G):
+    """One steep rate in every other node: its compartment's travelers turn negative at such destinations."""
+    sp = setups.fixup_graph(seed=7, n=n, G=G, outflow=0.8)
+    sp.age_params[::2, stay, :] = 0.3
+    _check(ctx, oracle, sp, 8, synthetic.fixed_cfg(0.05))
+
+
+@pytest.mark.parametrize("n,G", [(1, 1), (70, 1), (20, 3), (12, 8)])
+def test_negative_coefficients(ctx, oracle, n, G):
+    """Some edges carry travelers against their direction: every return walks its edges from the start."""
+    sp = synthetic.graph(num_nodes=n + 1, G=G, seed=52, mean_degree=min(5.0, n))
+    c = sp.edge_coeffs.copy()
+    c[::3] *= -0.1
+    c[1 % c.size] = abs(c[1 % c.size])
+    sp.set_edges(sp.edge_start, sp.edge_end, c)
+    _check(ctx, oracle, sp, 6)
 
 
 @pytest.mark.parametrize("G", [1, 4])

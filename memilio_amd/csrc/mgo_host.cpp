@@ -1166,7 +1166,7 @@ struct Batch {
         int64_t fx_total  = 0;
         int64_t pool_slots = 0;
         int wplanes        = 5;
-        bool any_icu = false, any_general = false;
+        bool any_icu = false, any_general = false, any_steep = false;
         bool features = false; // some node has a feature that the plain node kernel leaves out (see NodeMode)
         for (int ii : C.insts) {
             RunSpec& r    = runs[size_t(ii)];
@@ -1355,6 +1355,7 @@ struct Batch {
                     general     = general || soffs[size_t(sidx)].negative;
                     any_icu     = any_icu || icu;
                     any_general = any_general || general;
+                    any_steep   = any_steep || (steep && !general);
                 }
             }
             D.icu     = icu ? 1 : 0;
@@ -1570,6 +1571,7 @@ struct Batch {
         ld.kind        = C.kind;
         ld.mode        = !(C.npi.nodes0.empty() && C.oute.nodes0.empty()) ? NPIS : features ? FEATURES : PLAIN;
         ld.general     = any_general ? 1 : 0;
+        ld.steep       = any_steep ? 1 : 0;
         ld.edges       = 0;
         for (int ii : C.insts) {
             ld.edges               = ld.edges || inst[size_t(ii)].has_edges;
@@ -1626,6 +1628,7 @@ struct Batch {
                 gs.push_back(C->G);
                 m.launch.edges   = m.launch.edges || C->launch.edges;
                 m.launch.general = m.launch.general || C->launch.general;
+                m.launch.steep   = m.launch.steep || C->launch.steep;
             }
             block_tables_mixed(nodes, gs, bseg, bfirst);
             auto up = [&](DevBuf& b, auto&& v, auto& keep) {

@@ -288,7 +288,7 @@ struct LaunchDev {
     int32_t mode;               // NodeMode of the class's node kernel
     int32_t general;            // some instance's returns walk the edges (GENERAL)
     int32_t edges;              // some instance has edges
-    int32_t pad;
+    int32_t steep;              // some instance has steep rates (STEEP)
 };
 
 } // namespace mgo

@@ -1795,7 +1795,7 @@ __device__ __forceinline__ void edge_return(const EdgeCoef& ec, const double (&r
 // so all in-edges of a node change it in one direction and its extremes are at the ends of the sequence and at
 // the homecomings: ypre, ypre - arrivals and both with the homecomings added. Runs in which another rate exceeds
 // 1 / h (STEEP) take the bound of falls_short instead.
-template <int G>
+template <int G, bool ANY_STEEP>
 __device__ __forceinline__ void come_home(Seg& c, InstDev& I, int node, int age, int base)
 {
     Est& es = edge_struct(c, I.estruct);
@@ -1885,7 +1885,7 @@ __device__ __forceinline__ void come_home(Seg& c, InstDev& I, int node, int age,
     // travelers coming home
     double home[NC];
     homecoming<G>(c, I, es, v, lane, age, D_v, k0, k10, k12, home);
-    if (I.general == STEEP) {
+    if (ANY_STEEP && I.general == STEEP) {
         double ypre[NC];
         load_planes(c.ypre, np, lane, ypre);
         load_planes(c.arr, np, lane, m);
@@ -1913,8 +1913,9 @@ __device__ __forceinline__ void come_home(Seg& c, InstDev& I, int node, int age,
 }
 
 // Edge action of the cycle: arrivals or returns, one launch for both (a cycle has one or the other, or some runs
-// each; an idle launch costs about 4.5 us).
-template <int G>
+// each; an idle launch costs about 4.5 us). ANY_STEEP: instantiation for launches with steep rates (in all launches,
+// the code for them had 68 instead of 20 B of registers spilled).
+template <int G, bool ANY_STEEP>
 __device__ __forceinline__ void edge_body(const LaunchDev& ld, InstDev* __restrict__ inst)
 {
     int node, age, base;
@@ -1931,7 +1932,7 @@ __device__ __forceinline__ void edge_body(const LaunchDev& ld, InstDev* __restri
         arrive<G>(c, I, node, age);
     }
     else if (I.c_action == 2 && I.general != GENERAL) {
-        come_home<G>(c, I, node, age, base);
+        come_home<G, ANY_STEEP>(c, I, node, age, base);
     }
 }
 
@@ -2441,10 +2442,10 @@ __global__ void __launch_bounds__(BLOCK, M == PLAIN ? 2 : 1) node_phase_mixed(La
     MGO_DISPATCH_G(block_groups(ld), (node_body<GG, K, M>(ld, inst, wx)))
 }
 
-template <int G>
+template <int G, bool ANY_STEEP>
 __global__ void __launch_bounds__(BLOCK, EDGE_WAVES) edge_phase(LaunchDev ld, InstDev* __restrict__ inst)
 {
-    edge_body<G>(ld, inst);
+    edge_body<G, ANY_STEEP>(ld, inst);
 }
 
 template <int G>
@@ -2487,9 +2488,10 @@ __global__ void __launch_bounds__(SETTLE_BLOCK) settle_phase(LaunchDev ld, InstD
 }
 
 #if MGO_SHARD == 13
+template <bool ANY_STEEP>
 __global__ void __launch_bounds__(BLOCK, EDGE_WAVES) edge_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
 {
-    MGO_DISPATCH_G(block_groups(ld), (edge_body<GG>(ld, inst)))
+    MGO_DISPATCH_G(block_groups(ld), (edge_body<GG, ANY_STEEP>(ld, inst)))
 }
 
 __global__ void __launch_bounds__(BLOCK) walk_phase_mixed(LaunchDev ld, InstDev* __restrict__ inst)
@@ -2549,7 +2551,12 @@ template <int G>
 hipError_t launch_edge_g(const LaunchDev& c, InstDev* inst, bool clock, hipStream_t s)
 {
     if (c.edges) {
-        hipLaunchKernelGGL((edge_phase<G>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        if (c.steep) {
+            hipLaunchKernelGGL((edge_phase<G, true>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        }
+        else {
+            hipLaunchKernelGGL((edge_phase<G, false>), dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        }
         if (c.general) {
             hipLaunchKernelGGL((walk_phase<G>), walk_grid(c.num_blocks, G), dim3(BLOCK), 0, s, c, inst);
         }
@@ -2802,7 +2809,12 @@ template hipError_t launch_node_mixed<MGO_SHARD - 9>(const LaunchDev&, InstDev*,
 hipError_t launch_edge_mixed(const LaunchDev& c, InstDev* inst, bool clock, hipStream_t s)
 {
     if (c.edges) {
-        hipLaunchKernelGGL(edge_phase_mixed, dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        if (c.steep) {
+            hipLaunchKernelGGL(edge_phase_mixed<true>, dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        }
+        else {
+            hipLaunchKernelGGL(edge_phase_mixed<false>, dim3(c.num_blocks), dim3(BLOCK), 0, s, c, inst);
+        }
         if (c.general) {
             hipLaunchKernelGGL(walk_phase_mixed, walk_grid(c.num_blocks, 1), dim3(BLOCK), 0, s, c, inst);
         }

@@ -266,7 +266,7 @@ typedef struct mgo_run_info {
     int64_t steps;             /* accepted integration steps summed over all nodes */
     int64_t attempts;          /* step attempts summed over all nodes */
     int64_t exact_replays;     /* return phases resolved by the sequential negative-value fix-up replay */
-    int64_t fixup_passes;      /* extra parallel return passes run to settle negative-value fix-ups */
+    int64_t fixup_passes;      /* extra return passes run to settle negative-value fix-ups (a replay counts as one) */
     int32_t half_day_cycles;   /* graph steps executed */
     int32_t node_launches;     /* node-phase kernel launches timed (MGO_CTX_PROFILE_KERNELS) */
     double node_kernel_ms;     /* summed duration of those launches */

@@ -1573,10 +1573,13 @@ struct Batch {
         ld.general     = any_general ? 1 : 0;
         ld.steep       = any_steep ? 1 : 0;
         ld.edges       = 0;
+        int max_nodes = 0;
         for (int ii : C.insts) {
             ld.edges               = ld.edges || inst[size_t(ii)].has_edges;
+            max_nodes              = std::max(max_nodes, inst[size_t(ii)].num_nodes);
             idev[size_t(ii)].plain = ld.mode == PLAIN ? 1 : 0;
         }
+        settle_shape(ld, ld.edges ? max_nodes : 1);
     }
 
     // Launch tables of a cycle. Small classes that differ in G alone share one chain of launches whose blocks
@@ -1617,8 +1620,10 @@ struct Batch {
             std::vector<SegDev> segs;
             std::vector<int> nodes, gs;
             std::vector<int32_t> ids, bseg, bfirst;
+            int max_nodes = 1;
             for (ClassHost* C : group) {
                 for (int ii : C->insts) {
+                    max_nodes               = std::max(max_nodes, inst[size_t(ii)].num_nodes);
                     ids.push_back(ii);
                     idev[size_t(ii)].seg     = int32_t(segs.size());
                     inst[size_t(ii)].launch = int(launches.size());
@@ -1647,6 +1652,7 @@ struct Batch {
             m.launch.inst_ids    = m.inst_ids.as<int32_t>();
             m.launch.num_blocks  = int(m.block_seg.bytes / sizeof(int32_t));
             m.launch.G           = 0;
+            settle_shape(m.launch, m.launch.edges ? max_nodes : 1);
             launches.push_back(&m.launch);
         }
     }

@@ -148,7 +148,7 @@ struct InstDev {
     int64_t fx_pool_base; // first double of this instance's slots in SegDev::fx_pool
     int32_t fx_neg;       // negative travelers left at the last departure: their returns walk the edges
     int32_t fx_state;     // 2: the record pool is full, sequential replay needed
-    int32_t fx_changed;   // set when nodes are marked to walk their edges in the next pass
+    int32_t fx_changed;   // nodes marked to walk their edges in the next pass (FX_MANY: unknown, some)
     int32_t fx_count;     // pool slots used in this return phase
     int32_t fx_passes;    // extra passes run so far (statistics)
     int32_t fx_sequential; // resolve fix-ups with the sequential replay only
@@ -159,6 +159,8 @@ struct InstDev {
     int32_t general;      // GENERAL, STEEP or 0, see come_home
     int32_t plain;        // 1: the node kernel is the plain one (see NodeMode); PLAIN_LOST: confirmed cases came up,
                           // the run waits for the host to change the kernel
+    int32_t fx_pass;      // passes of this return phase that earlier launches walked
+    uint32_t fx_arrived;  // blocks that have walked their share of a pass, and their results (see settle_body)
 };
 constexpr int32_t GENERAL = 1; // every return walks the edges: some edge coefficient or rate is negative
 constexpr int32_t STEEP   = 2; // a rate exceeds 1 / dt_graph
@@ -177,8 +179,10 @@ constexpr int FX_SLOTS      = 1024; // pool slots per instance and return phase
 constexpr int FX_MAX_PASSES = 8;    // passes before falling back to the sequential replay
 constexpr int FX_EPOCH_STEP = 16;   // > FX_MAX_PASSES
 
-constexpr int SETTLE_BLOCK  = 512;  // threads of an instance's block (eight walks at a time)
-constexpr int SETTLE_LIST   = 1024; // marked nodes an instance's block holds in LDS at a time
+constexpr int FX_MANY       = 1 << 30;
+constexpr int SETTLE_BLOCK  = 512;  // threads of a block that settles returns (eight walks at a time)
+constexpr int SETTLE_LIST   = 4096; // marked nodes it holds in LDS at a time
+constexpr int SETTLE_SLICES = 64;   // blocks per instance at most
 
 // CSR edge structure of one graph (node indices local to the instance). In-edges of node v are sorted
 // by source; in_split[v] = number of in-edges whose source < v, so walking
@@ -289,6 +293,22 @@ struct LaunchDev {
     int32_t general;            // some instance's returns walk the edges (GENERAL)
     int32_t edges;              // some instance has edges
     int32_t steep;              // some instance has steep rates (STEEP)
+    int32_t slices;             // blocks per instance in the settling kernel
+    int32_t wide;               // launches of it before the last, one pass each
 };
+
+// Blocks and launches of the settling kernel. A block has a CU's registers: as many blocks per run as there are CUs,
+// up to one wavefront per node. us per half-day with one block per run / with this: 400 nodes of 6 groups, heavy
+// commuting 272 / 99; 10000 nodes of 1 group 178 / 115. From 1536 nodes the second pass is worth a launch of its own
+// (about 1.5 us where it is idle): 2000 nodes of 6 groups 71 / 72, of 3 groups with steep rates 411 / 179; 10000 nodes
+// of 1 group 115 / 101, 40000 nodes 230 / 140. A second one gains nothing.
+inline void settle_shape(LaunchDev& ld, int max_nodes)
+{
+    const int per_inst = 256 / (ld.num_inst > 0 ? ld.num_inst : 1);
+    const int useful   = (max_nodes + 7) / 8;
+    ld.slices          = per_inst < useful ? per_inst : useful;
+    ld.slices          = ld.slices < 1 ? 1 : ld.slices > SETTLE_SLICES ? SETTLE_SLICES : ld.slices;
+    ld.wide            = max_nodes >= 1536 ? 1 : 0;
+}
 
 } // namespace mgo

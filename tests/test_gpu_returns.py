@@ -129,3 +129,15 @@ def test_fixups_settle_and_replay(ctx, oracle):
     with Context(flags=capi.CTX_SEQUENTIAL_FIXUP) as seq:
         info = _check(seq, oracle, sp, 20, fixups=True)
         assert info.exact_replays > 0
+
+
+@pytest.mark.parametrize("n,G,runs", [(9, 8, 3), (70, 1, 40), (300, 3, 257), (1500, 1, 2), (1600, 1, 3)])
+def test_shares_of_a_pass(ctx, oracle, n, G, runs):
+    """A pass's nodes are shared out to 256 / runs blocks of eight wavefronts, at most one per node: the same bits
+    alone (up to 64 blocks), beside one other run, in a large batch (one block). 1600 nodes: two launches."""
+    sp = setups.fixup_graph(seed=9, n=n, G=G)
+    _check(ctx, oracle, sp, 4, fixups=n > 9)
+    alone, info = ctx.ensemble_run([sp], [synthetic.fixed_cfg(0.1)], [4.0])
+    out, both = ctx.ensemble_run([sp] * runs, [synthetic.fixed_cfg(0.1)] * runs, [4.0] * runs)
+    assert all(np.array_equal(o, alone[0]) for o in out)
+    assert both.fixup_passes == runs * info.fixup_passes

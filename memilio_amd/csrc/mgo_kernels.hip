@@ -2288,16 +2288,22 @@ __device__ __forceinline__ void replay(Seg& c, InstDev& I)
     const bool icu          = I.icu != 0;
     bool confirmed          = false;
     if (a < G) {
+        int src = -1;
+        double row[NC], D = 0.0; // of the source: the edges are sorted by it
         for (int k = 0; k < es.num_edges; ++k) {
             const EdgeEnt e   = oute[seq[3 * k + 2]];
             const size_t soff = seg_node(I, seq[3 * k]) * G + a;
             const size_t doff = seg_node(I, seq[3 * k + 1]) * G + a;
-            const EdgeCoef ec = edge_coef(es, e, es.out_min, seq[3 * k + 2], c.out_d ? c.out_d[soff] : 0.0, G, a);
+            if (seq[3 * k] != src) {
+                src = seq[3 * k];
+                load_planes(c.dep, np, soff, row);
+                D = c.out_d ? c.out_d[soff] : 0.0;
+            }
+            const EdgeCoef ec = edge_coef(es, e, es.out_min, seq[3 * k + 2], D, G, a);
             double m[NC], dm[NC], w[NFLOW];
-            load_planes(c.dep, np, soff, m);
             lane_rates(c, icu, doff, w);
             for (int i = 0; i < NC; ++i) {
-                m[i] = m[i] * coef_of(ec, i);
+                m[i] = row[i] * coef_of(ec, i);
             }
             euler_change(m, w, h, dm);
             double* yd = c.y + doff * NC;

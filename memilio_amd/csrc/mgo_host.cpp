@@ -218,7 +218,8 @@ struct DevBuf {
 // Results on their way to the caller's (pageable) memory. A plain copy runs at about 17 GB/s into memory that is
 // there and at half of that into memory that the call itself makes resident, page by page. Large downloads go in
 // chunks through pinned buffers, one per copying thread: the transfers of some overlap the host copies of the others
-// (115 MB of daily values: 11 -> 3 ms).
+// (115 MB of daily values: 11 -> 3 ms). Memory that HIP knows, pinned memory above all, takes the copy itself (211 MB
+// into pinned memory: 4.1 ms, through the chunks 5.3 ms).
 struct Piece {
     const char* src; // device
     char* dst;       // host
@@ -269,6 +270,17 @@ struct Downloader {
         buf = nullptr;
     }
 
+    // whether HIP knows the memory (of one allocation: the pieces are parts of one result)
+    static bool known(const void* p)
+    {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        return a.type != hipMemoryTypeUnregistered;
+    }
+
     // Copies the pieces once the work queued on `s` is done; returns when they are in host memory.
     void run(const std::vector<Piece>& pieces, hipStream_t s, int device)
     {
@@ -276,7 +288,7 @@ struct Downloader {
         for (const Piece& p : pieces) {
             total += p.bytes;
         }
-        if (total < MIN || !ready()) {
+        if (total < MIN || known(pieces[0].dst) || !ready()) {
             for (const Piece& p : pieces) {
                 if (p.bytes > 0) {
                     hip_check(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s), "download");

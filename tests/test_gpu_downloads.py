@@ -1,9 +1,11 @@
 """Downloads in chunks by several threads: sizes around the size from which they are used (8 MiB) and around a chunk
-(1 MiB), every value in its place, bitwise (the mean of one run is the run itself)."""
+(1 MiB), every value in its place, bitwise (the mean of one run is the run itself), into pageable and pinned memory."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from memilio_amd import synthetic
+from memilio_amd import capi, synthetic
 from memilio_amd.engine import Batch, Context
 
 pytestmark = pytest.mark.gpu
@@ -29,3 +31,20 @@ def test_runs_of_different_size_arrive_in_place():
         for k in range(4):
             assert np.array_equal(batch.read_daily(k, 1)[0], whole[k])
         batch.close()
+
+
+@pytest.mark.parametrize("n,offset", [(8 * MIB - 1, 0), (8 * MIB, 3), (17 * MIB + 5, 1)])
+def test_into_pinned_memory(n, offset):
+    """Pinned results, also from within an allocation, take the plain copy."""
+    v = np.random.default_rng(n).normal(size=n)
+    with Context() as ctx:
+        hip = C.CDLL("libamdhip64.so")
+        p = C.c_void_p()
+        assert hip.hipHostMalloc(C.byref(p), C.c_size_t((n + offset + 1) * 8), C.c_uint(0)) == 0
+        out = np.frombuffer((C.c_double * (n + offset + 1)).from_address(p.value))
+        out[:] = -1.0
+        ctx.check(ctx.lib.mgo_ensemble_mean_values(ctx.ptr, capi.dptr(v), 1, n, capi.dptr(out[offset:offset + n])))
+        assert np.array_equal(out[offset:offset + n], v)
+        assert (out[:offset] == -1.0).all() and out[offset + n] == -1.0
+        del out
+        assert hip.hipHostFree(p) == 0

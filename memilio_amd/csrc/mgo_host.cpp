@@ -20,7 +20,6 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <tuple>
 #include <unordered_map>
@@ -329,8 +328,8 @@ struct Downloader {
             try {
                 threads.emplace_back(work, t);
             }
-            catch (const std::system_error&) {
-                break; // no more threads to be had: the ones that run take the chunks
+            catch (const std::exception&) {
+                break; // no more threads or memory to be had: the threads that run take the chunks
             }
         }
         work(0);

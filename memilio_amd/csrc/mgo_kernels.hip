@@ -13,8 +13,8 @@
 //   edge_phase<G>      per node lane: the arriving travelers, one sum over the node's in-edges in the
 //                      reference's edge order (deterministic, no atomics); or the returns in closed form,
 //                      marking the nodes on which the negative-value fix-up can act
-//   walk_phase<G>      per node lane of the instances whose returns need the edge walk (see InstDev::general)
-//   settle_phase<G>    per instance: marked nodes walk their edges with the fix-up, in passes over the nodes
+//   walk_phase<G>      per node of the instances whose returns need the edge walk (GENERAL), one wavefront each
+//   settle_phase<G>    per instance (up to 64 blocks): marked nodes walk their edges with the fix-up, in passes over the nodes
 //                      whose inputs changed; sequential replay where these do not settle. Then the instance's
 //                      next cycle: step size, edge action and output day
 //
@@ -1002,8 +1002,8 @@ __device__ double out_damping(Seg& c, Lane<G, M>& L, InstDev& I, const double (&
 // neighbours in the wavefront.
 //
 // Bound by the FP64 issue rate and, with few wavefronts, by the chain of dependent operations of one attempt (six
-// right-hand sides with an LDS exchange each). The plain instantiation fits 256 registers without scratch, two
-// wavefronts per SIMD: eight compartments, no feature code (the arguments of sin, cos and pow alone took a third
+// right-hand sides with an LDS exchange each). The plain instantiation fits 256 registers, two wavefronts
+// per SIMD (12 B of scratch for Cash-Karp and G = 8, 20 B in the mixed Cash-Karp and RKF45 kernels, none else): eight compartments, no feature code (the arguments of sin, cos and pow alone took a third
 // of 107 KB of code, above the 64 KB instruction cache; 15 KB now), the scalars of a step in LDS (Cold). 512 runs x
 // 400 nodes x 6 groups at 1e-10: 580 us per half-day against 1030 us for ten compartments at one wavefront per
 // SIMD; a single 400-node graph 39 us against 50 us. Two wavefronts with the cold scalars in registers spilled 25
@@ -1488,7 +1488,7 @@ __device__ __forceinline__ bool fixup_negative(const double (&y)[NC], double (&m
     return neg;
 }
 
-constexpr int EDGE_WAVES   = 3; // wavefronts per SIMD of the edge kernel
+constexpr int EDGE_WAVES   = 3; // wavefronts per SIMD of the edge kernel (20 B of scratch, 28 B in the mixed one)
 constexpr int DEPART_ROWS  = 4; // departure rows in flight per lane
 constexpr int RETURN_EDGES = 8; // forces of infection in flight per lane
 
@@ -2667,8 +2667,8 @@ hipError_t launch_node_mixed(const LaunchDev& c, InstDev* inst, hipStream_t s)
 // theirs pairwise, quads with quads and so on. All lists ascend: a merge first compares mirrored elements, then
 // halves the distance; between lanes a value is fetched with a DPP move (distances within 16 lanes) or a
 // permute. Comparisons within a lane are a minimum and a maximum; the more values a lane holds, the fewer of the
-// costlier comparisons between lanes, and 64 doubles leave two wavefronts per SIMD (three spill and are no
-// faster). Values are read once; bound by the comparisons. 1000 runs x 33333 positions: 163 us, 512 runs x 744000
+// costlier comparisons between lanes, and 64 doubles leave two wavefronts per SIMD (with 36 to 64 B of scratch from
+// two lanes on; three spill more and are no faster). Values are read once; bound by the comparisons. 1000 runs x 33333 positions: 163 us, 512 runs x 744000
 // positions: 1.20 ms (2.5 TB/s), against 1720 us and 15.3 ms for the bitonic sort in LDS below, which was bound by
 // its LDS passes and barriers and remains for more than 4096 runs (two wavefronts per position).
 //

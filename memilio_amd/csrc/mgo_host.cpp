@@ -283,18 +283,22 @@ struct Downloader {
     // Copies the pieces once the work queued on `s` is done; returns when they are in host memory.
     void run(const std::vector<Piece>& pieces, hipStream_t s, int device)
     {
+        hip_check(copy(pieces, s, device), "download");
+    }
+    hipError_t copy(const std::vector<Piece>& pieces, hipStream_t s, int device)
+    {
+        hipError_t err = hipSuccess;
         size_t total = 0;
         for (const Piece& p : pieces) {
             total += p.bytes;
         }
         if (total < MIN || known(pieces[0].dst) || !ready()) {
             for (const Piece& p : pieces) {
-                if (p.bytes > 0) {
-                    hip_check(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s), "download");
+                if (p.bytes > 0 && err == hipSuccess) {
+                    err = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s);
                 }
             }
-            hip_check(hipStreamSynchronize(s), "download");
-            return;
+            return err == hipSuccess ? hipStreamSynchronize(s) : err;
         }
         std::vector<Piece> chunks;
         for (const Piece& p : pieces) {
@@ -302,7 +306,10 @@ struct Downloader {
                 chunks.push_back(Piece{p.src + off, p.dst + off, std::min(CHUNK, p.bytes - off)});
             }
         }
-        hip_check(hipStreamSynchronize(s), "download");
+        err = hipStreamSynchronize(s);
+        if (err != hipSuccess) {
+            return err;
+        }
         std::atomic<size_t> next{0};
         std::atomic<int> error{int(hipSuccess)};
         auto work = [&](int t) {
@@ -336,7 +343,7 @@ struct Downloader {
         for (std::thread& t : threads) {
             t.join();
         }
-        hip_check(hipError_t(error.load()), "download");
+        return hipError_t(error.load());
     }
 };
 

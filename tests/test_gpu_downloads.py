@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from memilio_amd import capi, synthetic
-from memilio_amd.engine import Batch, Context
+from memilio_amd.engine import Batch, Context, Server
 
 pytestmark = pytest.mark.gpu
 MIB = 1 << 17   # doubles
@@ -48,3 +48,19 @@ def test_into_pinned_memory(n, offset):
         assert (out[:offset] == -1.0).all() and out[offset + n] == -1.0
         del out
         assert hip.hipHostFree(p) == 0
+
+
+def test_served_results_beside_a_full_pool():
+    """Results that find no room in the pinned pool, above and below the size of chunked downloads, are whole."""
+    specs = [synthetic.graph(num_nodes=n, G=6, seed=n, mean_degree=3.0) for n in (300, 350, 40)]
+    cfgs, tmaxs = [synthetic.ck_cfg(1e-6)] * 3, [60.0] * 3
+    with Context() as ctx:
+        want, _ = ctx.ensemble_run(specs, cfgs, tmaxs)
+        assert want[0].nbytes > 8 << 20 > want[2].nbytes
+        server = Server(ctx, result_pool_bytes=1 << 20)
+        tickets = [server.submit(*r) for r in zip(specs, cfgs, tmaxs)]
+        infos = server.wait(tickets)
+        assert all(i.status == capi.OK for i in infos.values())
+        for k, t in enumerate(tickets):
+            assert np.array_equal(server.take(t), want[k])
+        server.stop()

@@ -438,7 +438,7 @@ struct RunSpec {
 };
 
 struct EdgeStructHost {
-    std::vector<int32_t> in_ptr, out_ptr, split, seq;
+    std::vector<int32_t> in_ptr, out_ptr, split;
     std::vector<EdgeEnt> in_ent, out_ent;
     std::vector<double> in_min, out_min; // uniform minimum per entry (empty: the graph has no minimum)
     // per node, over its out-edges: sums of the coefficients and minima (uniform: one value, else 10 G)
@@ -777,7 +777,6 @@ void build_edges(const mgo_graph_desc* g, EdgeStructHost& es, std::vector<double
         es.in_min.assign(edges.size(), 0.0);
     }
     es.split.assign(size_t(n), 0);
-    es.seq.clear();
     std::vector<int> ofill(es.out_ptr.begin(), es.out_ptr.end() - 1), ifill(es.in_ptr.begin(), es.in_ptr.end() - 1);
     // edges are sorted by (s, d): out lists come out sorted by d, in lists sorted by s
     for (auto& e : edges) {
@@ -792,9 +791,6 @@ void build_edges(const mgo_graph_desc* g, EdgeStructHost& es, std::vector<double
         if (e.s < e.d) {
             es.split[size_t(e.d)]++;
         }
-        es.seq.push_back(e.s);
-        es.seq.push_back(e.d);
-        es.seq.push_back(ko);
     }
     // sums over every node's out-edges, in their order
     const size_t w = es.uniform ? 1 : size_t(nv);
@@ -1168,7 +1164,7 @@ struct Batch {
         std::vector<EdgeEnt> epool;
         std::vector<double> cvec, cvec_min, mpool;
         struct StructOff {
-            size_t in_ptr, out_ptr, split, seq, in_ent, out_ent;
+            size_t in_ptr, out_ptr, split, in_ent, out_ent;
             int64_t in_min = -1, out_min = -1; // offsets into mpool, -1 = no minimum
             size_t in_src = 0, out_dst = 0;    // into ipool (uniform structures)
             int64_t in_c = -1, out_c = -1;     // into mpool (uniform structures)
@@ -1325,8 +1321,6 @@ struct Batch {
                     ipool.insert(ipool.end(), es.out_ptr.begin(), es.out_ptr.end());
                     so.split = ipool.size();
                     ipool.insert(ipool.end(), es.split.begin(), es.split.end());
-                    so.seq = ipool.size();
-                    ipool.insert(ipool.end(), es.seq.begin(), es.seq.end());
                     so.in_ent = epool.size();
                     epool.insert(epool.end(), es.in_ent.begin(), es.in_ent.end());
                     so.out_ent = epool.size();
@@ -1474,7 +1468,6 @@ struct Batch {
             sd.in_ptr               = ib + so.in_ptr;
             sd.out_ptr              = ib + so.out_ptr;
             sd.split                = ib + so.split;
-            sd.seq                  = ib + so.seq;
             sd.in_ent               = eb + so.in_ent;
             sd.out_ent              = eb + so.out_ent;
             sd.cvec                 = C.cvec.as<double>();

@@ -201,7 +201,6 @@ struct EdgeStructDev {
     const int32_t* in_ptr;   // [n+1]
     const int32_t* out_ptr;  // [n+1]
     const int32_t* split;    // [n]
-    const int32_t* seq;      // [num_edges][3] = (start, end, out-entry) in global edge order, exact replay
     const EdgeEnt* in_ent;
     const EdgeEnt* out_ent;
     const double* cvec;      // non-uniform coefficient vectors [k][10*G]

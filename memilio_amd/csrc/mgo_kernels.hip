@@ -14,9 +14,9 @@
 //                      reference's edge order (deterministic, no atomics); or the returns in closed form,
 //                      marking the nodes on which the negative-value fix-up can act
 //   walk_phase<G>      per node of the instances whose returns need the edge walk (GENERAL), one wavefront each
-//   settle_phase<G>    per instance (up to 64 blocks): marked nodes walk their edges with the fix-up, in passes over the nodes
-//                      whose inputs changed; sequential replay where these do not settle. Then the instance's
-//                      next cycle: step size, edge action and output day
+//   settle_phase<G>    per instance (up to 64 blocks): marked nodes walk their edges with the fix-up, in passes
+//                      over the nodes whose inputs changed; sequential replay where these do not settle. Then
+//                      the instance's next cycle: step size, edge action and output day
 //
 // The file is compiled once per shard (MGO_SHARD, see memilio_amd/build.py), in parallel: shard 0 holds the
 // launch dispatch and the kernels without a G, shards 1..8 the kernels of that G, shards 9..12 the node kernel
@@ -1002,12 +1002,12 @@ __device__ double out_damping(Seg& c, Lane<G, M>& L, InstDev& I, const double (&
 // neighbours in the wavefront.
 //
 // Bound by the FP64 issue rate and, with few wavefronts, by the chain of dependent operations of one attempt (six
-// right-hand sides with an LDS exchange each). The plain instantiation fits 256 registers, two wavefronts
-// per SIMD (12 B of scratch for Cash-Karp and G = 8, 20 B in the mixed Cash-Karp and RKF45 kernels, none else): eight compartments, no feature code (the arguments of sin, cos and pow alone took a third
-// of 107 KB of code, above the 64 KB instruction cache; 15 KB now), the scalars of a step in LDS (Cold). 512 runs x
-// 400 nodes x 6 groups at 1e-10: 580 us per half-day against 1030 us for ten compartments at one wavefront per
-// SIMD; a single 400-node graph 39 us against 50 us. Two wavefronts with the cold scalars in registers spilled 25
-// values per attempt: 768 us and 51 us.
+// right-hand sides with an LDS exchange each). The plain instantiation fits 256 registers, two wavefronts per SIMD (12 B
+// of scratch for Cash-Karp and G = 8, 20 B in the mixed Cash-Karp and RKF45 kernels, none else): eight compartments, no
+// feature code (the arguments of sin, cos and pow alone took a third of 107 KB of code, above the 64 KB instruction
+// cache; 15 KB now), the scalars of a step in LDS (Cold). 512 runs x 400 nodes x 6 groups at 1e-10: 580 us per half-day
+// against 1030 us for ten compartments at one wavefront per SIMD; a single 400-node graph 39 us against 50 us. Two
+// wavefronts with the cold scalars in registers spilled 25 values per attempt: 768 us and 51 us.
 constexpr uint32_t kMaxAttemptsPerPhase = 1u << 20;
 
 template <int G, int K, int M>
@@ -2264,13 +2264,16 @@ __device__ __forceinline__ void walk_body(const LaunchDev& ld, InstDev* __restri
 
 // ------------------------------------------------------------------------------- settling the fix-ups
 // Sequential return pass of one instance in the reference's edge order with the negative-value fix-up
-// (metapopulation_mobility_instant.h:568-603). Fallback for the rare return phases whose fix-up records
-// did not settle within FX_MAX_PASSES passes or overflowed the record pool; lanes = age groups.
+// (metapopulation_mobility_instant.h:568-603), for the return phases whose fix-up records did not settle within
+// FX_MAX_PASSES passes or overflowed the record pool. The edges are sorted by source and the edges of one source go to
+// different nodes, so their fix-ups do not depend on each other: one wavefront takes 64 / G of them at a time (an edge
+// from a node to itself alone) and adds what comes home in order. Edge by edge, on G lanes, a graph of 400 nodes and
+// 20k edges whose returns all replay took 12.5 ms per half-day; 2.8 ms so.
 template <int G>
-__device__ __forceinline__ void replay(Seg& c, InstDev& I)
+__device__ __forceinline__ void replay(Seg& c, InstDev& I, double* buf)
 {
-    const int a     = int(threadIdx.x);
-    const size_t np = size_t(c.num_nodes) * G;
+    constexpr int NPW = WAVE / G;
+    const size_t np   = size_t(c.num_nodes) * G;
     // restore the pre-return state of every node
     for (int k = int(threadIdx.x); k < I.num_nodes * G; k += int(blockDim.x)) {
         const size_t lane = seg_node(I, k / G) * G + size_t(k % G);
@@ -2282,63 +2285,100 @@ __device__ __forceinline__ void replay(Seg& c, InstDev& I)
     }
     __syncthreads();
     Est& es = edge_struct(c, I.estruct);
-    const int32_t* seq      = es.seq;
-    const EdgeEnt* oute     = es.out_ent;
-    const double h          = I.c_step;
-    const bool icu          = I.icu != 0;
-    bool confirmed          = false;
-    if (a < G) {
-        int src = -1;
-        double row[NC], D = 0.0; // of the source: the edges are sorted by it
-        for (int k = 0; k < es.num_edges; ++k) {
-            const EdgeEnt e   = oute[seq[3 * k + 2]];
-            const size_t soff = seg_node(I, seq[3 * k]) * G + a;
-            const size_t doff = seg_node(I, seq[3 * k + 1]) * G + a;
-            if (seq[3 * k] != src) {
-                src = seq[3 * k];
-                load_planes(c.dep, np, soff, row);
-                D = c.out_d ? c.out_d[soff] : 0.0;
-            }
-            const EdgeCoef ec = edge_coef(es, e, es.out_min, seq[3 * k + 2], D, G, a);
-            double m[NC], dm[NC], w[NFLOW];
-            lane_rates(c, icu, doff, w);
-            for (int i = 0; i < NC; ++i) {
-                m[i] = row[i] * coef_of(ec, i);
-            }
-            euler_change(m, w, h, dm);
-            double* yd = c.y + doff * NC;
-            double* ys = c.y + soff * NC;
-            double yl[NC];
-            for (int i = 0; i < NC; ++i) {
-                m[i]  = m[i] + dm[i];
-                yl[i] = yd[i];
-            }
-            fixup_negative(yl, m);
-            for (int i = 0; i < NC; ++i) {
-                ys[i] += m[i];
-            }
-            for (int i = 0; i < NC; ++i) {
-                yd[i] -= m[i];
-            }
-            confirmed = confirmed || confirmed_cases(m); // no others without a node that has some
-        }
-    }
-    confirmed = __any(confirmed);
-    __syncthreads();
-    if (a == 0) {
-        I.replays += 1;
-        if (confirmed && I.plain) {
-            I.plain = PLAIN_LOST;
-        }
-    }
-    if (I.c_out_day >= 0 && a < G) {
+    if (threadIdx.x < WAVE) {
+        const int lane  = int(threadIdx.x);
+        const int grp   = lane / G;
+        const int age   = lane - grp * G;
+        const double h  = I.c_step;
+        const bool icu  = I.icu != 0;
+        bool confirmed  = false;
         for (int v = 0; v < I.num_nodes; ++v) {
-            const size_t lane = seg_node(I, v) * G + a;
-            double yv[NC];
-            for (int i = 0; i < NC; ++i) {
-                yv[i] = c.y[lane * NC + i];
+            const int out_e   = es.out_ptr[v + 1];
+            int k             = es.out_ptr[v];
+            const size_t soff = seg_node(I, v) * G + age;
+            const double D    = c.out_d ? c.out_d[soff] : 0.0;
+            if (k == out_e) {
+                continue;
             }
-            write_phase_end_day<G>(c, I, lane, v, a, yv);
+            double row[NC], ys[NC];
+            load_planes(c.dep, np, soff, row);
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                ys[i] = c.y[soff * NC + i];
+            }
+            while (k < out_e) {
+                const int mine   = min(k + grp, out_e - 1);
+                const EdgeEnt e  = es.out_ent[mine];
+                const bool in    = grp < NPW && k + grp < out_e;
+                const auto selfs = __ballot(in && e.nbr == v);
+                const int ahead  = selfs ? (__ffsll(selfs) - 1) / G : NPW; // edges before one to the node itself
+                const int n      = min(max(ahead, 1), out_e - k);
+                if (in && grp < n) {
+                    const size_t doff = seg_node(I, e.nbr) * G + age;
+                    const EdgeCoef ec = edge_coef(es, e, es.out_min, mine, D, G, age);
+                    double rates[NFLOW], m[NC], y[NC];
+                    lane_rates(c, icu, doff, rates);
+#pragma unroll
+                    for (int i = 0; i < NC; ++i) {
+                        m[i] = row[i];
+                        y[i] = ahead == 0 ? ys[i] : c.y[doff * NC + i];
+                    }
+                    edge_return(ec, rates, h, m);
+                    fixup_negative(y, m);
+#pragma unroll
+                    for (int i = 0; i < NC; ++i) {
+                        buf[i * WAVE + lane] = m[i];
+                    }
+                    if (ahead != 0) {
+#pragma unroll
+                        for (int i = 0; i < NC; ++i) {
+                            c.y[doff * NC + i] = y[i] - m[i];
+                        }
+                    }
+                    confirmed = confirmed || confirmed_cases(m); // no others without a node that has some
+                }
+                wave_sync();
+                for (int j = 0; j < n; ++j) {
+#pragma unroll
+                    for (int i = 0; i < NC; ++i) {
+                        ys[i] += buf[i * WAVE + j * G + age];
+                    }
+                }
+                if (ahead == 0) {
+#pragma unroll
+                    for (int i = 0; i < NC; ++i) {
+                        ys[i] -= buf[i * WAVE + age];
+                    }
+                }
+                wave_sync(); // also before the next edges read the states written here
+                k += n;
+            }
+            if (grp == 0) {
+#pragma unroll
+                for (int i = 0; i < NC; ++i) {
+                    c.y[soff * NC + i] = ys[i];
+                }
+            }
+            wave_sync();
+        }
+        confirmed = __any(confirmed);
+        if (lane == 0) {
+            I.replays += 1;
+            if (confirmed && I.plain) {
+                I.plain = PLAIN_LOST;
+            }
+        }
+    }
+    __syncthreads();
+    if (I.c_out_day >= 0) {
+        for (int k = int(threadIdx.x); k < I.num_nodes * G; k += int(blockDim.x)) {
+            const int v       = k / G;
+            const size_t lane = seg_node(I, v) * G + size_t(k % G);
+            double y[NC];
+            for (int i = 0; i < NC; ++i) {
+                y[i] = c.y[lane * NC + i];
+            }
+            write_phase_end_day<G>(c, I, lane, v, k % G, y);
         }
     }
 }
@@ -2460,7 +2500,7 @@ __device__ __forceinline__ bool settle_body(const LaunchDev& ld, InstDev& I, int
     }
     if (sequential && last) {
         __syncthreads();
-        replay<G>(c, I);
+        replay<G>(c, I, buf);
     }
     return true;
 }

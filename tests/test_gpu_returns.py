@@ -131,6 +131,34 @@ def test_fixups_settle_and_replay(ctx, oracle):
         assert info.exact_replays > 0
 
 
+@pytest.mark.parametrize("G", [1, 3, 6])
+def test_edges_of_a_node_to_itself(ctx, oracle, G):
+    """The first, a middle and the last of a node's edges lead back to it; also resolved sequentially."""
+    n = 26
+    sp = setups.fixup_graph(seed=12, n=n, G=G)
+    loops = np.array([0, 7, 8, n - 1])
+    start = np.concatenate([sp.edge_start, loops])
+    c = np.concatenate([sp.edge_coeffs, [0.05, 0.02, 0.09, 0.05]])
+    c *= 0.98 / np.bincount(start, weights=c)[start]
+    sp.set_edges(start, np.concatenate([sp.edge_end, loops]), c)
+    _check(ctx, oracle, sp, 6, fixups=True)
+    with Context(flags=capi.CTX_SEQUENTIAL_FIXUP) as seq:
+        _check(seq, oracle, sp, 6, fixups=True)
+
+
+@pytest.mark.parametrize("G", [1, 2, 6, 8])
+def test_replay_of_many_edges(ctx, oracle, G):
+    """Out-degrees around the replay's 64 / G edges at a time, from 0 to 64 / G + 2."""
+    most = 64 // G + 2
+    n = max(40, most + 1)
+    sp = setups.fixup_graph(seed=12, n=n, G=G)
+    start, end = np.array([(s, (s + 1 + d) % n) for s in range(n) for d in range(s % (most + 1))]).T
+    sp.set_edges(start, end, 0.98 / np.bincount(start)[start])
+    with Context(flags=capi.CTX_SEQUENTIAL_FIXUP) as seq:
+        info = _check(seq, oracle, sp, 6, fixups=True)
+        assert info.exact_replays > 0
+
+
 @pytest.mark.parametrize("n,G,runs", [(9, 8, 3), (70, 1, 40), (300, 3, 257), (1500, 1, 2), (1600, 1, 3)])
 def test_shares_of_a_pass(ctx, oracle, n, G, runs):
     """A pass's nodes are shared out to 256 / runs blocks of eight wavefronts, at most one per node: the same bits

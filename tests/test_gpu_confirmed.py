@@ -6,11 +6,13 @@ Bar against the oracle (fixed steps): every value to 1e-12 of the run's largest.
 fused multiply-adds differs by at most 2e-15 on that scale over these runs; per compartment it is no measure, since
 a fix-up leaves values near zero whose sign decides the next one.
 """
+import time
+
 import numpy as np
 import pytest
 
 from memilio_amd import capi, synthetic
-from memilio_amd.engine import Batch, Context, GraphSim, Server
+from memilio_amd.engine import Batch, Context, GraphSim, MgoError, Server
 from memilio_amd.graphspec import INSC, ISYC
 
 pytestmark = pytest.mark.gpu
@@ -92,3 +94,20 @@ def test_forms_of_a_call(ctx, oracle, kind, G, seed, days):
         assert _close(server.take(tickets[0]), ref) and _close(server.take(tickets[2]), ref)
         assert np.array_equal(server.take(tickets[1]), alone[0])
         server.stop()
+
+
+@pytest.mark.parametrize("delay_ms", [0, 2, 6, 12])
+def test_update_while_the_clock_stands(ctx, delay_ms):
+    """A scenario update (of no effect) that finds the request waiting for its other kernel: it still runs to its end."""
+    sp = _spec("negative", 2, 3)
+    want, _ = ctx.ensemble_run([sp], [CFG], [120.0])
+    server = Server(ctx)
+    ticket = server.submit(sp, CFG, 120.0)
+    time.sleep(1e-3 * delay_ms)
+    try:
+        server.update(ticket, 1.0)
+    except MgoError:
+        pass  # finished already
+    assert server.wait([ticket])[ticket].status == capi.OK
+    assert np.array_equal(server.take(ticket), want[0], equal_nan=True)
+    server.stop()
